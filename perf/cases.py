@@ -31,7 +31,7 @@ import minim_amd as m
 
 SIGMA = [1.0, 0.8, 1.2]  # pairwise surface tensions of the three-fluid fields
 DENSITY = 0.85           # reduced density of the liquid
-RCUT, SKIN = 2.5, 0.3
+RCUT = 2.5
 LATTICE = (1.0 / DENSITY) ** (1.0 / 3.0)
 
 
@@ -53,7 +53,7 @@ def listed():
         # a Lennard-Jones cluster as the reference evaluates it, all pairs
         dict(name="cluster_1000_fp64", kind="cluster", n=1000, dim=3, prec="fp64"),
         # the benchmark's liquid: 64^3 particles within a cutoff
-        dict(name="liquid_64cubed_fp32", kind="liquid", side=64, prec="fp32"),
+        dict(name="liquid_64cubed_fp32", kind="liquid", side=64, skin=0.3, prec="fp32"),
         # the benchmark's elastic sheet: 1024 x 1024 nodes
         dict(name="sheet_1024sq_fp64", kind="sheet", nx=1024, ny=1024, prec="fp64"),
         # the start of the headline minimisation, mixed schedule, on the device
@@ -63,7 +63,7 @@ def listed():
         dict(name="relax_128sq_fp64", kind="relax", nx=128, ny=128, nz=1, nf=1, mode="fp64", iters=30, host=True),
         # FIRE steps of a medium liquid: two dozen dependent launches and a
         # list check per step
-        dict(name="fire_32cubed_fp64", kind="fire", side=32, prec="fp64", iters=100),
+        dict(name="fire_32cubed_fp64", kind="fire", side=32, skin=0.3, prec="fp64", iters=100),
         # a batch of uneven fields, sides spread over [32, 512]
         dict(name="batch_64_fp64", kind="batch", count=64, sides=4040, mode="fp64", iters=30),
     ]
@@ -100,7 +100,7 @@ def draw(rng):
     if kind == "cluster":
         return dict(kind=kind, n=_log(rng, 64, 4096), dim=rng.choice([2, 3]), prec=prec)
     if kind == "liquid":
-        return dict(kind=kind, side=_log(rng, 9, 64), prec=prec)
+        return dict(kind=kind, side=_log(rng, 9, 64), skin=round(rng.uniform(0.2, 0.4), 3), prec=prec)
     if kind == "sheet":
         return dict(kind=kind, nx=_log(rng, 24, 700), ny=_log(rng, 24, 700), prec=prec)
     if kind == "relax":
@@ -111,7 +111,8 @@ def draw(rng):
         return dict(kind=kind, nx=nx, ny=ny, nz=nz, nf=nf, mode=mode, iters=8 if mode == "mixed" else 30,
                     host=flat and rng.random() < 0.5)
     if kind == "fire":
-        return dict(kind=kind, side=_log(rng, 9, 40), prec="fp64", iters=100)
+        return dict(kind=kind, side=_log(rng, 9, 40), skin=round(rng.uniform(0.2, 0.4), 3), prec="fp64",
+                    iters=rng.randint(60, 100))
     return dict(kind="batch", count=_log(rng, 8, 64), sides=rng.randrange(1 << 20), mode="fp64", iters=30)
 
 
@@ -237,7 +238,7 @@ def prepare(case, seed):
         if kind == "cluster":
             pot = m.LjNd(case["dim"])
         elif kind == "liquid":
-            pot = m.Lj3d().setCutoff(RCUT, [case["side"] * LATTICE] * 3, SKIN)
+            pot = m.Lj3d().setCutoff(RCUT, [case["side"] * LATTICE] * 3, case["skin"])
         elif kind == "sheet":
             nx, ny = case["nx"], case["ny"]
             pot = m.BarAndHinge().setTriangulation(_sheet_triangles(nx, ny)).setRigidity(1.0, 0.01)
@@ -267,7 +268,7 @@ def prepare(case, seed):
         return st
     if kind == "fire":
         x = _liquid_input(case, gen, torch.float32).to(dtype)
-        pot = m.Lj3d().setCutoff(RCUT, [case["side"] * LATTICE] * 3, SKIN)
+        pot = m.Lj3d().setCutoff(RCUT, [case["side"] * LATTICE] * 3, case["skin"])
         st.update(state=m.State(pot, _host(x), prec), x0=x.reshape(-1),
                   mini=m.Fire(0.02).setDt0(0.002).setMaxForceConvergence(3).setMaxIter(case["iters"] - 1))
         return st
