@@ -54,6 +54,57 @@ def test_lj_golden_vectors(gpu, case, prec):
         assert rel_err(g, c["gradient"]) <= 1e-12
 
 
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 257, 1024, 1025, 2047, 2048, 2050])
+@pytest.mark.parametrize("dim", [1, 2, 3, 4])
+def test_lj_all_pairs_sizes(gpu, dim, n, prec):
+    """Energy, gradient and the trial energy at x + t d around the kernel's
+    block and group sizes, against numpy's FP64 pair sums, which add pairwise.
+    (The oracle adds its n(n-1)/2 terms one after another: at n = 2,047 in one
+    dimension each of the far pairs, below half an ulp of the running sum, is
+    lost there -- about 2,047 * 4/5 * 185^-5 = 8e-9 of 2,010, over 1e-12.)  On a
+    jittered lattice the pair terms of one sign dominate, so the rounding errors
+    of the sums stay within the usual tolerance."""
+    import torch
+
+    def pair_sums(x):
+        p = x.reshape(n, dim)
+        dx = p[:, None, :] - p[None, :, :]
+        r2 = (dx * dx).sum(-1)
+        np.fill_diagonal(r2, 1.0)
+        i6 = r2 ** -3
+        pair, f = 4 * (i6 * i6 - i6), -24 * (2 * i6 * i6 - i6) / r2
+        np.fill_diagonal(pair, 0.0)
+        np.fill_diagonal(f, 0.0)
+        return 0.5 * pair.sum(), np.einsum("ijk,ij->ik", dx, f).reshape(-1)
+
+    m = gpu
+    print("case lj all pairs", dim, n, prec, flush=True)
+    rng = np.random.default_rng(1000 * dim + n)
+    side = int(np.ceil(n ** (1.0 / dim) - 1e-9))
+    pts = np.array(np.meshgrid(*[np.arange(side) * 1.15] * dim, indexing="ij")).reshape(dim, -1).T[:n]
+    x = r32((pts + rng.uniform(-0.05, 0.05, pts.shape)).reshape(-1))
+    d = r32(rng.uniform(-0.1, 0.1, x.shape))
+    eo, go = pair_sums(x)
+    h = m.LjNd(dim).handle(x)
+    dt = torch.float64 if prec == "fp64" else torch.float32
+    xd = torch.tensor(x, dtype=dt, device="cuda")
+    dd = torch.tensor(d, dtype=dt, device="cuda")
+    g = torch.full_like(xd, float("nan"))
+    e = m.potential_eval(h, prec, xd.data_ptr(), x.size, g_ptr=g.data_ptr())
+    g2 = torch.full_like(xd, float("nan"))
+    m.potential_eval(h, prec, xd.data_ptr(), x.size, g_ptr=g2.data_ptr(), want_energy=False)
+    et = m.potential_eval(h, prec, xd.data_ptr(), x.size, d_ptr=dd.data_ptr(), t=0.25)
+    assert torch.equal(g, g2)
+    if n == 1:
+        assert e == 0.0 and et == 0.0 and not g.any()
+        return
+    assert abs(e - eo) <= TOL[prec] * abs(eo)
+    eto = pair_sums(x + 0.25 * d)[0]
+    assert abs(et - eto) <= TOL[prec] * abs(eto)
+    assert rel_err(g.cpu().numpy(), go) <= TOL[prec]
+
+
 def lattice(n_side, a, jitter, rng):
     g = np.arange(n_side) * a
     pts = np.array(np.meshgrid(g, g, g, indexing="ij")).reshape(3, -1).T
