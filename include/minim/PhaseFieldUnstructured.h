@@ -91,7 +91,8 @@ class PhaseFieldUnstructured : public NewPotential<PhaseFieldUnstructured> {
   vector<double> nodeVol;  // per DOF, as the reference's initLocal stores it
   vector<int> fluidType;   // per DOF
   size_t nElements = 0;    // energy elements built by init
-  size_t listBytes = 0;    // device bytes of the element list (records, parameters, chunk and site tables)
+  size_t listBytes = 0;    // device bytes of the elements as stored (records, parameters, chunk and site tables;
+                           // gathered per site: launch arguments, and the site codes of solids)
 
  private:
   void setDefaults();

@@ -133,7 +133,9 @@ int minim_pfu_create(const minim_pf_params* p, minim_potential** out);
 /* Number of energy elements init built (the size of the reference's
  * Potential::elements, include/Potential.h:90) and the device bytes of the
  * list as this library stores it (16-byte records, parameters, chunk and
- * site tables); either pointer may be NULL. */
+ * site tables; where the elements are gathered per site and no list is
+ * stored, the launch arguments and, with solid nodes, a 4-byte code per site);
+ * either pointer may be NULL. */
 int minim_pfu_element_list(const minim_potential* pot, size_t* n_elements, size_t* device_bytes);
 
 /* LjNd(nDim, sigma, epsilon) (include/potentials/LjNd.h:12-44): all pairs, no cutoff. */

@@ -1,6 +1,8 @@
 // pf.hpp -- launch interface of the PhaseField stencil kernels (pf.hip).
 #pragma once
 
+#include <vector>
+
 #include "common.hpp"
 
 namespace minim_amd {
@@ -138,3 +140,10 @@ void pf_launch_volume_projection(const PFArgs& a, int prec, void* v, size_t nsit
 void pf_launch_volumes(const PFArgs& a, int prec, const void* x, size_t nsite, RedScratch rs, hipStream_t s);
 
 }  // namespace minim_amd
+
+namespace minim {
+// Host set-up shared by the grid and the element form (phasefield.cpp).
+void pf_canonical(const int grid[3], int canon[3], int cmap[3]);
+void pf_bond_codes(const int grid[3], const char* solid, const std::vector<int>& kinds, std::vector<uint16_t>* codeOut,
+                   std::vector<uint32_t>& wcode);
+}  // namespace minim

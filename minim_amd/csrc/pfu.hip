@@ -6,18 +6,25 @@
 // site and fluid (or per site for the "fixed" density mode, whose last fluid
 // is implicit), one-DOF pressure, surface, force and confinement elements and
 // a soft-density element per site, then the volume term over the whole field
-// (blockEnergyGradient, :280-308).  Here the host groups the elements into
-// chunks of nearby sites; a block takes one chunk at a time, one thread per
-// element, accumulates the energy in FP64 for a deterministic two-stage
-// reduction and the gradient contributions in an FP64 LDS accumulator
-// (ds_add_f64), then stores the gradient of every site only its chunk touches
-// and writes the partial sums of the sites other chunks also touch to a
-// scratch slot; a second pass sums those partials per site in chunk order.
-// No global atomics; the LDS adds of one chunk land in the order its threads
-// reach them, so the gradient's last bits may vary from launch to launch.  Each element keeps the reference's formula,
-// including its choices, so that the element form serves as the independent
-// cross-check of the gather-form kernels it is in the reference.
+// (blockEnergyGradient, :280-308).  Two forms here, chosen by init:
+//
+//  * gathered per site (pfu_site_kernel) when the list holds nothing but fluid,
+//    pressure and three-fluid soft-density elements: one thread per site adds
+//    the seven-site elements that its site is part of, so nothing is read but
+//    the concentrations (and a 4-byte code per site next to solid nodes);
+//  * the list itself (pfu_chunk_kernel) otherwise: the host groups the elements
+//    into chunks of nearby sites; a block takes one chunk at a time, one thread
+//    per element, accumulates the energy in FP64 for a deterministic two-stage
+//    reduction and the gradient contributions in an FP64 LDS accumulator
+//    (ds_add_f64), then stores the gradient of every site only its chunk touches
+//    and writes the partial sums of the sites other chunks also touch to a
+//    scratch slot; a second pass sums those partials per site in chunk order.
+//    No global atomics; the LDS adds of one chunk land in the order its threads
+//    reach them, so the gradient's last bits may vary from launch to launch.
+//
+// Each element keeps the reference's formula, including its choices.
 #include "common.hpp"
+#include "pf_tile.hpp"
 #include "pfu.hpp"
 
 namespace minim_amd {
@@ -274,6 +281,320 @@ __global__ __launch_bounds__(kBlock) void pfu_gather_kernel(PFUArgs u, T* __rest
   }
 }
 
+// ---------------------------------------------------------------- per-site form
+// Barrier that orders LDS traffic only (no wait on outstanding global accesses).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <typename T, int N>
+struct SiteVec {
+  T v[N];
+};
+
+// Concentrations (x, or x + t*d) and codes of the R own rows and the halo site
+// of one x plane.
+template <typename T, int NF, int R, bool SOLID>
+struct SitePlane {
+  T x[R][NF];
+  T hx[NF];
+  unsigned q[SOLID ? R : 1];
+  unsigned hq;
+};
+
+template <typename T, int NF, int R, bool SOLID, bool DIR>
+__device__ __forceinline__ void load_site_plane(const PFUArgs& u, size_t pl, const T* __restrict__ x,
+                                                const T* __restrict__ d, T t, const TileThread& th,
+                                                SitePlane<T, NF, R, SOLID>& p) {
+  auto one = [&](unsigned site, T(&v)[NF]) {
+    const unsigned off = site * (unsigned)(NF * sizeof(T));
+    const char* xb = reinterpret_cast<const char*>(x + pl * NF);
+    const SiteVec<T, NF> xv = *reinterpret_cast<const SiteVec<T, NF>*>(xb + off);
+#pragma unroll
+    for (int k = 0; k < NF; k++) v[k] = xv.v[k];
+    if constexpr (DIR) {
+      const char* db = reinterpret_cast<const char*>(d + pl * NF);
+      const SiteVec<T, NF> dv = *reinterpret_cast<const SiteVec<T, NF>*>(db + off);
+#pragma unroll
+      for (int k = 0; k < NF; k++) {
+        const T st = t * dv.v[k];
+        v[k] = v[k] + st;
+      }
+    }
+  };
+#pragma unroll
+  for (int r = 0; r < R; r++) one(th.site[r], p.x[r]);
+  one(th.hsite, p.hx);
+  if constexpr (SOLID) {
+    const uint32_t* qp = u.wcode + pl;
+#pragma unroll
+    for (int r = 0; r < R; r++) p.q[r] = qp[th.site[r]];
+    p.hq = qp[th.hsite];
+  }
+}
+
+// Weight of the bond to the plus neighbour along canonical dimension j.
+template <typename T>
+__device__ __forceinline__ T bond_w(unsigned q, int j) {
+  return (T)((q >> (kPFWeightShift + kPFWeightBits * j)) & ((1u << kPFWeightBits) - 1u)) * (T)0.0625;
+}
+
+// One site: the energy of its own elements (each bond's two halves counted at
+// its minus end), and its gradient, to which every seven-site element that
+// contains it contributes: for a bond (i, j) the elements of both ends give
+// 2 f w (c_i - c_j), with w = (v_i h_i->j + v_j h_j->i) / res^3 (1 away from
+// solid nodes).  The contributions are added in FP64 in either precision, as
+// the list form's accumulator does, and the projection is applied before the
+// one rounding.  Bonds of weight zero do not read the other site's value (a
+// solid site may hold anything).
+template <typename T, int NF, bool WE, bool WG, bool SOLID>
+__device__ __forceinline__ void site_elements(const PFUArgs& u, const PFArgs& con, const T (&c)[NF],
+                                              const T (&xm)[NF], const T (&xp)[NF], const T (&ym)[NF],
+                                              const T (&yp)[NF], const T (&zm)[NF], const T (&zp)[NF], unsigned qc,
+                                              unsigned qxm, unsigned qym, unsigned qzm, double& ea,
+                                              double (&g)[NF]) {
+  const int kind = (int)(qc & 15u);
+  const T vc = !SOLID ? (T)1 : kind >= 2 ? (T)(kind - 1) * (T)0.125 : (T)kind;
+  const bool fluid = !SOLID || kind != 0;
+  const T wf[3] = {SOLID ? bond_w<T>(qc, 0) : (T)1, SOLID ? bond_w<T>(qc, 1) : (T)1,
+                   SOLID ? bond_w<T>(qc, 2) : (T)1};
+  const T wb[3] = {SOLID ? bond_w<T>(qxm, 0) : (T)1, SOLID ? bond_w<T>(qym, 1) : (T)1,
+                   SOLID ? bond_w<T>(qzm, 2) : (T)1};
+#pragma unroll
+  for (int k = 0; k < NF; k++) {
+    const T ck = c[k];
+    T dm[3] = {ck - xm[k], ck - ym[k], ck - zm[k]};
+    T dp[3] = {ck - xp[k], ck - yp[k], ck - zp[k]};
+    if constexpr (SOLID) {
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        dm[j] = wb[j] == (T)0 ? (T)0 : dm[j];
+        dp[j] = wf[j] == (T)0 ? (T)0 : dp[j];
+      }
+    }
+    const T a2 = ck - (T)1;
+    if (WE && fluid) {
+      // fluidEnergy (:518-538) and the halves of phaseGradient's squares
+      T sq = (T)0;
+#pragma unroll
+      for (int j = 0; j < 3; j++) sq = fma(SOLID ? wf[j] * dp[j] : dp[j], dp[j], sq);
+      T e;
+      if (NF == 1) {
+        const T a1 = ck + (T)1;
+        e = ((T)u.fb[k] * vc) * ((a1 * a1) * (a2 * a2));
+      } else {
+        e = ((T)u.fb[k] * vc) * ((ck * ck) * (a2 * a2));
+      }
+      e = fma((T)u.fg[k], sq, e);
+      const T pr = (T)u.pressure[k];  // pressureEnergy (:613-628)
+      if (pr != (T)0) e = e - pr * ((NF == 1 ? (T)0.5 * (ck + (T)1) : ck) * (vc * (T)u.v1));
+      ea += (double)e;
+    }
+    if (WG) {
+      double lap = 0.0;
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        lap = SOLID ? fma((double)wb[j], (double)dm[j], lap) : lap + (double)dm[j];
+        lap = SOLID ? fma((double)wf[j], (double)dp[j], lap) : lap + (double)dp[j];
+      }
+      T bg;
+      if (NF == 1) bg = (((T)4 * (T)u.fb[k]) * vc) * (ck * fma(ck, ck, (T)-1));
+      else bg = (((T)2 * (T)u.fb[k]) * vc) * ((ck * a2) * fma((T)2, ck, (T)-1));
+      double gk = fma(2.0 * u.fg[k], lap, (double)bg);
+      const double pr = u.pressure[k];
+      if (pr != 0.0) gk -= (NF == 1 ? 0.5 * pr : pr) * ((double)vc * u.v1);
+      g[k] = fluid ? gk : 0.0;
+    }
+  }
+  if constexpr (NF == 3) {
+    if (u.soft && fluid) {  // densityConstraintEnergy (:631-642)
+      const T rho = ((c[0] + c[1]) + c[2]) - (T)1;
+      const T coef = (T)u.coef_density;
+      if (WE) ea += (double)(coef * (rho * rho));
+      if (WG) {
+        const T gr = ((T)2 * coef) * rho;
+#pragma unroll
+        for (int k = 0; k < NF; k++) g[k] += (double)gr;
+      }
+    }
+  }
+  if (WG) {
+    // fixed fluids zeroed, then the mean of the variable ones removed
+    if (con.fixmask) {
+#pragma unroll
+      for (int k = 0; k < NF; k++)
+        if (con.fixmask & (1u << k)) g[k] = 0.0;
+    }
+    if (NF > 1 && con.density == kDensityHard && con.nvar > 0) {
+      double comp = g[0];
+#pragma unroll
+      for (int k = 1; k < NF; k++) comp += g[k];
+      comp *= con.inv_nvar;
+#pragma unroll
+      for (int k = 0; k < NF; k++)
+        if (!(con.fixmask & (1u << k))) g[k] -= comp;
+    }
+  }
+}
+
+// The grid form's decomposition (pf_tile.hpp): a block streams the x planes of
+// a 64 x 4R (z, y) tile through a two-plane LDS ring, the loads of plane i+2
+// in flight while plane i is computed; own columns and x neighbours stay in
+// registers.  Bound by memory: 128x112x120x3, energy and gradient with the
+// reduction, FP64 21.7 us = 3.8 TB/s of concentrations in and gradient out,
+// FP32 16.4 us; the list form, which reads 16 bytes and issues some 200
+// instructions per element, took 156 and 130 us there.  Gradient error against
+// 64 bits 1.53e-16 (list 1.59e-16) and 2.8e-8 in FP32 (list 5.5e-8).
+// MODE bits: 1 = energy, 2 = gradient, 4 = at x + t*d.
+template <typename T, int NF, int MODE, int R, bool SOLID>
+__global__ __launch_bounds__(kBlock) void pfu_site_kernel(PFUArgs u, PFArgs con, TileGeom G,
+                                                          const T* __restrict__ x, const T* __restrict__ d, T t,
+                                                          T* __restrict__ g, RedScratch rs) {
+  constexpr bool WE = MODE & 1, WG = MODE & 2, DIR = MODE & 4;
+  constexpr int LH = kTileWaves * R + 2, LW = kTileZ + 2;
+  using Plane = SitePlane<T, NF, R, SOLID>;
+  __shared__ T lds[2][LH][LW][NF];
+  __shared__ unsigned lq[SOLID ? 2 : 1][SOLID ? LH : 1][SOLID ? LW : 1];
+
+  TileThread th;
+  tile_thread(G, xcd_logical_block(blockIdx.x, gridDim.x), threadIdx.x, th);
+  const size_t YZ = (size_t)G.Y * G.Z;
+  const int X = G.X, x0 = th.x0, x1 = th.x1;
+  const bool halo = th.hrow >= 0;
+  auto load = [&](int plane, Plane& p) {
+    load_site_plane<T, NF, R, SOLID, DIR>(u, (size_t)tile_plane(plane, X) * YZ, x, d, t, th, p);
+  };
+  auto fill = [&](int b, const Plane& p) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+#pragma unroll
+      for (int k = 0; k < NF; k++) lds[b][th.lrow0 + r][th.lcol][k] = p.x[r][k];
+      if constexpr (SOLID) lq[b][th.lrow0 + r][th.lcol] = p.q[r];
+    }
+    if (halo) {
+#pragma unroll
+      for (int k = 0; k < NF; k++) lds[b][th.hrow][th.hcol][k] = p.hx[k];
+      if constexpr (SOLID) lq[b][th.hrow][th.hcol] = p.hq;
+    }
+  };
+
+  T A[R][NF], B[R][NF], Cn[R][NF];  // planes i-1, i, i+1 of the own rows
+  unsigned qA[R], qB[R], qC[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) qA[r] = qB[r] = qC[r] = 0;
+  {
+    Plane pm, p0, p1;
+    load(x0 - 1, pm);
+    load(x0, p0);
+    load(x0 + 1, p1);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+#pragma unroll
+      for (int k = 0; k < NF; k++) {
+        A[r][k] = pm.x[r][k];
+        B[r][k] = p0.x[r][k];
+        Cn[r][k] = p1.x[r][k];
+      }
+      if constexpr (SOLID) {
+        qA[r] = pm.q[r];
+        qB[r] = p0.q[r];
+        qC[r] = p1.q[r];
+      }
+    }
+    fill(0, p0);
+    fill(1, p1);
+  }
+  __syncthreads();
+
+  double acc[1] = {0.0};
+#pragma nounroll
+  for (int i = x0; i < x1; i++) {
+    const int b = (i - x0) & 1;
+    Plane q;
+    load(i + 2, q);
+    T* gp = g + (size_t)i * YZ * NF;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      T ym[NF], yp[NF], zm[NF], zp[NF];
+#pragma unroll
+      for (int k = 0; k < NF; k++) {
+        ym[k] = (r > 0) ? B[r > 0 ? r - 1 : 0][k] : lds[b][th.lrow0 + r - 1][th.lcol][k];
+        yp[k] = (r < R - 1) ? B[r < R - 1 ? r + 1 : 0][k] : lds[b][th.lrow0 + r + 1][th.lcol][k];
+        zm[k] = lds[b][th.lrow0 + r][th.lcol - 1][k];
+        zp[k] = lds[b][th.lrow0 + r][th.lcol + 1][k];
+      }
+      unsigned qym = 0, qzm = 0;
+      if constexpr (SOLID) {
+        qym = (r > 0) ? qB[r > 0 ? r - 1 : 0] : lq[b][th.lrow0 + r - 1][th.lcol];
+        qzm = lq[b][th.lrow0 + r][th.lcol - 1];
+      }
+      double es = 0.0, gv[NF];
+      site_elements<T, NF, WE, WG, SOLID>(u, con, B[r], A[r], Cn[r], ym, yp, zm, zp, qB[r], qA[r], qym, qzm, es, gv);
+      if (th.own & (1u << r)) {
+        if (WE) acc[0] += es;
+        if (WG) {
+          T* gs = gp + (size_t)th.site[r] * NF;  // streaming stores: not re-read here
+#pragma unroll
+          for (int k = 0; k < NF; k++) __builtin_nontemporal_store((T)gv[k], gs + k);
+        }
+      }
+    }
+    lds_barrier();  // every wave is done reading buffer b
+    fill(b, q);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+#pragma unroll
+      for (int k = 0; k < NF; k++) {
+        A[r][k] = B[r][k];
+        B[r][k] = Cn[r][k];
+        Cn[r][k] = q.x[r][k];
+      }
+      if constexpr (SOLID) {
+        qA[r] = qB[r];
+        qB[r] = qC[r];
+        qC[r] = q.q[r];
+      }
+    }
+  }
+  grid_sum_store<1>(acc, rs);
+}
+
+// Rows per thread: three plane copies of the own rows and the plane in flight
+// stay in registers.
+template <typename T, int NF, bool SOLID>
+constexpr int site_rows() {
+  return sizeof(T) * NF <= (SOLID ? 12 : 24) ? 4 : 2;
+}
+
+constexpr int kSiteTargetBlocks = 512;  // two blocks of 4 waves per CU
+
+template <typename T, int NF, int MODE, bool SOLID>
+int launch_site_solid(const PFUArgs& u, const PFArgs& con, const T* x, const T* d, T t, T* g, RedScratch rs,
+                      hipStream_t s) {
+  constexpr int R = site_rows<T, NF, SOLID>();
+  TileGeom G;
+  if (!tile_geom(u.X, u.Y, u.Z, R, 0, kSiteTargetBlocks, kMaxRedBlocks, G))
+    throw std::invalid_argument("PhaseFieldUnstructured: grid too large for one launch");
+  pfu_site_kernel<T, NF, MODE, R, SOLID><<<G.nblocks, kBlock, 0, s>>>(u, con, G, x, d, t, g, rs);
+  return G.nblocks;
+}
+
+template <typename T, int NF, int MODE>
+int launch_site_nf(const PFUArgs& u, const PFArgs& con, const T* x, const T* d, T t, T* g, RedScratch rs,
+                   hipStream_t s) {
+  return u.wcode ? launch_site_solid<T, NF, MODE, true>(u, con, x, d, t, g, rs, s)
+                 : launch_site_solid<T, NF, MODE, false>(u, con, x, d, t, g, rs, s);
+}
+
+template <typename T, int MODE>
+int launch_site(const PFUArgs& u, const PFArgs& con, const T* x, const T* d, T t, T* g, RedScratch rs,
+                hipStream_t s) {
+  switch (u.nf) {
+    case 1: return launch_site_nf<T, 1, MODE>(u, con, x, d, t, g, rs, s);
+    case 2: return launch_site_nf<T, 2, MODE>(u, con, x, d, t, g, rs, s);
+    case 3: return launch_site_nf<T, 3, MODE>(u, con, x, d, t, g, rs, s);
+    default: return launch_site_nf<T, 4, MODE>(u, con, x, d, t, g, rs, s);
+  }
+}
+
 // Fluid volumes for the volume term (:284-293).
 template <typename T, typename TV, bool DIR>
 __global__ __launch_bounds__(kBlock) void pfu_volumes_kernel(PFUArgs u, const T* __restrict__ x,
@@ -298,7 +619,7 @@ __global__ __launch_bounds__(kBlock) void pfu_volumes_kernel(PFUArgs u, const T*
 // volCoef * volDiff per fluid, and (with the energy) the term's energy added to
 // the elements' (:295-300).  One thread.
 __global__ void pfu_volfix_kernel(PFUArgs u, const double* __restrict__ vol, double* __restrict__ energy,
-                                  int want_energy) {
+                                  int want_energy, double* eOut) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   double e = want_energy ? energy[0] : 0.0;
   for (int k = 0; k < u.nf; k++) {
@@ -307,6 +628,7 @@ __global__ void pfu_volfix_kernel(PFUArgs u, const double* __restrict__ vol, dou
     u.volg[k] = u.vol_coef * diff;
   }
   if (want_energy) energy[0] = e;
+  if (eOut) *eOut = e;
 }
 
 // The volume term's gradient, weighted towards interfaces (:301-306).
@@ -340,25 +662,44 @@ void launch_chunk(const PFUArgs& u, int nb, const T* x, const T* d, T t, T* g, R
 // kMaxRedBlocks blocks write reduction partials).
 int chunk_blocks(const PFUArgs& u) { return u.nchunk < 1 ? 1 : (u.nchunk < 2048 ? u.nchunk : 2048); }
 
+// The elements' energies (reduction value 0 of the block count returned) and
+// gradient: constrained when gathered per site, else not.
 template <typename T>
-void eval_t(const PFUArgs& u, int mode, const void* x, const void* d, double t, void* g, RedScratch rs,
-            hipStream_t s) {
+int launch_elements(const PFUArgs& u, const PFArgs& con, int mode, const T* x, const T* d, T t, T* g, RedScratch rs,
+                    hipStream_t s) {
+  if (u.gather) {
+    switch (mode) {
+      case 1: return launch_site<T, 1>(u, con, x, d, t, g, rs, s);
+      case 2: return launch_site<T, 2>(u, con, x, d, t, g, rs, s);
+      case 3: return launch_site<T, 3>(u, con, x, d, t, g, rs, s);
+      case 5: return launch_site<T, 5>(u, con, x, d, t, g, rs, s);
+      default: throw std::invalid_argument("pfu: unsupported evaluation mode");
+    }
+  }
+  const int nb = chunk_blocks(u);
+  switch (mode) {
+    case 1: launch_chunk<T, 1>(u, nb, x, d, t, g, rs, s); break;
+    case 2: launch_chunk<T, 2>(u, nb, x, d, t, g, rs, s); break;
+    case 3: launch_chunk<T, 3>(u, nb, x, d, t, g, rs, s); break;
+    case 5: launch_chunk<T, 5>(u, nb, x, d, t, g, rs, s); break;
+    default: throw std::invalid_argument("pfu: unsupported evaluation mode");
+  }
+  if ((mode & 2) && u.ngather)
+    pfu_gather_kernel<T><<<grid_blocks(u.ngather * u.nf, 1, 8192), kBlock, 0, s>>>(u, g);
+  return nb;
+}
+
+template <typename T>
+void eval_t(const PFUArgs& u, const PFArgs& con, int mode, const void* x, const void* d, double t, void* g,
+            RedScratch rs, hipStream_t s, double* eOut) {
   const T* xx = static_cast<const T*>(x);
   const T* dd = static_cast<const T*>((mode & 4) ? d : x);
   T* gg = static_cast<T*>(g);
   const T tt = (T)t;
   const size_t nd = u.ngrid * u.nf;
-  const int nb = chunk_blocks(u);
-  switch (mode) {
-    case 1: launch_chunk<T, 1>(u, nb, xx, dd, tt, gg, rs, s); break;
-    case 2: launch_chunk<T, 2>(u, nb, xx, dd, tt, gg, rs, s); break;
-    case 3: launch_chunk<T, 3>(u, nb, xx, dd, tt, gg, rs, s); break;
-    case 5: launch_chunk<T, 5>(u, nb, xx, dd, tt, gg, rs, s); break;
-    default: throw std::invalid_argument("pfu: unsupported evaluation mode");
-  }
-  if ((mode & 2) && u.ngather)
-    pfu_gather_kernel<T><<<grid_blocks(u.ngather * u.nf, 1, 8192), kBlock, 0, s>>>(u, gg);
-  launch_finalize(rs, 2, nb, s);
+  const int nb = launch_elements<T>(u, con, mode, xx, dd, tt, gg, rs, s);
+  MINIM_HIP_CHECK(hipGetLastError());
+  launch_finalize(rs, 1, nb, s, 0, (mode & 1) && !u.volfix ? eOut : nullptr);
   if (u.volfix) {
     RedScratch slot{rs.partials, rs.result + kPFVolSlot};
     const int nbv = grid_blocks(u.ngrid, 4, 2048);
@@ -367,47 +708,39 @@ void eval_t(const PFUArgs& u, int mode, const void* x, const void* d, double t, 
     else
       pfu_volumes_kernel<T, T, false><<<nbv, kBlock, 0, s>>>(u, xx, dd, tt, slot);
     launch_finalize(slot, kPFMaxFluid, nbv, s);
-    pfu_volfix_kernel<<<1, 64, 0, s>>>(u, rs.result + kPFVolSlot, rs.result, (mode & 1) ? 1 : 0);
+    pfu_volfix_kernel<<<1, 64, 0, s>>>(u, rs.result + kPFVolSlot, rs.result, (mode & 1) ? 1 : 0,
+                                       (mode & 1) ? eOut : nullptr);
     if (mode & 2) pfu_volgrad_kernel<T, T, false><<<grid_blocks(nd, 4, 4096), kBlock, 0, s>>>(u, xx, dd, tt, gg);
+    MINIM_HIP_CHECK(hipGetLastError());
   }
+  // the site kernel has projected the elements' gradient; the projection of
+  // what the volume term adds to it gives the projection of the sum
+  if ((mode & 2) && (!u.gather || u.volfix)) pf_launch_constrain(con, sizeof(T) == 8 ? F64 : F32, gg, u.ngrid, rs, s);
 }
 
 }  // namespace
 
-void pfu_launch_eval(const PFUArgs& u, int prec, int mode, const void* x, const void* d, double t, void* g,
-                     RedScratch rs, hipStream_t s) {
+void pfu_launch_eval(const PFUArgs& u, const PFArgs& con, int prec, int mode, const void* x, const void* d, double t,
+                     void* g, RedScratch rs, hipStream_t s, double* eOut) {
   if ((mode & 4) && (mode & 2)) throw std::invalid_argument("pfu: gradients at a trial point are not supported");
   if (u.ngrid * (size_t)u.nf >= (size_t)1 << 31) throw std::invalid_argument("pfu: more than 2^31 DOFs");
-  if (prec == F64) eval_t<double>(u, mode, x, d, t, g, rs, s);
-  else eval_t<float>(u, mode, x, d, t, g, rs, s);
-  MINIM_HIP_CHECK(hipGetLastError());
+  if (prec == F64) eval_t<double>(u, con, mode, x, d, t, g, rs, s, eOut);
+  else eval_t<float>(u, con, mode, x, d, t, g, rs, s, eOut);
 }
 
-double pfu_time_elements(const PFUArgs& u, int prec, int mode, const void* x, void* g, int reps, RedScratch rs,
-                         hipStream_t s) {
-  const int nb = chunk_blocks(u);
+double pfu_time_elements(const PFUArgs& u, const PFArgs& con, int prec, int mode, const void* x, void* g, int reps,
+                         RedScratch rs, hipStream_t s) {
   auto launch = [&]() {
     if (prec == F64) {
       const double* xx = static_cast<const double*>(x);
-      if (mode == 1) {
-        launch_chunk<double, 1>(u, nb, xx, xx, 0.0, (double*)g, rs, s);
-      } else {
-        launch_chunk<double, 3>(u, nb, xx, xx, 0.0, (double*)g, rs, s);
-        if (u.ngather)
-          pfu_gather_kernel<double><<<grid_blocks(u.ngather * u.nf, 1, 8192), kBlock, 0, s>>>(u, (double*)g);
-      }
+      launch_elements<double>(u, con, mode == 1 ? 1 : 3, xx, xx, 0.0, (double*)g, rs, s);
     } else {
       const float* xx = static_cast<const float*>(x);
-      if (mode == 1) {
-        launch_chunk<float, 1>(u, nb, xx, xx, 0.0f, (float*)g, rs, s);
-      } else {
-        launch_chunk<float, 3>(u, nb, xx, xx, 0.0f, (float*)g, rs, s);
-        if (u.ngather)
-          pfu_gather_kernel<float><<<grid_blocks(u.ngather * u.nf, 1, 8192), kBlock, 0, s>>>(u, (float*)g);
-      }
+      launch_elements<float>(u, con, mode == 1 ? 1 : 3, xx, xx, 0.0f, (float*)g, rs, s);
     }
   };
   launch();
+  MINIM_HIP_CHECK(hipGetLastError());
   hipEvent_t e0, e1;
   MINIM_HIP_CHECK(hipEventCreate(&e0));
   MINIM_HIP_CHECK(hipEventCreate(&e1));

@@ -22,6 +22,16 @@ constexpr uint32_t kPFUShared = 0x80000000u;  // site-table flag: other chunks t
 // type (8 bits) and the fluid (8 bits).  Surface, force and confinement
 // elements carry their parameters in par, through pidx.
 struct PFUArgs {
+  // the elements of every site gathered per site (pfu_site_kernel) instead of
+  // through the list below: canonical grid (size-1 dimensions first), per-site
+  // forward-bond code (pf.hpp) when there are solid nodes, volume of a bulk
+  // site, bulk and gradient factors of a bulk site, soft constraint
+  int gather;
+  int X, Y, Z;
+  const uint32_t* wcode;
+  double v1;
+  double fb[4], fg[4];
+  int soft;
   size_t nel;
   int nchunk;
   const uint4* rec;           // nel
@@ -54,14 +64,14 @@ struct PFUArgs {
   double* volg;            // nf factors volCoef * volDiff (device scratch)
 };
 
-// Energy (rs.result[0]) and/or gradient (g, unconstrained) of every element
-// and the volume term, at x or x + t*d.  prec is the storage precision of x,
-// d and g.
-void pfu_launch_eval(const PFUArgs& u, int prec, int mode, const void* x, const void* d, double t, void* g,
-                     RedScratch rs, hipStream_t s);
+// Energy (rs.result[0], and eOut when given) and/or constrained gradient g
+// (con: the per-site projection) of every element and the volume term, at x or
+// x + t*d.  prec is the storage precision of x, d and g.
+void pfu_launch_eval(const PFUArgs& u, const PFArgs& con, int prec, int mode, const void* x, const void* d, double t,
+                     void* g, RedScratch rs, hipStream_t s, double* eOut = nullptr);
 // Average duration (ms) of reps launches of the element kernel (with the
 // gather pass of the shared sites when mode has the gradient).
-double pfu_time_elements(const PFUArgs& u, int prec, int mode, const void* x, void* g, int reps, RedScratch rs,
+double pfu_time_elements(const PFUArgs& u, const PFArgs& con, int prec, int mode, const void* x, void* g, int reps, RedScratch rs,
                          hipStream_t s);
 
 }  // namespace minim_amd

@@ -121,6 +121,76 @@ std::vector<int> pf_site_types(const int grid[3], const char* solid) {
   return type;
 }
 
+// Canonical dimensions of a grid: size-1 dimensions dropped to the front (the
+// linear index is kept).  cmap[j] is the grid dimension of canonical
+// dimension j, or -1.
+void pf_canonical(const int grid[3], int canon[3], int cmap[3]) {
+  int nd = 0, dims[3];
+  for (int i = 0; i < 3; i++)
+    if (grid[i] > 1) dims[nd++] = i;
+  for (int j = 0; j < 3; j++) cmap[j] = -1;
+  for (int i = 0; i < nd; i++) cmap[3 - nd + i] = dims[i];
+  for (int j = 0; j < 3; j++) canon[j] = cmap[j] >= 0 ? grid[cmap[j]] : 1;
+}
+
+// Per-site codes of a layout with solid nodes (kinds: 0 solid, 1 + the
+// surface type): the per-side bond weights (code) and the forward-bond
+// weights (wcode), as described in pf.hpp.
+void pf_bond_codes(const int grid[3], const char* solid, const std::vector<int>& kinds, std::vector<uint16_t>* codeOut,
+                   std::vector<uint32_t>& wcode) {
+  const size_t ng = kinds.size();
+  int canon[3], cmap[3];
+  pf_canonical(grid, canon, cmap);
+  // bond weights per canonical dimension: 0 towards a solid site, 1 towards
+  // the fluid side when the other neighbour is solid, else one half
+  std::vector<uint16_t> code(ng);
+  const int n0 = grid[0], n1 = grid[1], n2 = grid[2];
+  for (int x = 0; x < n0; x++)
+    for (int y = 0; y < n1; y++)
+      for (int z = 0; z < n2; z++) {
+        const size_t i = ((size_t)x * n1 + y) * n2 + z;
+        unsigned q = (unsigned)kinds[i];
+        if (!solid[i]) {
+          for (int j = 0; j < 3; j++) {
+            const int dd = cmap[j];
+            if (dd < 0) continue;
+            int cm[3] = {x, y, z}, cp[3] = {x, y, z};
+            cm[dd] = (cm[dd] - 1 + grid[dd]) % grid[dd];
+            cp[dd] = (cp[dd] + 1) % grid[dd];
+            const bool sm = solid[((size_t)cm[0] * n1 + cm[1]) * n2 + cm[2]] != 0;
+            const bool sp = solid[((size_t)cp[0] * n1 + cp[1]) * n2 + cp[2]] != 0;
+            const unsigned hm = sm ? 0u : (sp ? 2u : 1u);
+            const unsigned hp = sp ? 0u : (sm ? 2u : 1u);
+            q |= hm << (minim_amd::kPFCodeShift + 4 * j);
+            q |= hp << (minim_amd::kPFCodeShift + 4 * j + 2);
+          }
+        }
+        code[i] = (uint16_t)q;
+      }
+  // forward-bond weights for the tiled kernel: w(i, i+e) = (v_i h_i->i+e +
+  // v_{i+e} h_{i+e}->i) / res^3 in sixteenths (v/res^3 in eighths, h in halves)
+  wcode.resize(ng);
+  auto v8 = [](unsigned q) { const unsigned k = q & 15u; return k >= 2 ? k - 1 : 8 * k; };
+  auto hq = [](unsigned q, int j, int side) { return (q >> (minim_amd::kPFCodeShift + 4 * j + 2 * side)) & 3u; };
+  for (int x = 0; x < n0; x++)
+    for (int y = 0; y < n1; y++)
+      for (int z = 0; z < n2; z++) {
+        const size_t i = ((size_t)x * n1 + y) * n2 + z;
+        uint32_t w = (uint32_t)kinds[i];
+        for (int j = 0; j < 3; j++) {
+          const int dd = cmap[j];
+          if (dd < 0) continue;
+          int cp[3] = {x, y, z};
+          cp[dd] = (cp[dd] + 1) % grid[dd];
+          const size_t ip = ((size_t)cp[0] * n1 + cp[1]) * n2 + cp[2];
+          const unsigned w16 = v8(code[i]) * hq(code[i], j, 1) + v8(code[ip]) * hq(code[ip], j, 0);
+          w |= w16 << (minim_amd::kPFWeightShift + minim_amd::kPFWeightBits * j);
+        }
+        wcode[i] = w;
+      }
+  if (codeOut) *codeOut = std::move(code);
+}
+
 PhaseField& PhaseField::setNFluid(int n) {
   nFluid = n;
   dofPerNode = n;  // PhaseField.cpp:753-757
@@ -409,12 +479,8 @@ void PhaseField::init(const vector<double>& coords) {
   PFArgs& A = h->a;
   A = PFArgs{};
   // canonical grid: drop size-1 dimensions to the front (keeps the linear index)
-  int cmap[3] = {-1, -1, -1}, nd = 0, dims[3];
-  for (int i = 0; i < 3; i++)
-    if (gridSize[i] > 1) dims[nd++] = i;
-  for (int i = 0; i < nd; i++) cmap[3 - nd + i] = dims[i];
-  int canon[3];
-  for (int j = 0; j < 3; j++) canon[j] = cmap[j] >= 0 ? gridSize[cmap[j]] : 1;
+  int canon[3], cmap[3];
+  pf_canonical(gridSize.data(), canon, cmap);
   A.X = canon[0];
   A.Y = canon[1];
   A.Z = canon[2];
@@ -469,53 +535,9 @@ void PhaseField::init(const vector<double>& coords) {
       nodeVol[i] = E.vol[kinds[i]];
       surfaceArea[i] = E.area[kinds[i]];
     }
-    // bond weights per canonical dimension: 0 towards a solid site, 1 towards
-    // the fluid side when the other neighbour is solid, else one half
-    std::vector<uint16_t> code(ng);
-    const int n0 = gridSize[0], n1 = gridSize[1], n2 = gridSize[2];
-    for (int x = 0; x < n0; x++)
-      for (int y = 0; y < n1; y++)
-        for (int z = 0; z < n2; z++) {
-          const size_t i = ((size_t)x * n1 + y) * n2 + z;
-          unsigned q = (unsigned)kinds[i];
-          if (!solid[i]) {
-            for (int j = 0; j < 3; j++) {
-              const int dd = cmap[j];
-              if (dd < 0) continue;
-              int cm[3] = {x, y, z}, cp[3] = {x, y, z};
-              cm[dd] = (cm[dd] - 1 + gridSize[dd]) % gridSize[dd];
-              cp[dd] = (cp[dd] + 1) % gridSize[dd];
-              const bool sm = solid[((size_t)cm[0] * n1 + cm[1]) * n2 + cm[2]] != 0;
-              const bool sp = solid[((size_t)cp[0] * n1 + cp[1]) * n2 + cp[2]] != 0;
-              const unsigned hm = sm ? 0u : (sp ? 2u : 1u);
-              const unsigned hp = sp ? 0u : (sm ? 2u : 1u);
-              q |= hm << (minim_amd::kPFCodeShift + 4 * j);
-              q |= hp << (minim_amd::kPFCodeShift + 4 * j + 2);
-            }
-          }
-          code[i] = (uint16_t)q;
-        }
-    // forward-bond weights for the tiled kernel: w(i, i+e) = (v_i h_i->i+e +
-    // v_{i+e} h_{i+e}->i) / res^3 in sixteenths (v/res^3 in eighths, h in halves)
-    std::vector<uint32_t> wcode(ng);
-    auto v8 = [](unsigned q) { const unsigned k = q & 15u; return k >= 2 ? k - 1 : 8 * k; };
-    auto hq = [](unsigned q, int j, int side) { return (q >> (minim_amd::kPFCodeShift + 4 * j + 2 * side)) & 3u; };
-    for (int x = 0; x < n0; x++)
-      for (int y = 0; y < n1; y++)
-        for (int z = 0; z < n2; z++) {
-          const size_t i = ((size_t)x * n1 + y) * n2 + z;
-          uint32_t w = (uint32_t)kinds[i];
-          for (int j = 0; j < 3; j++) {
-            const int dd = cmap[j];
-            if (dd < 0) continue;
-            int cp[3] = {x, y, z};
-            cp[dd] = (cp[dd] + 1) % gridSize[dd];
-            const size_t ip = ((size_t)cp[0] * n1 + cp[1]) * n2 + cp[2];
-            const unsigned w16 = v8(code[i]) * hq(code[i], j, 1) + v8(code[ip]) * hq(code[ip], j, 0);
-            w |= w16 << (minim_amd::kPFWeightShift + minim_amd::kPFWeightBits * j);
-          }
-          wcode[i] = w;
-        }
+    std::vector<uint16_t> code;
+    std::vector<uint32_t> wcode;
+    pf_bond_codes(gridSize.data(), solid.data(), kinds, &code, wcode);
     h->code_h = std::move(code);
     h->wcode_h = std::move(wcode);
   }

@@ -2,9 +2,9 @@
 against the oracle, the reference's unit-test known answers
 (test/unit/PhaseFieldUnstructured_test.cpp) and the gather-form PhaseField.
 
-Within a chunk of elements the gradient is accumulated with LDS atomics, so
-its summation order (and, in the last bits, its value) varies from launch to
-launch.  Tolerances: FP64 within
+Within a chunk of the element list the gradient is accumulated with LDS
+atomics, so its summation order (and, in the last bits, its value) varies from
+launch to launch; the per-site form has a fixed order.  Tolerances: FP64 within
 1e-12 relative (gradients norm-wise; energies relative to the sum of the
 magnitudes of the energy terms), FP32 within 1e-5, on identical (for FP32:
 FP32-rounded) coordinates.
@@ -326,3 +326,57 @@ def test_element_form_mixed_schedule_widens(gpu):
         assert lb.stats["converged"], mode
         res[mode] = o.energy(x)
     assert abs(res["mixed"] - res["fp64"]) <= 1e-6 * max(1.0, abs(res["fp64"]))
+
+
+# the soft constraint is refused with two fluids and goes through the list with four
+PER_SITE = [(g, nf, density)
+            for g, nf in [((1, 1, 5), 1), ((2, 3, 4), 3), ((1, 65, 64), 2), ((3, 17, 66), 4), ((5, 16, 129), 3),
+                          ((9, 33, 63), 1), ((2, 2, 130), 2), ((70, 8, 9), 3)]
+            for density in ("hard", "none", "soft") if not (density == "soft" and nf in (2, 4))]
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("layout", ["plain", "pressure", "solid"])
+@pytest.mark.parametrize("grid,nf,density", PER_SITE)
+def test_elements_gathered_per_site_vs_oracle(gpu, grid, nf, density, layout, prec):
+    """The per-site form around its tile edges: energy and gradient (together
+    and alone) and the trial energy, against the oracle's element list.  Solid
+    sites hold NaN, which no element reads."""
+    import torch
+
+    m = gpu
+    print("case pfu per site", grid, nf, density, layout, prec, flush=True)
+    rng = np.random.default_rng(sum(grid) + nf)
+    opts = {}
+    solid = None
+    if layout != "plain":
+        opts["pressure"] = [0.5, -0.25, 0.0, 0.75][:nf]
+    if layout == "solid":
+        solid = structured_solid(grid, rng, "pillar" if min(grid) > 1 else "wall")
+        opts["solid"] = solid
+    if nf > 1:
+        opts["fix_fluid"] = [False, True, False, False][:nf]
+    c = dict(grid=grid, nfluid=nf, resolution=0.8, surface_tension=[1.0, 0.8, 1.2, 0.9][:nf], interface_size=[1.5],
+             density=density, opts=opts)
+    n = int(np.prod(grid)) * nf
+    x = rng.uniform(0, 1, n).astype(np.float32).astype(np.float64)
+    d = rng.uniform(-0.2, 0.2, n).astype(np.float32).astype(np.float64)
+    c["x0"] = x
+    o = oracle_of(c)
+    h = device_pf(m, c, "PhaseFieldUnstructured").handle(x)
+    assert m.PhaseFieldUnstructured.elementList(None, handle=h)[0] == o.nelements
+    dt = torch.float64 if prec == "fp64" else torch.float32
+    xh = x.copy()
+    if solid is not None:
+        xh.reshape(-1, nf)[solid.astype(bool)] = np.nan
+    xd = torch.tensor(xh, dtype=dt, device="cuda")
+    dd = torch.tensor(d, dtype=dt, device="cuda")
+    g, g2 = torch.empty_like(xd), torch.empty_like(xd)
+    e = m.potential_eval(h, prec, xd.data_ptr(), n, g_ptr=g.data_ptr())
+    m.potential_eval(h, prec, xd.data_ptr(), n, g_ptr=g2.data_ptr(), want_energy=False)
+    e1 = m.potential_eval(h, prec, xd.data_ptr(), n)
+    et = m.potential_eval(h, prec, xd.data_ptr(), n, d_ptr=dd.data_ptr(), t=0.5)
+    assert e == e1 and torch.equal(g, g2)
+    assert rel_err(g.cpu().numpy(), o.gradient(x)) <= TOL[prec]
+    for got, at in ((e, x), (et, x + 0.5 * d)):
+        assert abs(got - o.energy(at)) <= TOL[prec] * max(energy_scale(c, at), abs(o.energy(at)))
