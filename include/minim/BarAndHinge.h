@@ -41,9 +41,9 @@ class BarAndHinge : public NewPotential<BarAndHinge> {
   void evaluateMixedAsync(const void* x, const void* d, double t, bool wantE, double* e_dev, void* g,
                           void* stream) const override;
   // Fused accepted step: x + t*d into xout (formed as the line-search trials
-  // form it), then energy and gradient there in one energy pass that keeps
-  // what the gradient gather needs; d and g in precision pv (px, or FP32
-  // against FP64 coordinates without normal constraints).
+  // form it) and the energy there, with the gradient unless g is null; d and g
+  // in precision pv (px, or FP32 against FP64 coordinates without normal
+  // constraints).
   bool supportsStep() const override;
   bool stepDefersGradient() const override;
   void evaluateStepAsync(int px, int pv, const void* x, const void* d, double t, void* xout, void* g,
@@ -68,7 +68,9 @@ class BarAndHinge : public NewPotential<BarAndHinge> {
   vector2d<int> tri_, bonds_, hinges_;
   vector<double> kBond_, kHinge_, length0_, theta0_, force_;
   std::shared_ptr<Dev> dev_;
+  std::shared_ptr<const vector<int>> order_;  // the nodes in cluster order
   void upload();
+  bool maskHolds() const;
 };
 
 }  // namespace minim

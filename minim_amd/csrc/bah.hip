@@ -5,21 +5,16 @@
 // 0.5*k*dl^2 energy), bending (:293-356) and forceEnergy (:359-369); element
 // order and the all-DOFs-fixed skip follow BarAndHinge::init (:16-67).
 //
-// The reference loops over heap elements and scatters into g.  Here the
-// energy is one thread per element with an FP64 reduction, and the gradient is
-// gathered: one thread per node walks its incident bars and hinges (CSR built
-// once on the host, in element order) and adds each element's contribution to
-// that node, so every gradient entry is written once, without atomics, in a
-// fixed order.  A bar's contribution is recomputed at each of its two nodes.
-// For a hinge, the energy pass (or, for a gradient without energy, the hinge
-// pass) stores per hinge what the gather needs beyond the node positions:
-// in FP32 the terms its four nodes share -- k dtheta times each scaled
-// normal, and the two skews (8 values) -- so that the gather recomputes no
-// geometry; in FP64 only the angle deviation, the gather recomputing the
-// geometry at each node.  Measured at 1024^2 nodes: FP32 gather 114 -> 77 us
-// with the terms (energy pass 54 -> 70 us); FP64 gather 158 -> 149 us but
-// energy pass 78 -> 127 us (64 B instead of 8 B written per hinge), so FP64
-// keeps the angle alone.
+// The reference loops over heap elements and scatters into g.  Here a block
+// takes a cluster of up to 128 nodes (bah_mesh.hpp), stages the positions that
+// its elements need in LDS, evaluates each bar and hinge that touches the
+// cluster once, keeps the terms that the element's nodes share in LDS, and
+// then one thread per own node adds the terms of its elements in the order of
+// the element lists.  Energy and gradient come from the same pass, every
+// gradient entry is written once, and there are no atomics and no per-element
+// stores: bitwise reproducible.  At 1024^2 nodes, energy and gradient: 116 us in
+// FP64 and 72 in FP32; an energy pass that stored each hinge's angle, then a
+// gather per node that recomputed four hinges per hinge, took 240 and 150.
 //
 // Rigidities, rest lengths and rest angles that are the same for every
 // element are passed as scalars instead of per-element streams.
@@ -29,10 +24,9 @@
 // acos's loss of precision near 0 and pi.
 #include <algorithm>
 #include <cmath>
-#include <map>
 #include <stdexcept>
-#include <unordered_map>
 
+#include "bah_mesh.hpp"
 #include "common.hpp"
 #include "minim/BarAndHinge.h"
 #include "runtime.hpp"
@@ -42,34 +36,27 @@ namespace minim_amd {
 namespace {
 
 struct BaHArgs {
-  int nnode, nbar, nhinge;
-  const int* bar;     // 2 per bar
-  const double* bk;   // per bar, or null: every bar has bkU
-  const double* bl0;  // ... bl0U
-  const int* hinge;   // 4 per hinge
-  const double* hk;   // per hinge, or null: hkU
-  const double* ht0;  // ... ht0U
+  int nnode, ncluster, nchunk;
+  const BaHChunk* chunk;
+  const int* cluster;    // first chunk of each cluster
+  const int* node;       // node tables
+  const double* bk;      // per bar code, or null: every bar has bkU
+  const double* bl0;     // ... bl0U
+  const ushort4* hinge;
+  const double* hk;      // per hinge record, or null: hkU
+  const double* ht0;     // ... ht0U
   double bkU, bl0U, hkU, ht0U;
-  const int* bptr;    // node -> incident bars CSR (nnode+1)
-  const int* bidx;    // (bar << 1) | local
-  const int* hptr;    // node -> incident hinges CSR
-  const int* hidx;    // (hinge << 2) | local
-  const double* fz;   // per-node z force or nullptr
-  const unsigned char* nodeActive;  // force element exists for the node
+  const ushort4* bcode;  // BaHCodes, four codes each
+  const ushort4* hcode;
+  const double* fz;      // per node (cluster order) z force or nullptr
+  const unsigned char* flags;  // per node (cluster order): bits 0-2 the fixed components, bit 3 the force exists
 };
 
-template <typename T>
-__device__ inline void ld3(const T* __restrict__ x, const T* __restrict__ d, T t, int n, T (&p)[3]) {
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    T c = x[(size_t)n * 3 + k];
-    if (d) {
-      T s = t * d[(size_t)n * 3 + k];
-      c = c + s;
-    }
-    p[k] = c;
-  }
-}
+// flags
+constexpr unsigned char kForced = 8;
+
+// Parts of the energy (componentEnergy asks for one of them).
+enum BaHParts : int { kBars = 1, kHinges = 2, kForces = 4, kAllParts = 7 };
 
 template <typename T>
 __device__ inline void cross(const T (&a)[3], const T (&b)[3], T (&c)[3]) {
@@ -82,6 +69,40 @@ template <typename T>
 __device__ inline T dot3(const T (&a)[3], const T (&b)[3]) {
   return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
 }
+
+// Correctly rounded FP64 quotients and roots as the compiler's, without its
+// scaling of operands near the ends of the exponent range (12 and 22
+// instructions become 8 and 13).  The operands here are lengths to the powers
+// 1 to 4; the angle's cosine already takes one to the power 8.  A reciprocal by
+// Newton's iteration, then one correction by the exact remainder (Markstein,
+// IA-64 and Elementary Functions, 2000, ch. 8 and 9).
+__device__ inline double reciprocal(double b) {
+  double r = __builtin_amdgcn_rcp(b);
+  r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+}
+__device__ inline float reciprocal(float b) { return b; }
+// a / b, with r = reciprocal(b)
+__device__ inline double quotient(double a, double b, double r) {
+  const double q = a * r;
+  return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+}
+__device__ inline float quotient(float a, float b, float) { return a / b; }
+template <typename T>
+__device__ inline T quotient(T a, T b) {
+  return quotient(a, b, reciprocal(b));
+}
+__device__ inline double root(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, e, g);
+  h = __builtin_fma(h, e, h);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  return x == 0.0 || x == __builtin_inf() ? x : g;
+}
+__device__ inline float root(float x) { return sqrt(x); }
 
 // Hinge geometry shared by energy and gradient.
 template <typename T>
@@ -100,7 +121,7 @@ __device__ inline void hinge_geo_vec(const T (&x1)[3], const T (&x2)[3], const T
     G.b2[k] = x3[k] - x2[k];
     G.b3[k] = x4[k] - x3[k];
   }
-  G.b2m = sqrt(dot3(G.b2, G.b2));
+  G.b2m = root(dot3(G.b2, G.b2));
   cross(G.b1, G.b2, G.n1);
   cross(G.b2, G.b3, G.n2);
   G.n1sq = dot3(G.n1, G.n1);
@@ -114,7 +135,7 @@ __device__ inline void hinge_dtheta(HingeGeo<T>& G, T t0) {
   const T pi = (T)3.14159265358979323846;
   T theta;
   if (sizeof(T) == 8) {
-    T c = dot3(G.n1, G.n2) / sqrt(G.n1sq * G.n2sq);
+    T c = quotient(dot3(G.n1, G.n2), root(G.n1sq * G.n2sq));
     c = c < (T)-1 ? (T)-1 : c;
     c = c > (T)1 ? (T)1 : c;
     theta = (n1b3 >= 0) ? acos(c) : (T)2 * pi - acos(c);
@@ -133,252 +154,253 @@ __device__ inline void hinge_dtheta(HingeGeo<T>& G, T t0) {
   G.dtheta = r - pi;
 }
 
-// Hinge geometry from the four node positions and the rest angle.
+// A hinge's gradient at its four nodes (BarAndHinge.cpp:336-354).  With
+// A = k dtheta |b2| n1 / |n1|^2, B = k dtheta |b2| n2 / |n2|^2,
+// skew1 = -b1.b2 / |b2|^2, skew2 = -b3.b2 / |b2|^2: node 0 gets -A, node 1
+// (1 - skew1) A - skew2 B, node 2 skew1 A - (1 - skew2) B, node 3 B.
 template <typename T>
-__device__ inline void hinge_geo_at(const T (&x1)[3], const T (&x2)[3], const T (&x3)[3], const T (&x4)[3], T t0,
-                                    HingeGeo<T>& G) {
-  hinge_geo_vec(x1, x2, x3, x4, G);
-  hinge_dtheta(G, t0);
-}
-
-// Node positions and rest angle of hinge h (one int4 of node ids).
-template <typename T>
-struct HingeIn {
-  T x1[3], x2[3], x3[3], x4[3];
-  T t0, k;
-};
-
-template <typename T>
-__device__ inline void hinge_load(const T* __restrict__ x, const T* __restrict__ d, T t, const BaHArgs& a, int h,
-                                  HingeIn<T>& H) {
-  const int4 nd = reinterpret_cast<const int4*>(a.hinge)[h];
-  ld3(x, d, t, nd.x, H.x1);
-  ld3(x, d, t, nd.y, H.x2);
-  ld3(x, d, t, nd.z, H.x3);
-  ld3(x, d, t, nd.w, H.x4);
-  H.t0 = (T)(a.ht0 ? a.ht0[h] : a.ht0U);
-  H.k = (T)(a.hk ? a.hk[h] : a.hkU);
-}
-
-// A hinge's gradient (BarAndHinge.cpp:336-354) through the terms its four
-// nodes share: A = k dtheta |b2| n1 / |n1|^2, B = k dtheta |b2| n2 / |n2|^2,
-// skew1 = -b1.b2 / |b2|^2, skew2 = -b3.b2 / |b2|^2 (8 values, HingeTerms);
-// node 0 gets -A, node 1 (1 - skew1) A - skew2 B, node 2 skew1 A - (1 - skew2) B,
-// node 3 B.
-template <typename T>
-struct alignas(sizeof(T) * 4) HingeTerms {
-  T A[3], s1, B[3], s2;
-};
-
-template <typename T>
-__device__ inline void hinge_terms(const HingeGeo<T>& G, T k, HingeTerms<T>& H) {
+__device__ inline void hinge_gradient(const HingeGeo<T>& G, T k, T (&f)[4][3]) {
   const T gf = k * (G.dtheta);
-  const T f1 = G.b2m / G.n1sq, f2 = G.b2m / G.n2sq;
+  const T f1 = quotient(G.b2m, G.n1sq), f2 = quotient(G.b2m, G.n2sq);
+  const T bb = G.b2m * G.b2m, rb = reciprocal(bb);
+  const T s1 = quotient(-dot3(G.b1, G.b2), bb, rb);
+  const T s2 = quotient(-dot3(G.b3, G.b2), bb, rb);
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    H.A[c] = gf * (f1 * G.n1[c]);
-    H.B[c] = gf * (f2 * G.n2[c]);
-  }
-  const T bb = G.b2m * G.b2m;
-  H.s1 = -dot3(G.b1, G.b2) / bb;
-  H.s2 = -dot3(G.b3, G.b2) / bb;
-}
-
-// What the energy or hinge pass stores per hinge for the gradient gather.
-template <typename T>
-struct HingeStore {
-  using type = T;  // FP64: the angle deviation
-};
-template <>
-struct HingeStore<float> {
-  using type = HingeTerms<float>;
-};
-template <typename T>
-using HStore = typename HingeStore<T>::type;
-template <typename T>
-constexpr bool kHingeTerms = sizeof(HStore<T>) != sizeof(T);
-
-template <typename T>
-__device__ inline void hinge_store(const HingeGeo<T>& G, T k, HStore<T>* __restrict__ out, size_t h) {
-  if constexpr (kHingeTerms<T>) {
-    HingeTerms<T> tm;
-    hinge_terms(G, k, tm);
-    out[h] = tm;
-  } else {
-    out[h] = G.dtheta;
+    const T A = gf * (f1 * G.n1[c]);
+    const T B = gf * (f2 * G.n2[c]);
+    f[0][c] = -A;
+    f[1][c] = ((T)1 - s1) * A - s2 * B;
+    f[2][c] = s1 * A - ((T)1 - s2) * B;
+    f[3][c] = B;
   }
 }
 
+// Barrier that orders LDS traffic only (no wait on outstanding global accesses).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// What a thread reads for a chunk: one node of the table, two hinge records,
+// and the first codes of the node that it adds up.
+template <typename T, typename TV>
+struct ChunkIn {
+  T x[3];
+  TV d[3];
+  int node;
+  ushort4 hinge[2], bcode, hcode[2];
+};
+
+// The neighbouring lane's value (lanes 2 i and 2 i + 1 exchange).
+__device__ inline int swap_pair(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true); }
+__device__ inline float swap_pair(float v) { return __int_as_float(swap_pair(__float_as_int(v))); }
+__device__ inline double swap_pair(double v) {
+  return __hiloint2double(swap_pair(__double2hiint(v)), swap_pair(__double2loint(v)));
+}
+
+// Adds the four terms of this lane, then the four of its neighbour: in the even
+// lane of a pair, the order of the codes.
 template <typename T>
-__device__ inline void hinge_grad_at(const HingeTerms<T>& H, int loc, T (&gn)[3]) {
+__device__ inline void add_pair(T (&sum)[3], const T (&f)[4][3]) {
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
-    T v;
-    if (loc == 0) v = -H.A[c];
-    else if (loc == 1) v = ((T)1 - H.s1) * H.A[c] - H.s2 * H.B[c];
-    else if (loc == 2) v = H.s1 * H.A[c] - ((T)1 - H.s2) * H.B[c];
-    else v = H.B[c];
-    gn[c] += v;
-  }
+  for (int v = 0; v < 4; v++)
+#pragma unroll
+    for (int m = 0; m < 3; m++) sum[m] += f[v][m];
+#pragma unroll
+  for (int v = 0; v < 4; v++)
+#pragma unroll
+    for (int m = 0; m < 3; m++) sum[m] += swap_pair(f[v][m]);
 }
 
-// Energy: bars, then hinges, then the external force, each a grid-stride
-// loop that takes U elements per step and issues all their loads first.
-// With SD, each hinge's gradient terms also go to ht (for the gradient
-// kernel, which then recomputes no hinge geometry).
-template <typename T, bool SD>
-__global__ __launch_bounds__(kBlock) void bah_energy_kernel(BaHArgs a, const T* __restrict__ x,
-                                                            const T* __restrict__ d, T t, RedScratch rs,
-                                                            HStore<T>* __restrict__ ht) {
-  constexpr int U = 4;
+// Blocks of a launch: as many as are resident at once (LDS and registers let
+// three FP64 and five FP32 blocks share a CU), each with an equal run of clusters.
+template <typename T>
+constexpr int kBaHBlocks = 256 * (sizeof(T) == 8 ? 3 : 5);
+
+// The whole evaluation: a block works through its run of clusters (runs are
+// contiguous per XCD: neighbours share nodes in one L2).  E, G: the energy, the
+// gradient.  d: evaluate at x + t*d (as axpy forms it), which also goes to xout
+// when given.  TV: the storage of d and g (FP32 for FP64 arithmetic in the
+// mixed schedule).  mask: fixed components of the gradient are zero.
+//
+// Per chunk: positions to LDS, barrier, bars (at each end: two threads per
+// node, every other entry of its codes) and hinges (two per thread), whose
+// forces on their four nodes go to LDS component by component, barrier, then a
+// node's two threads fetch its hinges' forces, and the even one adds them up,
+// bars and hinges in the order of the lists.  The next chunk's reads are in
+// flight during all of it, two barriers per chunk.
+//
+// Bound by VALU issue: 1,190 instructions per wave and chunk in FP64, 74 % of
+// the time of the three blocks per CU (one chunk per block without the reads
+// ahead, with bars in LDS and four barriers: 54 %, 155 us at 1024^2 nodes; eight
+// terms per hinge in LDS that each node combined itself: 160 us).  FP64 blocks
+// stand three to a CU by their 52 KB of LDS and 150 registers.
+template <typename T, typename TV, bool E, bool G>
+__global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 5) void bah_kernel(
+    BaHArgs a, const BaHChunk* __restrict__ chunks, const int* __restrict__ nodes, const T* __restrict__ x,
+    const TV* __restrict__ d, T t, T* __restrict__ xout, TV* __restrict__ g, bool mask, int parts, RedScratch rs) {
+  static_assert(kBaHTable == kBlock && kBaHHinges <= 2 * kBlock && 2 * kBaHNodes <= kBlock, "threads");
+  __shared__ T sx[3][kBaHTable];
+  __shared__ int sn[G ? kBaHNodes : 1];
+  __shared__ T st[G ? 12 * kBaHCol : 1];
+  const int tid = threadIdx.x, own = tid >> 1, half = tid & 1;
+  if (G && tid < 12) st[tid * kBaHCol + kBaHHinges] = (T)0;
   double acc[1] = {0.0};
-  const size_t stride = (size_t)gridDim.x * kBlock;
-  // contiguous ranges of blocks per XCD: neighbouring elements share nodes in one L2
-  const size_t tid = (size_t)xcd_logical_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-  for (size_t w0 = tid; w0 < (size_t)a.nbar; w0 += U * stride) {
-    T p1[U][3], p2[U][3], k[U], l0[U];
+  const int b = xcd_logical_block(blockIdx.x, gridDim.x);
+  const int k0 = (int)((long long)a.ncluster * b / gridDim.x);
+  const int k1 = (int)((long long)a.ncluster * (b + 1) / gridDim.x);
+  const int c0 = k0 < a.ncluster ? a.cluster[k0] : a.nchunk;
+  const int c1 = k1 < a.ncluster ? a.cluster[k1] : a.nchunk;
+
+  // entry 2 q + half of this thread's node
+  auto codes = [&](const ushort4* from, uint32_t at, int nCode, int nOwn, int q, unsigned short pad) {
+    ushort4 w = make_ushort4(pad, pad, pad, pad);
+    if (own < nOwn && 2 * q + half < nCode) w = from[at + (size_t)(2 * q + half) * nOwn + own];
+    return w;
+  };
+  auto node_of = [&](const BaHChunk& c) { return tid < c.nNode ? nodes[c.node0 + tid] : 0; };
+  auto read = [&](const BaHChunk& c, int node, ChunkIn<T, TV>& in) {
+    in.node = node;
+    if (tid < c.nNode) {
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const size_t w = w0 + u * stride;
-      const int b = (int)(w < (size_t)a.nbar ? w : (size_t)a.nbar - 1);
-      const int2 nd = reinterpret_cast<const int2*>(a.bar)[b];
-      ld3(x, d, t, nd.x, p1[u]);
-      ld3(x, d, t, nd.y, p2[u]);
-      k[u] = (T)(a.bk ? a.bk[b] : a.bkU);
-      l0[u] = (T)(a.bl0 ? a.bl0[b] : a.bl0U);
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      if (w0 + u * stride >= (size_t)a.nbar) break;
-      T dx[3] = {p1[u][0] - p2[u][0], p1[u][1] - p2[u][1], p1[u][2] - p2[u][2]};
-      const T l = sqrt(dot3(dx, dx));
-      const T dl = l - l0[u];
-      acc[0] += (double)((T)0.5 * k[u] * (dl * dl));
-    }
-  }
-  for (size_t w0 = tid; w0 < (size_t)a.nhinge; w0 += U * stride) {
-    HingeIn<T> H[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const size_t w = w0 + u * stride;
-      hinge_load(x, d, t, a, (int)(w < (size_t)a.nhinge ? w : (size_t)a.nhinge - 1), H[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      if (w0 + u * stride >= (size_t)a.nhinge) break;
-      HingeGeo<T> G;
-      hinge_geo_at(H[u].x1, H[u].x2, H[u].x3, H[u].x4, H[u].t0, G);
-      acc[0] += (double)((T)0.5 * H[u].k * (G.dtheta * G.dtheta));
-      if (SD) hinge_store(G, H[u].k, ht, w0 + u * stride);
-    }
-  }
-  if (a.fz) {
-    for (size_t n = tid; n < (size_t)a.nnode; n += stride) {
-      if (a.nodeActive[n]) {
-        T p[3];
-        ld3(x, d, t, (int)n, p);
-        acc[0] -= a.fz[n] * (double)p[2];
+      for (int q = 0; q < 3; q++) {
+        in.x[q] = x[(size_t)node * 3 + q];
+        if (d) in.d[q] = d[(size_t)node * 3 + q];
       }
     }
-  }
-  grid_sum_store<1>(acc, rs);
-}
+    const int nHinge = G ? c.nHinge : c.nHingeOwn;
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+      if (tid + u * kBlock < nHinge) in.hinge[u] = a.hinge[c.hinge0 + tid + u * kBlock];
+    in.bcode = codes(a.bcode, c.bcode0, c.nBarCode, c.nOwn, 0, kBaHNoBar);
+    if (G) {
+#pragma unroll
+      for (int q = 0; q < 2; q++) in.hcode[q] = codes(a.hcode, c.hcode0, c.nHingeCode, c.nOwn, q, kBaHNoHinge);
+    }
+  };
 
-// What the gradient gather needs of every hinge (gradient without energy).
-template <typename T>
-__global__ __launch_bounds__(kBlock) void bah_hinge_kernel(BaHArgs a, const T* __restrict__ x,
-                                                           HStore<T>* __restrict__ ht) {
-  for (size_t h = (size_t)blockIdx.x * kBlock + threadIdx.x; h < (size_t)a.nhinge; h += (size_t)gridDim.x * kBlock) {
-    HingeIn<T> H;
-    hinge_load<T>(x, nullptr, (T)0, a, (int)h, H);
-    HingeGeo<T> G;
-    hinge_geo_at(H.x1, H.x2, H.x3, H.x4, H.t0, G);
-    hinge_store(G, H.k, ht, h);
-  }
-}
-
-// Gradient, gathered per node over its incident bars and hinges (CSR in
-// element order), U elements at a time with all their loads issued first;
-// contributions are added in list order.  Hinge terms (FP32) or angle
-// deviations (FP64) come from ht, stored by the energy or the hinge kernel.
-// TG: the gradient's storage (FP32 for FP64 arithmetic in the mixed schedule).
-template <typename T, typename TG = T>
-__global__ __launch_bounds__(kBlock) void bah_gradient_kernel(BaHArgs a, const T* __restrict__ x,
-                                                              const HStore<T>* __restrict__ ht,
-                                                              TG* __restrict__ g) {
-  constexpr int U = 4;
-  for (int n = xcd_logical_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; n < a.nnode;
-       n += gridDim.x * kBlock) {
+  if (c0 < c1) {
+    BaHChunk c = chunks[c0], next = chunks[min(c0 + 1, c1 - 1)];
+    ChunkIn<T, TV> in;
+    read(c, node_of(c), in);
+    int nextNode = node_of(next);
     T gn[3] = {(T)0, (T)0, (T)0};
-    const int qb0 = a.bptr[n], qb1 = a.bptr[n + 1];
-    for (int q0 = qb0; q0 < qb1; q0 += U) {
-      T p1[U][3], p2[U][3], k[U], l0[U];
-      int loc[U];
+    for (int ci = c0; ci < c1; ci++) {
+      if (tid < c.nNode) {
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int code = a.bidx[min(q0 + u, qb1 - 1)];
-        const int b = code >> 1;
-        loc[u] = code & 1;
-        const int2 nd = reinterpret_cast<const int2*>(a.bar)[b];
-        ld3<T>(x, nullptr, (T)0, nd.x, p1[u]);
-        ld3<T>(x, nullptr, (T)0, nd.y, p2[u]);
-        k[u] = (T)(a.bk ? a.bk[b] : a.bkU);
-        l0[u] = (T)(a.bl0 ? a.bl0[b] : a.bl0U);
+        for (int q = 0; q < 3; q++) {
+          T p = in.x[q];
+          if (d) {
+            const T s = t * (T)in.d[q];
+            p = p + s;
+          }
+          sx[q][tid] = p;
+          if (xout && tid < c.nOwn) xout[(size_t)in.node * 3 + q] = p;
+        }
+        if (G && tid < c.nOwn) sn[tid] = in.node;
       }
+      const ChunkIn<T, TV> now = in;
+      const BaHChunk after = chunks[min(ci + 2, c1 - 1)];
+      lds_barrier();
+      read(next, nextNode, in);
+      nextNode = node_of(after);
+
+      const bool mine = own < c.nOwn;
+      const int me = mine ? own : 0;
+      T p[3];
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        if (q0 + u >= qb1) break;
-        T dx[3] = {p1[u][0] - p2[u][0], p1[u][1] - p2[u][1], p1[u][2] - p2[u][2]};
-        const T l = sqrt(dot3(dx, dx));
-        const T dl = l - l0[u];
-        // stretching gradient 2 k (l - l0) / l * dx (BarAndHinge.cpp:282)
-        const T gf = (T)2 * k[u] * dl / l;
-        const T sg = loc[u] == 0 ? (T)1 : (T)-1;
+      for (int q = 0; q < 3; q++) p[q] = sx[q][me];
+      const int gnode = G ? sn[me] : 0;
+      if (G || (parts & kBars)) {
+        auto bars = [&](const ushort4& w, int q) {
+          const int cs[4] = {w.x, w.y, w.z, w.w};
+          T f[4][3];
 #pragma unroll
-        for (int c = 0; c < 3; c++) gn[c] += sg * (gf * dx[c]);
+          for (int v = 0; v < 4; v++) {
+            f[v][0] = f[v][1] = f[v][2] = (T)0;
+            if (cs[v] == kBaHNoBar || (!G && (cs[v] & 1))) continue;
+            const size_t at = 4 * (c.bcode0 + (size_t)(2 * q + half) * c.nOwn + own) + v;
+            const T kb = (T)(a.bk ? a.bk[at] : a.bkU), l0 = (T)(a.bl0 ? a.bl0[at] : a.bl0U);
+            T dx[3];
+#pragma unroll
+            for (int m = 0; m < 3; m++) dx[m] = p[m] - sx[m][cs[v] >> 1];
+            const T l = root(dot3(dx, dx));
+            const T dl = l - l0;
+            if (E && (cs[v] & 1) == 0) acc[0] += (double)((T)0.5 * kb * (dl * dl));
+            // stretching gradient 2 k (l - l0) / l * dx (BarAndHinge.cpp:282)
+            const T gf = quotient((T)2 * kb * dl, l);
+#pragma unroll
+            for (int m = 0; m < 3; m++) f[v][m] = gf * dx[m];
+          }
+          if constexpr (G) add_pair(gn, f);
+        };
+        bars(now.bcode, 0);
+        for (int q = 1; 2 * q < c.nBarCode; q++)
+          bars(codes(a.bcode, c.bcode0, c.nBarCode, c.nOwn, q, kBaHNoBar), q);
       }
+      if (G || (parts & kHinges)) {
+        const int nHinge = G ? c.nHinge : c.nHingeOwn;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const int i = tid + u * kBlock;
+          if (i >= nHinge) break;
+          const T kh = (T)(a.hk ? a.hk[c.hinge0 + i] : a.hkU), t0 = (T)(a.ht0 ? a.ht0[c.hinge0 + i] : a.ht0U);
+          T x1[3], x2[3], x3[3], x4[3];
+#pragma unroll
+          for (int q = 0; q < 3; q++) {
+            x1[q] = sx[q][now.hinge[u].x];
+            x2[q] = sx[q][now.hinge[u].y];
+            x3[q] = sx[q][now.hinge[u].z];
+            x4[q] = sx[q][now.hinge[u].w];
+          }
+          HingeGeo<T> geo;
+          hinge_geo_vec(x1, x2, x3, x4, geo);
+          hinge_dtheta(geo, t0);
+          if (E && i < c.nHingeOwn) acc[0] += (double)((T)0.5 * kh * (geo.dtheta * geo.dtheta));
+          if constexpr (G) {
+            T f[4][3];
+            hinge_gradient(geo, kh, f);
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+#pragma unroll
+              for (int q = 0; q < 3; q++) st[bah_slot(i, v) + q * kBaHCol] = f[v][q];
+          }
+        }
+      }
+      if (a.fz && !c.more && mine && half == 0 && (a.flags[c.own0 + own] & kForced)) {
+        const double f = a.fz[c.own0 + own];
+        if (E && (parts & kForces)) acc[0] -= f * (double)p[2];
+        gn[2] -= (T)f;
+      }
+      lds_barrier();
+      if constexpr (G) {
+        auto add = [&](const ushort4& w) {
+          const int cs[4] = {w.x, w.y, w.z, w.w};
+          T f[4][3];
+#pragma unroll
+          for (int v = 0; v < 4; v++)
+#pragma unroll
+            for (int m = 0; m < 3; m++) f[v][m] = st[cs[v] + m * kBaHCol];
+          add_pair(gn, f);
+        };
+        add(now.hcode[0]);
+        if (c.nHingeCode > 2) add(now.hcode[1]);
+        for (int q = 2; 2 * q < c.nHingeCode; q++)
+          add(codes(a.hcode, c.hcode0, c.nHingeCode, c.nOwn, q, kBaHNoHinge));
+        if (!c.more) {
+          const int fl = mask && mine ? a.flags[c.own0 + own] : 0;
+#pragma unroll
+          for (int q = 0; q < 3; q++) {
+            if (mine && half == 0) g[(size_t)gnode * 3 + q] = fl >> q & 1 ? (TV)0 : (TV)gn[q];
+            gn[q] = (T)0;
+          }
+        }
+      }
+      c = next;
+      next = after;
     }
-    const int qh0 = a.hptr[n], qh1 = a.hptr[n + 1];
-    for (int q0 = qh0; q0 < qh1; q0 += U) {
-      int loc[U];
-      if constexpr (kHingeTerms<T>) {
-        HingeTerms<T> H[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const int code = a.hidx[min(q0 + u, qh1 - 1)];
-          loc[u] = code & 3;
-          H[u] = ht[code >> 2];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          if (q0 + u >= qh1) break;
-          hinge_grad_at(H[u], loc[u], gn);
-        }
-      } else {
-        HingeIn<T> H[U];
-        T dt[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const int code = a.hidx[min(q0 + u, qh1 - 1)];
-          loc[u] = code & 3;
-          hinge_load<T>(x, nullptr, (T)0, a, code >> 2, H[u]);
-          dt[u] = ht[code >> 2];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          if (q0 + u >= qh1) break;
-          HingeGeo<T> G;
-          hinge_geo_vec(H[u].x1, H[u].x2, H[u].x3, H[u].x4, G);
-          G.dtheta = dt[u];
-          HingeTerms<T> tm;
-          hinge_terms(G, H[u].k, tm);
-          hinge_grad_at(tm, loc[u], gn);
-        }
-      }
-    }
-    if (a.fz && a.nodeActive[n]) gn[2] -= (T)a.fz[n];
-#pragma unroll
-    for (int k = 0; k < 3; k++) g[(size_t)n * 3 + k] = (TG)gn[k];
+  }
+  if constexpr (E) {
+    __syncthreads();
+    grid_sum_store<1>(acc, rs);
   }
 }
 
@@ -393,15 +415,7 @@ using minim_amd::kBlock;
 struct BarAndHinge::Dev {
   minim_amd::BaHArgs args{};
   DeviceBuffer mem;
-  DeviceBuffer ht;      // per-hinge store of the last gradient evaluation (HStore, either precision)
-  DeviceBuffer xtrial;  // node coordinates at a line-search trial point (FP64-sized)
-  std::vector<int> activeBars, activeHinges;  // element index -> original bond/hinge index
-  // The coordinates (and their precision) for which a fused step's energy
-  // pass kept the hinge store with no gradient yet; any other evaluation
-  // clears it, and the next gradient-only evaluation at exactly those
-  // coordinates skips the hinge pass.
-  mutable const void* keptAt = nullptr;
-  mutable int keptPrec = -1;
+  size_t nFixed = 0;  // single-DOF constraints that the node flags hold
 };
 
 BarAndHinge& BarAndHinge::setTriangulation(const vector2d<int>& triList) {
@@ -449,47 +463,75 @@ BarAndHinge& BarAndHinge::setForce(const vector<double>& f) {
 
 namespace {
 
+// The edges of all triangles, sorted by (lower node, upper node, triangle):
+// edge k of triangle t joins its nodes k and k + 1.
+struct Edges {
+  struct Edge {
+    int lo, hi, id;  // id: 3 t + k
+  };
+  std::vector<Edge> e;
+  std::vector<int> first;  // per id: the first of the edges that join the same nodes
+  explicit Edges(const vector2d<int>& tris) : e(3 * tris.size()), first(3 * tris.size()) {
+    int least = 0, most = -1;
+    for (size_t t = 0; t < tris.size(); t++) {
+      if (tris[t].size() != 3) throw std::invalid_argument("BarAndHinge: triangles need three nodes.");
+      for (int k = 0; k < 3; k++) {
+        const int a = tris[t][k], b = tris[t][(k + 1) % 3];
+        e[3 * t + k] = {std::min(a, b), std::max(a, b), (int)(3 * t + k)};
+        least = std::min(least, e[3 * t + k].lo);
+        most = std::max(most, e[3 * t + k].hi);
+      }
+    }
+    auto before = [](const Edge& u, const Edge& v) {
+      return u.lo != v.lo ? u.lo < v.lo : u.hi != v.hi ? u.hi < v.hi : u.id < v.id;
+    };
+    if (least >= 0 && (size_t)most < 4 * e.size()) {
+      // by lower node first (a count per node), then each node's few edges
+      std::vector<size_t> at(most + 2, 0);
+      for (const auto& x : e) at[x.lo + 1]++;
+      for (int n = 0; n <= most; n++) at[n + 1] += at[n];
+      std::vector<Edge> s(e.size());
+      auto next = at;
+      for (const auto& x : e) s[next[x.lo]++] = x;
+      e.swap(s);
+      for (int n = 0; n <= most; n++) std::sort(e.begin() + at[n], e.begin() + at[n + 1], before);
+    } else {
+      std::sort(e.begin(), e.end(), before);
+    }
+    for (size_t i = 0; i < e.size(); i++)
+      first[e[i].id] = i > 0 && same(i - 1, i) ? first[e[i - 1].id] : (int)i;
+  }
+  bool same(size_t i, size_t j) const { return e[i].lo == e[j].lo && e[i].hi == e[j].hi; }
+};
+
 // Bond list of BarAndHinge::computeBondList (BarAndHinge.cpp:70-93): sorted
 // node pairs of every triangle, lexicographically sorted and unique.
 vector2d<int> bonds_from_tris(const vector2d<int>& tris) {
-  std::vector<std::pair<int, int>> e;
-  e.reserve(tris.size() * 3);
-  for (const auto& t0 : tris) {
-    if (t0.size() != 3) throw std::invalid_argument("BarAndHinge: triangles need three nodes.");
-    int t[3] = {t0[0], t0[1], t0[2]};
-    std::sort(t, t + 3);
-    e.push_back({t[0], t[1]});
-    e.push_back({t[0], t[2]});
-    e.push_back({t[1], t[2]});
-  }
-  std::sort(e.begin(), e.end());
-  e.erase(std::unique(e.begin(), e.end()), e.end());
+  const Edges g(tris);
   vector2d<int> out;
-  out.reserve(e.size());
-  for (auto& p : e) out.push_back({p.first, p.second});
+  out.reserve(g.e.size() / 2 + 1);
+  for (size_t i = 0; i < g.e.size(); i++)
+    if (i == 0 || !g.same(i - 1, i)) out.push_back({g.e[i].lo, g.e[i].hi});
   return out;
 }
 
 // Hinge list of BarAndHinge::computeHingeList (BarAndHinge.cpp:96-147) in
-// the same order, built in O(T) from an edge -> triangles map instead of the
+// the same order, built from the triangles of each edge instead of the
 // reference's all-pairs triangle loop: for each triangle it1 and each later
 // triangle it2 sharing exactly two nodes, nodes = [unshared of it1, the next
 // two of it1 in cyclic order, unshared of it2].
 vector2d<int> hinges_from_tris(const vector2d<int>& tris) {
-  std::unordered_map<long long, std::vector<int>> edge;
-  edge.reserve(tris.size() * 3);
-  auto key = [](int a, int b) {
-    if (a > b) std::swap(a, b);
-    return ((long long)a << 32) | (unsigned)b;
-  };
-  for (int it = 0; it < (int)tris.size(); it++)
-    for (int k = 0; k < 3; k++) edge[key(tris[it][k], tris[it][(k + 1) % 3])].push_back(it);
+  const Edges g(tris);
   vector2d<int> out;
+  out.reserve(g.e.size() / 2 + 1);
+  std::vector<int> cand;
   for (int it1 = 0; it1 < (int)tris.size(); it1++) {
-    std::vector<int> cand;
-    for (int k = 0; k < 3; k++)
-      for (int it2 : edge[key(tris[it1][k], tris[it1][(k + 1) % 3])])
-        if (it2 > it1) cand.push_back(it2);
+    cand.clear();
+    for (int k = 0; k < 3; k++) {
+      const size_t i0 = g.first[3 * (size_t)it1 + k];
+      for (size_t i = i0; i < g.e.size() && g.same(i0, i); i++)
+        if (g.e[i].id / 3 > it1) cand.push_back(g.e[i].id / 3);
+    }
     std::sort(cand.begin(), cand.end());
     cand.erase(std::unique(cand.begin(), cand.end()), cand.end());
     for (int it2 : cand) {
@@ -512,7 +554,7 @@ vector2d<int> hinges_from_tris(const vector2d<int>& tris) {
         }
       for (int b = 0; b < 3; b++)
         if (!s2[b]) nodes[3] = tris[it2][b];
-      out.push_back(nodes);
+      out.push_back(std::move(nodes));
     }
   }
   return out;
@@ -590,6 +632,7 @@ void BarAndHinge::init(const vector<double>& coords) {
     throw std::invalid_argument("BarAndHinge: force must have 3 or 3*nNode entries.");
   uploadFixed(coords.size());
   nNodeHint = nnode;
+  order_ = std::make_shared<const vector<int>>(minim_amd::bah_mesh::order(coords, minim_amd::bah_mesh::parts(nnode)));
   upload();
 }
 
@@ -612,184 +655,138 @@ void BarAndHinge::upload() {
   auto dev = std::make_shared<Dev>();
   std::vector<int> bar, hin;
   std::vector<double> bk, bl, hk, ht;
+  bar.reserve(2 * bonds_.size());
+  hin.reserve(4 * hinges_.size());
   for (size_t i = 0; i < bonds_.size(); i++) {
     int nd[2] = {bonds_[i][0], bonds_[i][1]};
     if (allFixed(nd, 2)) continue;
-    bar.push_back(nd[0]);
-    bar.push_back(nd[1]);
+    bar.insert(bar.end(), nd, nd + 2);
     bk.push_back(kBond_[i]);
     bl.push_back(length0_[i]);
-    dev->activeBars.push_back((int)i);
   }
   for (size_t i = 0; i < hinges_.size(); i++) {
     int nd[4] = {hinges_[i][0], hinges_[i][1], hinges_[i][2], hinges_[i][3]};
     if (allFixed(nd, 4)) continue;
-    for (int k = 0; k < 4; k++) hin.push_back(nd[k]);
+    hin.insert(hin.end(), nd, nd + 4);
     hk.push_back(kHinge_[i]);
     ht.push_back(theta0_[i]);
-    dev->activeHinges.push_back((int)i);
   }
-  const int nb = (int)bk.size(), nh = (int)hk.size();
-  // node -> incident element CSR, in element order
-  std::vector<int> bptr(nnode + 1, 0), hptr(nnode + 1, 0);
-  for (int b = 0; b < nb; b++)
-    for (int l = 0; l < 2; l++) bptr[bar[2 * b + l] + 1]++;
-  for (int h = 0; h < nh; h++)
-    for (int l = 0; l < 4; l++) hptr[hin[4 * h + l] + 1]++;
-  for (int n = 0; n < nnode; n++) {
-    bptr[n + 1] += bptr[n];
-    hptr[n + 1] += hptr[n];
-  }
-  std::vector<int> bidx(bptr[nnode]), hidx(hptr[nnode]);
-  {
-    std::vector<int> cb(bptr.begin(), bptr.end() - 1), ch(hptr.begin(), hptr.end() - 1);
-    for (int b = 0; b < nb; b++)
-      for (int l = 0; l < 2; l++) bidx[cb[bar[2 * b + l]]++] = (b << 1) | l;
-    for (int h = 0; h < nh; h++)
-      for (int l = 0; l < 4; l++) hidx[ch[hin[4 * h + l]]++] = (h << 2) | l;
-  }
+  minim_amd::BaHLists lists;
+  lists.nnode = nnode;
+  lists.bar = &bar;
+  lists.hinge = &hin;
+  const auto mesh = minim_amd::bah_mesh::build(lists, *order_, minim_amd::bah_mesh::parts(nnode));
   std::vector<double> fz;
-  std::vector<unsigned char> active(nnode, 0);
-  if (!force_.empty()) {
-    fz.resize(nnode);
-    for (int n = 0; n < nnode; n++) {
-      fz[n] = force_.size() == 3 ? force_[2] : force_[3 * (size_t)n + 2];
-      int nd[1] = {n};
-      active[n] = allFixed(nd, 1) ? 0 : 1;
-    }
+  std::vector<unsigned char> flags(nnode, 0);
+  if (!force_.empty()) fz.resize(nnode);
+  for (int o = 0; o < nnode; o++) {
+    const int n = (*order_)[o];
+    for (int k = 0; k < 3; k++) flags[o] |= fixed[3 * (size_t)n + k] << k;
+    if (force_.empty()) continue;
+    fz[o] = force_.size() == 3 ? force_[2] : force_[3 * (size_t)n + 2];
+    if (!allFixed(&n, 1)) flags[o] |= minim_amd::kForced;
   }
-  // one allocation, 256-byte aligned sub-buffers
-  size_t off = 0;
-  auto reserve = [&](size_t bytes) {
-    size_t o = off;
-    off += (bytes + 255) / 256 * 256;
-    return o;
-  };
-  const size_t o_bar = reserve(sizeof(int) * bar.size()), o_bk = reserve(sizeof(double) * bk.size()),
-               o_bl = reserve(sizeof(double) * bl.size()), o_hin = reserve(sizeof(int) * hin.size()),
-               o_hk = reserve(sizeof(double) * hk.size()), o_ht = reserve(sizeof(double) * ht.size()),
-               o_bptr = reserve(sizeof(int) * bptr.size()), o_bidx = reserve(sizeof(int) * bidx.size()),
-               o_hptr = reserve(sizeof(int) * hptr.size()), o_hidx = reserve(sizeof(int) * hidx.size()),
-               o_fz = reserve(sizeof(double) * fz.size()), o_act = reserve(active.size());
-  dev->mem.reset(off + 256);
-  char* base = static_cast<char*>(dev->mem.get());
-  auto put = [&](size_t o, const void* src, size_t bytes) {
-    if (bytes) MINIM_HIP_CHECK(hipMemcpy(base + o, src, bytes, hipMemcpyHostToDevice));
-  };
-  put(o_bar, bar.data(), sizeof(int) * bar.size());
-  put(o_bk, bk.data(), sizeof(double) * bk.size());
-  put(o_bl, bl.data(), sizeof(double) * bl.size());
-  put(o_hin, hin.data(), sizeof(int) * hin.size());
-  put(o_hk, hk.data(), sizeof(double) * hk.size());
-  put(o_ht, ht.data(), sizeof(double) * ht.size());
-  put(o_bptr, bptr.data(), sizeof(int) * bptr.size());
-  put(o_bidx, bidx.data(), sizeof(int) * bidx.size());
-  put(o_hptr, hptr.data(), sizeof(int) * hptr.size());
-  put(o_hidx, hidx.data(), sizeof(int) * hidx.size());
-  put(o_fz, fz.data(), sizeof(double) * fz.size());
-  put(o_act, active.data(), active.size());
-  auto& a = dev->args;
-  a.nnode = nnode;
-  a.nbar = nb;
-  a.nhinge = nh;
-  a.bar = (const int*)(base + o_bar);
-  // parameters shared by every element go as scalars
+  dev->nFixed = constraints.size();
+  // parameters shared by every element go as scalars, others per bar code and hinge record
   auto uniform = [](const std::vector<double>& v) {
     for (double x : v)
       if (!(x == v[0]) || std::signbit(x) != std::signbit(v[0])) return false;
     return true;
   };
-  a.bk = uniform(bk) ? nullptr : (const double*)(base + o_bk);
-  a.bl0 = uniform(bl) ? nullptr : (const double*)(base + o_bl);
-  a.hinge = (const int*)(base + o_hin);
-  a.hk = uniform(hk) ? nullptr : (const double*)(base + o_hk);
-  a.ht0 = uniform(ht) ? nullptr : (const double*)(base + o_ht);
+  auto records = [&](const std::vector<double>& v, const std::vector<int>& id) {
+    std::vector<double> r;
+    if (uniform(v)) return r;
+    r.reserve(id.size());
+    for (int i : id) r.push_back(v[i]);
+    return r;
+  };
+  const auto bkR = records(bk, mesh.barId), blR = records(bl, mesh.barId), hkR = records(hk, mesh.hingeId),
+             htR = records(ht, mesh.hingeId);
+  // one allocation, 256-byte aligned sub-buffers
+  std::vector<std::pair<const void*, size_t>> src;
+  std::vector<size_t> at;
+  size_t off = 0;
+  auto reserve = [&](const auto& v) {
+    src.push_back({v.data(), v.size() * sizeof(v[0])});
+    at.push_back(off);
+    off += (src.back().second + 255) / 256 * 256;
+    return at.size() - 1;
+  };
+  const size_t i_chunk = reserve(mesh.chunk), i_cluster = reserve(mesh.cluster), i_node = reserve(mesh.node),
+               i_hinge = reserve(mesh.hinge), i_bcode = reserve(mesh.bcode),
+               i_hcode = reserve(mesh.hcode), i_bk = reserve(bkR), i_bl = reserve(blR), i_hk = reserve(hkR),
+               i_ht = reserve(htR), i_fz = reserve(fz), i_flags = reserve(flags);
+  dev->mem.reset(off + 256);
+  char* base = static_cast<char*>(dev->mem.get());
+  for (size_t i = 0; i < src.size(); i++)
+    if (src[i].second) MINIM_HIP_CHECK(hipMemcpy(base + at[i], src[i].first, src[i].second, hipMemcpyHostToDevice));
+  auto dptr = [&](size_t i) { return (const double*)(src[i].second ? base + at[i] : nullptr); };
+  auto& a = dev->args;
+  a.nnode = nnode;
+  a.ncluster = (int)mesh.cluster.size();
+  a.nchunk = (int)mesh.chunk.size();
+  a.chunk = (const minim_amd::BaHChunk*)(base + at[i_chunk]);
+  a.cluster = (const int*)(base + at[i_cluster]);
+  a.node = (const int*)(base + at[i_node]);
+  a.bk = dptr(i_bk);
+  a.bl0 = dptr(i_bl);
+  a.hinge = (const ushort4*)(base + at[i_hinge]);
+  a.hk = dptr(i_hk);
+  a.ht0 = dptr(i_ht);
   a.bkU = bk.empty() ? 0.0 : bk[0];
   a.bl0U = bl.empty() ? 0.0 : bl[0];
   a.hkU = hk.empty() ? 0.0 : hk[0];
   a.ht0U = ht.empty() ? 0.0 : ht[0];
-  a.bptr = (const int*)(base + o_bptr);
-  a.bidx = (const int*)(base + o_bidx);
-  a.hptr = (const int*)(base + o_hptr);
-  a.hidx = (const int*)(base + o_hidx);
-  a.fz = fz.empty() ? nullptr : (const double*)(base + o_fz);
-  a.nodeActive = (const unsigned char*)(base + o_act);
-  dev->ht.reset(std::max(sizeof(minim_amd::HStore<double>), sizeof(minim_amd::HStore<float>)) *
-                (size_t)(nh > 0 ? nh : 1));
-  dev->xtrial.reset(3 * sizeof(double) * (size_t)(nnode > 0 ? nnode : 1));
+  a.bcode = (const ushort4*)(base + at[i_bcode]);
+  a.hcode = (const ushort4*)(base + at[i_hcode]);
+  a.fz = dptr(i_fz);
+  a.flags = (const unsigned char*)(base + at[i_flags]);
   dev_ = dev;
 }
 
 namespace {
-// Energy kernel (into rs.result[0] when wantE, and to eDev when given) and
-// gradient kernel (when g; the hinge terms come from the energy kernel, or
-// from the hinge kernel without an energy).  prec: the coordinates and the
-// arithmetic; pv: the direction d and the gradient g (FP32 against FP64
-// coordinates in the mixed schedule).
-void launch_bah(const BarAndHinge::Dev& dv, int prec, int pv, const void* x, const void* d, double t, bool wantE,
-                void* g, minim_amd::RedScratch rs, hipStream_t s, double* eDev = nullptr, bool keep = false) {
+// One evaluation: energy (into rs.result[0], and to eDev when given) when
+// wantE, gradient when g; at x + t*d when d, which also goes to xout when
+// given.  prec: the coordinates and the arithmetic; pv: d and g (FP32 against
+// FP64 coordinates in the mixed schedule).  mask: the gradient of single-DOF
+// constraints comes out zero.
+void launch_bah(const BarAndHinge::Dev& dv, int prec, int pv, const void* x, const void* d, double t, void* xout,
+                bool wantE, void* g, bool mask, minim_amd::RedScratch rs, hipStream_t s, double* eDev = nullptr,
+                int parts = minim_amd::kAllParts) {
   const auto& a = dv.args;
   if (pv != prec && !(prec == FP64 && pv == FP32))
     throw std::invalid_argument("BarAndHinge: FP32 coordinates with FP64 vectors are not supported.");
-  const bool reuse = !d && !wantE && g && dv.keptAt == x && dv.keptPrec == prec;
-  dv.keptAt = nullptr;
-  auto go = [&](auto tag, auto gtag) {
+  // the same blocks with and without the gradient: the energy is the same bit for bit
+  const int most = prec == FP64 ? minim_amd::kBaHBlocks<double> : minim_amd::kBaHBlocks<float>;
+  const int nb = std::max(1, std::min(a.ncluster, most));
+  auto go = [&](auto tag, auto vtag) {
     using T = decltype(tag);
-    using TG = decltype(gtag);
-    auto* ht = static_cast<minim_amd::HStore<T>*>(dv.ht.get());
-    const T* xx = (const T*)x;
-    if (d) {
-      // a trial point: materialised once (x + t*d, as the element loads would
-      // form it), so that the energy pass reads one array per node
-      T* xt = static_cast<T*>(dv.xtrial.get());
-      const size_t n3 = 3 * (size_t)a.nnode;
-      minim_amd::device_copy(xt, x, n3 * sizeof(T), s);
-      minim_amd::launch_axpy_mixed(prec, xt, pv, d, t, n3, s);
-      xx = xt;
-    }
-    if (wantE) {
-      const size_t tot = (size_t)a.nbar + a.nhinge + a.nnode;
-      const int nb = minim_amd::grid_blocks(tot, 4, 2048);
-      if (g || keep)
-        minim_amd::bah_energy_kernel<T, true><<<nb, kBlock, 0, s>>>(a, xx, (const T*)nullptr, (T)0, rs, ht);
-      else
-        minim_amd::bah_energy_kernel<T, false><<<nb, kBlock, 0, s>>>(a, xx, (const T*)nullptr, (T)0, rs, ht);
+    using TV = decltype(vtag);
+    auto run = [&](auto kernel) {
+      kernel<<<nb, kBlock, 0, s>>>(a, a.chunk, a.node, (const T*)x, (const TV*)d, (T)t, (T*)xout, (TV*)g, mask, parts, rs);
       MINIM_HIP_CHECK(hipGetLastError());
-      minim_amd::launch_finalize(rs, 1, nb, s, 0, eDev);
-    } else if (g && a.nhinge > 0 && !reuse) {
-      minim_amd::bah_hinge_kernel<T><<<minim_amd::grid_blocks(a.nhinge, 1, 1 << 20), kBlock, 0, s>>>(a, xx, ht);
-      MINIM_HIP_CHECK(hipGetLastError());
-    }
-    if (g) {
-      const int nb = minim_amd::grid_blocks(a.nnode, 1, 1 << 20);
-      minim_amd::bah_gradient_kernel<T, TG><<<nb, kBlock, 0, s>>>(a, xx, ht, (TG*)g);
-      MINIM_HIP_CHECK(hipGetLastError());
-    }
+    };
+    if (wantE && g) run(minim_amd::bah_kernel<T, TV, true, true>);
+    else if (wantE) run(minim_amd::bah_kernel<T, TV, true, false>);
+    else if (g) run(minim_amd::bah_kernel<T, TV, false, true>);
   };
   if (prec == FP64 && pv == FP64) go(0.0, 0.0);
   else if (prec == FP64) go(0.0, 0.0f);
   else go(0.0f, 0.0f);
-  if (keep && wantE && !d) {
-    dv.keptAt = x;
-    dv.keptPrec = prec;
-  }
+  if (wantE) minim_amd::launch_finalize(rs, 1, nb, s, 0, eDev);
 }
 }  // namespace
 
+// The node flags hold every constraint (none was added since the upload, and
+// none reads the coordinates): the kernel zeroes the fixed components itself.
+bool BarAndHinge::maskHolds() const { return constraints.size() == dev_->nFixed && !hasNormalConstraints(); }
+
 void BarAndHinge::evaluate(int prec, const void* x, const void* d, double t, double* e, void* g,
                            void* stream) const {
-  if (!dev_) throw std::runtime_error("BarAndHinge: not initialised (construct a State first).");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  auto& ws = minim_amd::Workspace::current();
-  const auto& a = dev_->args;
-  if (g && d) throw std::invalid_argument("BarAndHinge: gradients at a trial point are not supported.");
-  if (e || g) {
-    launch_bah(*dev_, prec, prec, x, d, t, e != nullptr, g, ws.rs(), s);
-    if (g) constrainDevice(prec, x, g, 3 * (size_t)a.nnode, stream);
-  }
+  evaluateAsync(prec, x, d, t, e != nullptr, nullptr, g, stream);
   if (e) {
     double r[1];
-    ws.fetch(s, 1, r);
+    minim_amd::Workspace::current().fetch(static_cast<hipStream_t>(stream), 1, r);
     *e = r[0];
   }
 }
@@ -801,9 +798,10 @@ void BarAndHinge::evaluateAsync(int prec, const void* x, const void* d, double t
   if (!dev_) throw std::runtime_error("BarAndHinge: not initialised (construct a State first).");
   if (g && d) throw std::invalid_argument("BarAndHinge: gradients at a trial point are not supported.");
   if (!wantE && !g) return;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  launch_bah(*dev_, prec, prec, x, d, t, wantE, g, minim_amd::Workspace::current().rs(), s, wantE ? e_dev : nullptr);
-  if (g) constrainDevice(prec, x, g, 3 * (size_t)dev_->args.nnode, stream);
+  const bool mask = maskHolds();
+  launch_bah(*dev_, prec, prec, x, d, t, nullptr, wantE, g, mask, minim_amd::Workspace::current().rs(),
+             static_cast<hipStream_t>(stream), wantE ? e_dev : nullptr);
+  if (g && !mask) constrainDevice(prec, x, g, 3 * (size_t)dev_->args.nnode, stream);
 }
 
 // The mixed schedule's second phase: FP64 coordinates and arithmetic, the
@@ -817,16 +815,15 @@ void BarAndHinge::evaluateMixedAsync(const void* x, const void* d, double t, boo
   if (g && d) throw std::invalid_argument("BarAndHinge: gradients at a trial point are not supported.");
   if (!supportsMixed()) throw std::invalid_argument("BarAndHinge: no mixed evaluation with normal constraints.");
   if (!wantE && !g) return;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  launch_bah(*dev_, FP64, FP32, x, d, t, wantE, g, minim_amd::Workspace::current().rs(), s, wantE ? e_dev : nullptr);
-  if (g) constrainDevice(FP32, nullptr, g, 3 * (size_t)dev_->args.nnode, stream);
+  const bool mask = maskHolds();
+  launch_bah(*dev_, FP64, FP32, x, d, t, nullptr, wantE, g, mask, minim_amd::Workspace::current().rs(),
+             static_cast<hipStream_t>(stream), wantE ? e_dev : nullptr);
+  if (g && !mask) constrainDevice(FP32, nullptr, g, 3 * (size_t)dev_->args.nnode, stream);
 }
 
-// An accepted first trial then needs no second energy pass and no separate
-// hinge pass for its gradient; xout holds exactly what the in-place update
-// x += t*d would (the same copy-and-axpy as the trial point).  With g null
-// the gradient is deferred: the energy pass keeps the hinge store for xout,
-// and the gradient evaluation at xout that follows runs only the gather.
+// x + t*d, formed exactly as the in-place update x += t*d would, goes to xout
+// from the pass that evaluates there.  With g null only the energy is
+// evaluated (the gradient is deferred until the trial is accepted).
 bool BarAndHinge::supportsStep() const { return dev_ != nullptr; }
 bool BarAndHinge::stepDefersGradient() const { return true; }
 
@@ -835,12 +832,24 @@ void BarAndHinge::evaluateStepAsync(int px, int pv, const void* x, const void* d
   if (!dev_) throw std::runtime_error("BarAndHinge: not initialised (construct a State first).");
   if (pv != px && !supportsMixed())
     throw std::invalid_argument("BarAndHinge: no mixed evaluation with normal constraints.");
+  const bool mask = maskHolds();
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const size_t n3 = 3 * (size_t)dev_->args.nnode;
-  minim_amd::device_copy(xout, x, n3 * (px == FP64 ? sizeof(double) : sizeof(float)), s);
-  minim_amd::launch_axpy_mixed(px, xout, pv, d, t, n3, s);
-  launch_bah(*dev_, px, pv, xout, nullptr, 0.0, true, g, minim_amd::Workspace::current().rs(), s, nullptr, !g);
-  if (g) constrainDevice(pv, pv == px ? xout : nullptr, g, n3, stream);
+  const size_t n3 = 3 * (size_t)dev_->args.nnode, bx = px == FP64 ? 8 : 4, bv = pv == FP64 ? 8 : 4;
+  auto overlap = [n3](const void* p, size_t bp, const void* q, size_t bq) {
+    const auto a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+    return p && q && a < b + n3 * bq && b < a + n3 * bp;
+  };
+  if (overlap(xout, bx, x, bx) || overlap(xout, bx, d, bv) || overlap(g, bv, x, bx) || overlap(g, bv, d, bv)) {
+    // a cluster reads x and d at its neighbours' nodes too: with an output over
+    // an input, the point is formed first
+    if (xout != x) minim_amd::device_copy(xout, x, n3 * bx, s);
+    minim_amd::launch_axpy_mixed(px, xout, pv, d, t, n3, s);
+    x = xout;
+    d = nullptr;
+    xout = nullptr;
+  }
+  launch_bah(*dev_, px, pv, x, d, t, xout, true, g, mask, minim_amd::Workspace::current().rs(), s);
+  if (g && !mask) constrainDevice(pv, pv == px ? (xout ? xout : x) : nullptr, g, n3, stream);
 }
 
 void BarAndHinge::evaluateMixed(const void* x, const void* d, double t, double* e, void* g, void* stream) const {
@@ -857,42 +866,33 @@ void BarAndHinge::evaluateMixed(const void* x, const void* d, double t, double* 
 // nodes (2) alone, in FP64 at the host coordinates.
 double BarAndHinge::componentEnergy(int component, const vector<double>& coords) const {
   if (!dev_) throw std::runtime_error("BarAndHinge: not initialised (construct a State first).");
-  auto a = dev_->args;
+  const auto& a = dev_->args;
   if ((size_t)coords.size() != 3 * (size_t)a.nnode)
     throw std::invalid_argument("BarAndHinge: coordinates have the wrong size.");
-  if (component != 0) a.nbar = 0;
-  if (component != 1) a.nhinge = 0;
-  if (component != 2) a.fz = nullptr;
-  if (component < 0 || component > 2 || (component == 2 && !dev_->args.fz)) return 0.0;
+  if (component < 0 || component > 2 || (component == 2 && !a.fz)) return 0.0;
   hipStream_t s = nullptr;
   auto& ws = minim_amd::Workspace::current();
   void* xd = minim_amd::Staging::current().device(0, coords.size() * sizeof(double));
   minim_amd::upload_raw(coords.data(), coords.size(), FP64, xd, s);
-  const size_t tot = (size_t)a.nbar + a.nhinge + a.nnode;
-  const int nb = minim_amd::grid_blocks(tot, 4, 2048);
-  minim_amd::bah_energy_kernel<double, false>
-      <<<nb, kBlock, 0, s>>>(a, (const double*)xd, (const double*)nullptr, 0.0, ws.rs(),
-                             (minim_amd::HStore<double>*)nullptr);
-  MINIM_HIP_CHECK(hipGetLastError());
-  minim_amd::launch_finalize(ws.rs(), 1, nb, s);
+  launch_bah(*dev_, FP64, FP64, xd, nullptr, 0.0, nullptr, true, nullptr, false, ws.rs(), s, nullptr, 1 << component);
   double r[1];
   ws.fetch(s, 1, r);
   return r[0];
 }
 
-// Average duration (ms) of reps evaluations on the device (energy kernel with
-// its reduction, gradient kernel; no constraints, no host copy).
+// Average duration (ms) of reps evaluations on the device (with the energy's
+// reduction; no constraints, no host copy).
 double BarAndHinge::timeKernel(int prec, const void* x, bool wantE, void* g, int reps, void* stream) const {
   if (!dev_) throw std::runtime_error("BarAndHinge: not initialised (construct a State first).");
   if ((!wantE && !g) || reps < 1) throw std::invalid_argument("BarAndHinge: nothing to time");
   hipStream_t s = static_cast<hipStream_t>(stream);
   auto& ws = minim_amd::Workspace::current();
-  launch_bah(*dev_, prec, prec, x, nullptr, 0.0, wantE, g, ws.rs(), s);
+  launch_bah(*dev_, prec, prec, x, nullptr, 0.0, nullptr, wantE, g, false, ws.rs(), s);
   hipEvent_t e0, e1;
   MINIM_HIP_CHECK(hipEventCreate(&e0));
   MINIM_HIP_CHECK(hipEventCreate(&e1));
   MINIM_HIP_CHECK(hipEventRecord(e0, s));
-  for (int i = 0; i < reps; i++) launch_bah(*dev_, prec, prec, x, nullptr, 0.0, wantE, g, ws.rs(), s);
+  for (int i = 0; i < reps; i++) launch_bah(*dev_, prec, prec, x, nullptr, 0.0, nullptr, wantE, g, false, ws.rs(), s);
   MINIM_HIP_CHECK(hipEventRecord(e1, s));
   MINIM_HIP_CHECK(hipEventSynchronize(e1));
   float ms = 0;

@@ -263,6 +263,73 @@ def test_bah_golden_vectors(gpu, case, prec):
         assert rel_err(g2, g) <= 1e-14
 
 
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("nnode", [8, 121, 700])
+def test_bah_any_lists_vs_oracle(gpu, nnode, prec):
+    """Bond and hinge lists that are no sheet, with their own parameters, a
+    force per node and single fixed components: every hinge at one hub (more
+    than a chunk of the kernel holds for 700 nodes), bars between any two
+    nodes.  The nodes lie on a unit sphere around the hub, and a hinge's
+    triangles have a sine of at least 0.7 at the hub, so that an element's
+    rounding stays within a few tens of its operands': TOL."""
+    import torch
+
+    m = gpu
+    print("case bah lists", nnode, prec, flush=True)
+    rng = np.random.default_rng(nnode)
+    p = rng.normal(size=(nnode, 3))
+    p /= np.linalg.norm(p, axis=1)[:, None]
+    hub = nnode // 3
+    p[hub] = 0
+    bars, hinges = [], []
+    for _ in range(3 * nnode):
+        a, b = rng.integers(nnode, size=2)
+        if a != b and np.linalg.norm(p[a] - p[b]) > 0.3:
+            bars.append((a, b))
+    for _ in range(40 * nnode):
+        i, j, k = rng.integers(nnode, size=3)
+        if hub not in (i, j, k) and len({i, j, k}) == 3 and max(abs(p[i] @ p[j]), abs(p[j] @ p[k])) < 0.7:
+            hinges.append((i, hub, j, k))
+    if nnode == 700:
+        assert len(hinges) > 4 * 480
+    nb, nh = len(bars), len(hinges)
+    bk, bl = rng.uniform(0.5, 2, nb), rng.uniform(0.5, 1, nb)
+    hk, ht = rng.uniform(0.5, 2, nh), rng.uniform(2, 4, nh)
+    force = rng.normal(size=3 * nnode)
+    fixed = rng.choice(3 * nnode, nnode // 2, replace=False)
+    x = p.reshape(-1)
+    x = r32(x) if prec == "fp32" else x
+    pot = m.BarAndHinge().setForce(force.tolist())
+    assert nb and nh
+    pot.setBondList(np.array(bars)).setHingeList(np.array(hinges)).setRigidity(bk, hk).setLength0(bl).setTheta0(ht)
+    pot.setConstraints(fixed.tolist())
+    fx = np.zeros(3 * nnode, np.uint8)
+    fx[fixed] = 1
+    o = OracleBaH(nnode, np.array(bars), bk, bl, np.array(hinges), hk, ht, force=force, force_per_node=True, fixed=fx)
+    s = m.State(pot, x, prec)
+    e, g = s.energyGradient(x)
+    eo, go = o.energy(x), o.gradient(x)
+    scale = np.sum(bk) + np.sum(hk) + np.sum(np.abs(force))  # the energy's terms have either sign
+    assert abs(e - eo) <= TOL[prec] * max(abs(eo), scale)
+    assert rel_err(g, go) <= TOL[prec]
+    assert np.all(g[fixed] == 0)
+    assert np.array_equal(s.gradient(x), g)
+    assert s.energy(x) == e
+    # the step: into a buffer of its own, and over its input
+    h = pot.handle(x)
+    dt = torch.float64 if prec == "fp64" else torch.float32
+    d = torch.tensor(rng.normal(0, 0.01, x.size), dtype=dt, device="cuda")
+    out = []
+    for over in (False, True):
+        xd = torch.tensor(x, dtype=dt, device="cuda")
+        xo = xd if over else torch.empty_like(xd)
+        gd = torch.empty_like(xd)
+        es = m.potential_eval_step(h, prec, prec, xd.data_ptr(), x.size, d.data_ptr(), 0.5, xo.data_ptr(), gd.data_ptr())
+        out.append((es, xo.cpu(), gd.cpu()))
+    assert out[0][0] == out[1][0]
+    assert torch.equal(out[0][1], out[1][1]) and torch.equal(out[0][2], out[1][2])
+
+
 def test_bah_two_triangle_minima(gpu):
     # BarAndHinge_test.cpp:13-56: L-BFGS minima for five rest angles, within 1e-4
     m = gpu
