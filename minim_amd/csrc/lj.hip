@@ -137,7 +137,7 @@ struct BoxArgs {
 // where both images are far beyond any cutoff.
 template <typename T>
 __device__ inline T min_image(T v, T L, T invL) {
-  return v - L * rint(v * invL);
+  return fma(-L, rint(v * invL), v);
 }
 
 template <typename T>
@@ -242,6 +242,15 @@ __host__ __device__ inline size_t nbr_at(int i, int k, int maxn) {
 }
 inline size_t nbr_elems(int N, int maxn) { return (size_t)((N + 63) / 64) * 64 * maxn; }
 
+// A list's rows are filled up to a multiple of kListPad (which maxn is too)
+// with the particle itself, which the force pass skips: it reads whole chunks.
+constexpr int kListPad = 32;
+__device__ inline void pad_list(int i, int cnt, int maxn, int* __restrict__ nn, int* __restrict__ nbr) {
+  const int n = min(cnt, maxn);
+  nn[i] = n;
+  for (int k = n; k % kListPad != 0; k++) nbr[nbr_at(i, k, maxn)] = i;
+}
+
 // A coordinate wrapped into [0, L), as the cell index takes it.
 __device__ __forceinline__ double wrap_box(double v, double L) { return v - L * floor(v / L); }
 
@@ -325,7 +334,7 @@ __global__ __launch_bounds__(kBlock) void lj_build_list_kernel(int N, BoxArgs b,
       }
     }
   }
-  nn[i] = cnt < maxn ? cnt : maxn;
+  pad_list(i, cnt, maxn, nn, nbr);
   if (cnt > maxn) atomicMax(overflow, cnt);
 }
 
@@ -356,107 +365,125 @@ __global__ __launch_bounds__(kBlock) void lj_build_list_brute_kernel(const T* __
       cnt++;
     }
   }
-  nn[i] = cnt < maxn ? cnt : maxn;
+  pad_list(i, cnt, maxn, nn, nbr);
   if (cnt > maxn) atomicMax(overflow, cnt);
 }
 
+// The evaluated point x + t*d, for a line-search trial.
 template <typename T>
-struct Vec4;
-template <>
-struct Vec4<float> {
-  using type = float4;
-};
-template <>
-struct Vec4<double> {
-  using type = double4;
-};
-
-// Positions at the evaluated point (x, or x + t*d) padded to four components,
-// so that the force pass reads a neighbour with one vector access.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void lj_pad_kernel(const T* __restrict__ x, const T* __restrict__ d, T t, int N,
-                                                        typename Vec4<T>::type* __restrict__ xp) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= N) return;
-  T p[3];
-  load_pos<T, 3>(x, d, t, i, p);
-  typename Vec4<T>::type v;
-  v.x = p[0];
-  v.y = p[1];
-  v.z = p[2];
-  v.w = (T)0;
-  xp[i] = v;
+__global__ __launch_bounds__(kBlock) void lj_point_kernel(const T* __restrict__ x, const T* __restrict__ d, T t,
+                                                          size_t n, T* __restrict__ xt) {
+  const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const T s = t * d[i];
+  xt[i] = x[i] + s;
 }
 
-// One thread per particle over its Verlet list, in chunks of U neighbours whose
-// indices and positions are all requested before any is used (the list rows
-// of a chunk are clamped to the last entry, and the repeats are skipped), so
-// the gathers overlap instead of forming one dependent chain per neighbour.
-// Positions come padded (lj_pad_kernel): one vector load per neighbour.
-// Pairs are summed in list order.  The same pass counts the particles that
-// have moved more than skin/2 since the list was built (reduction slot 1):
-// when any has, the caller rebuilds the list and evaluates again.  Blocks are
-// spread over the XCDs in contiguous ranges, so each L2 holds the positions
-// of one spatially coherent range of particles.  (Two to eight lanes per
-// particle, each taking every P-th entry, measured no faster at 262,144
-// particles.)
+// 1 / v by the hardware's estimate and Newton's iteration: within an ulp.
+__device__ __forceinline__ float newton_rcp(float v) {
+  const float r = __builtin_amdgcn_rcpf(v);
+  return __builtin_fmaf(__builtin_fmaf(-v, r, 1.0f), r, r);
+}
+__device__ __forceinline__ double newton_rcp(double v) {
+  double r = __builtin_amdgcn_rcp(v);
+  r = __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
+}
+
 template <typename T>
-__global__ __launch_bounds__(kBlock) void lj_cut_kernel(const typename Vec4<T>::type* __restrict__ xp, int N,
-                                                        BoxArgs b, T sig2, T eps, T eshift, int mode,
-                                                        const int* __restrict__ nn, const int* __restrict__ nbr,
-                                                        int maxn, const double* __restrict__ xbuild,
-                                                        T* __restrict__ g, RedScratch rs) {
-  constexpr int U = 8;
-  using V = typename Vec4<T>::type;
-  const int i = xcd_logical_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+struct Pos3 {
+  T c[3];
+};
+
+// P lanes per particle over its Verlet list, each taking U of every U P
+// entries: their indices and then their positions are all requested before any
+// is used.  Each lane sums its pairs in list order, and the lanes are added in
+// a fixed tree.  The same pass counts the particles that have moved more than
+// skin/2 since the list was built (reduction slot 1): when any has, the caller
+// rebuilds the list and evaluates again.  Blocks are spread over the XCDs in
+// contiguous ranges, so each L2 holds the positions of one spatially coherent
+// range of particles.  MODE bit 1 energy, bit 2 gradient.
+//
+// Bound by VALU issue, about 40 instructions per entry: the reciprocal by
+// Newton's iteration, fused products, constant factors and the energy shift
+// taken out of the loop, and list rows filled up to whole chunks instead of
+// clamped indices (69 before).  Positions are read in place, one 12-byte load
+// in FP32 and two loads in FP64.  Force pass at 262,144 particles: 31 us FP32,
+// 53 us FP64; with padded copies of the positions and one lane 43 and 69, and at
+// 32,768 particles 7.9 and 11.5 against 20 and 23.
+template <typename T, int P, int U, int MODE>
+__global__ __launch_bounds__(kBlock) void lj_cut_kernel(const T* __restrict__ x, int N, BoxArgs b, T sig2, double eps,
+                                                        double eshift, const int* __restrict__ nn,
+                                                        const int* __restrict__ nbr, int maxn,
+                                                        const double* __restrict__ xbuild, T* __restrict__ g,
+                                                        RedScratch rs) {
+  static_assert(kListPad % (P * U) == 0, "whole chunks");
+  constexpr bool WE = MODE & 1, WG = MODE & 2;
+  const int tid = xcd_logical_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+  const int i = tid / P, sub = tid % P;
+  auto at = [&](unsigned j) {
+    // a 32-bit byte offset from a uniform base
+    return *reinterpret_cast<const Pos3<T>*>(reinterpret_cast<const char*>(x) + j * (unsigned)sizeof(Pos3<T>));
+  };
   double ei = 0.0, moved = 0.0;
   if (i < N) {
-    const V vi = xp[i];
-    const T xi[3] = {vi.x, vi.y, vi.z};
-    double dr2 = 0;
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const double v = (double)xi[k] - xbuild[(size_t)i * 3 + k];
-      dr2 += v * v;
-    }
-    if (dr2 > b.half_skin2) moved = 1.0;
+    const Pos3<T> xi = at(i);
     const T L0 = (T)b.L[0], L1 = (T)b.L[1], L2 = (T)b.L[2];
     const T rc2 = (T)b.rc2;
     const T iL0 = (T)b.invL[0], iL1 = (T)b.invL[1], iL2 = (T)b.invL[2];
     T gi[3] = {(T)0, (T)0, (T)0};
+    int pairs = 0;
     const int cnt = nn[i];
-    for (int k0 = 0; k0 < cnt; k0 += U) {
+    const int* row = nbr + nbr_at(i, sub, maxn);
+    for (int k0 = 0; k0 < cnt; k0 += U * P, row += U * P * 64) {
       int jj[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) jj[u] = nbr[nbr_at(i, min(k0 + u, cnt - 1), maxn)];
-      V xj[U];
+      for (int u = 0; u < U; u++) jj[u] = row[u * P * 64];
+      Pos3<T> xj[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) xj[u] = xp[jj[u]];
+      for (int u = 0; u < U; u++) xj[u] = at(jj[u]);
 #pragma unroll
       for (int u = 0; u < U; u++) {
-        if (k0 + u >= cnt) break;
-        const T r0 = min_image(xi[0] - xj[u].x, L0, iL0);
-        const T r1 = min_image(xi[1] - xj[u].y, L1, iL1);
-        const T r2v = min_image(xi[2] - xj[u].z, L2, iL2);
-        const T r2 = r0 * r0 + r1 * r1 + r2v * r2v;
-        if (r2 >= rc2) continue;
-        const T ir2 = (T)1 / r2;  // one division per pair
+        const T r0 = min_image(xi.c[0] - xj[u].c[0], L0, iL0);
+        const T r1 = min_image(xi.c[1] - xj[u].c[1], L1, iL1);
+        const T r2v = min_image(xi.c[2] - xj[u].c[2], L2, iL2);
+        const T r2 = fma(r0, r0, fma(r1, r1, r2v * r2v));
+        const bool in = !(r2 >= rc2) && jj[u] != i;
+        const T ir2 = in ? newton_rcp(r2) : (T)0;
         const T s2 = sig2 * ir2;
         const T lj6 = s2 * s2 * s2;
-        const T lj12 = lj6 * lj6;
-        if (mode & 1) ei += 0.5 * ((double)((T)4 * eps * (lj12 - lj6)) - (double)eshift);
-        if (mode & 2) {
-          const T f = (T)-24 * eps * ((T)2 * lj12 - lj6) * ir2;
-          gi[0] += r0 * f;
-          gi[1] += r1 * f;
-          gi[2] += r2v * f;
+        if (WE) {
+          ei += (double)fma(lj6, lj6, -lj6);
+          pairs += in;
+        }
+        if (WG) {
+          const T f = fma((T)2 * lj6, lj6, -lj6) * ir2;
+          gi[0] = fma(r0, f, gi[0]);
+          gi[1] = fma(r1, f, gi[1]);
+          gi[2] = fma(r2v, f, gi[2]);
         }
       }
     }
-    if (mode & 2) {
-      g[(size_t)i * 3] = gi[0];
-      g[(size_t)i * 3 + 1] = gi[1];
-      g[(size_t)i * 3 + 2] = gi[2];
+    if (WE) ei = 0.5 * (4 * eps * ei - pairs * eshift);
+    if (WG) {
+#pragma unroll
+      for (int off = 1; off < P; off <<= 1)
+#pragma unroll
+        for (int k = 0; k < 3; k++) gi[k] += __shfl_xor(gi[k], off, kWave);
+    }
+    if (sub == 0) {
+      double dr2 = 0;
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const double v = (double)xi.c[k] - xbuild[(size_t)i * 3 + k];
+        dr2 += v * v;
+      }
+      if (dr2 > b.half_skin2) moved = 1.0;
+      if (WG) {
+        const T f = (T)(-24 * eps);
+#pragma unroll
+        for (int k = 0; k < 3; k++) g[(size_t)i * 3 + k] = f * gi[k];
+      }
     }
   }
   double acc[2] = {ei, moved};
@@ -514,10 +541,10 @@ using minim_amd::kBlock;
 struct LjNd::Impl {
   minim_amd::BoxArgs box{};
   bool cellMode = false;
-  int maxn = 128;
+  int maxn = 128;  // a multiple of kListPad
   long builds = 0;
   bool built = false;
-  DeviceBuffer cell, count, start, cursor, order, nn, nbr, flag, xbuild, xpad, xcell;
+  DeviceBuffer cell, count, start, cursor, order, nn, nbr, flag, xbuild, xtrial, xcell;
   int ncell = 0;
 };
 
@@ -605,30 +632,58 @@ void LjNd::init(const vector<double>& coords) {
     impl_->nbr.reset(sizeof(int) * minim_amd::nbr_elems(N, impl_->maxn));
     impl_->flag.reset(sizeof(int));
     impl_->xbuild.reset(sizeof(double) * 3 * N);
-    impl_->xpad.reset(sizeof(double) * 4 * N);
   }
 }
 
 namespace {
-int cut_blocks(int N) { return (N + kBlock - 1) / kBlock; }
+// Lanes per particle of the force pass: as many as 512 blocks (two per CU) hold.
+// One lane per particle leaves small systems waiting for a chain of 80 list
+// entries (4,096 particles, FP64: 15.3 us with one lane, 5.0 with 16); where one
+// fills the chip, more lanes only add their sums and unused entries (262,144,
+// FP64: 53 us with one, 56 with two).
+int cut_lanes(int N) {
+  int p = 16;
+  while (p > 1 && (size_t)N * p > 512 * (size_t)kBlock) p /= 2;
+  return p;
+}
+int cut_blocks(int N) { return (int)(((size_t)N * cut_lanes(N) + kBlock - 1) / kBlock); }
 
-void launch_cut(const LjNd::Impl& I, int prec, const void* x, const void* d, double t, int N, double sigma,
-                double epsilon, double eshift, int mode, void* g, minim_amd::RedScratch rs, hipStream_t s) {
-  const int nb = cut_blocks(N);
-  if (prec == FP64) {
-    auto* xp = (double4*)I.xpad.get();
-    minim_amd::lj_pad_kernel<double><<<nb, kBlock, 0, s>>>((const double*)x, (const double*)d, t, N, xp);
-    minim_amd::lj_cut_kernel<double><<<nb, kBlock, 0, s>>>(xp, N, I.box, sigma * sigma, epsilon, eshift, mode,
-                                                           (const int*)I.nn.get(), (const int*)I.nbr.get(), I.maxn,
-                                                           (const double*)I.xbuild.get(), (double*)g, rs);
-  } else {
-    auto* xp = (float4*)I.xpad.get();
-    minim_amd::lj_pad_kernel<float><<<nb, kBlock, 0, s>>>((const float*)x, (const float*)d, (float)t, N, xp);
-    minim_amd::lj_cut_kernel<float><<<nb, kBlock, 0, s>>>(xp, N, I.box, (float)(sigma * sigma), (float)epsilon,
-                                                          (float)eshift, mode, (const int*)I.nn.get(),
-                                                          (const int*)I.nbr.get(), I.maxn,
-                                                          (const double*)I.xbuild.get(), (float*)g, rs);
+template <typename T>
+void launch_cut_t(LjNd::Impl& I, const T* x, const T* d, T t, int N, double sigma, double eps, double eshift, int mode,
+                  T* g, minim_amd::RedScratch rs, hipStream_t s) {
+  if (d) {
+    const size_t n = 3 * (size_t)N;
+    if (I.xtrial.bytes() < n * sizeof(double)) I.xtrial.reset(n * sizeof(double));
+    T* xt = static_cast<T*>(I.xtrial.get());
+    minim_amd::lj_point_kernel<T><<<(int)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>(x, d, t, n, xt);
+    x = xt;
   }
+  auto go = [&](auto lanes, auto unroll) {
+    constexpr int P = decltype(lanes)::value, U = decltype(unroll)::value;
+    auto run = [&](auto kernel) {
+      kernel<<<cut_blocks(N), kBlock, 0, s>>>(x, N, I.box, (T)(sigma * sigma), eps, eshift, (const int*)I.nn.get(),
+                                              (const int*)I.nbr.get(), I.maxn, (const double*)I.xbuild.get(), g, rs);
+    };
+    if (mode == 1) run(minim_amd::lj_cut_kernel<T, P, U, 1>);
+    else if (mode == 2) run(minim_amd::lj_cut_kernel<T, P, U, 2>);
+    else run(minim_amd::lj_cut_kernel<T, P, U, 3>);
+  };
+  using std::integral_constant;
+  switch (cut_lanes(N)) {
+    case 1: go(integral_constant<int, 1>(), integral_constant<int, 8>()); break;
+    case 2: go(integral_constant<int, 2>(), integral_constant<int, 8>()); break;
+    case 4: go(integral_constant<int, 4>(), integral_constant<int, 8>()); break;
+    case 8: go(integral_constant<int, 8>(), integral_constant<int, 4>()); break;
+    default: go(integral_constant<int, 16>(), integral_constant<int, 2>()); break;
+  }
+}
+
+void launch_cut(LjNd::Impl& I, int prec, const void* x, const void* d, double t, int N, double sigma, double epsilon,
+                double eshift, int mode, void* g, minim_amd::RedScratch rs, hipStream_t s) {
+  if (prec == FP64)
+    launch_cut_t(I, (const double*)x, (const double*)d, t, N, sigma, epsilon, eshift, mode, (double*)g, rs, s);
+  else
+    launch_cut_t(I, (const float*)x, (const float*)d, (float)t, N, sigma, epsilon, eshift, mode, (float*)g, rs, s);
   MINIM_HIP_CHECK(hipGetLastError());
 }
 
@@ -689,7 +744,7 @@ void rebuild_list(LjNd::Impl& I, int prec, const void* x, const void* d, double 
     MINIM_HIP_CHECK(hipStreamSynchronize(s));
     if (over == 0) break;
     if (attempt == 1) throw std::runtime_error("LjNd: neighbour list overflow");
-    I.maxn = over + 32;
+    I.maxn = (over + 2 * minim_amd::kListPad - 1) / minim_amd::kListPad * minim_amd::kListPad;
     I.nbr.reset(sizeof(int) * minim_amd::nbr_elems(N, I.maxn));
   }
   I.built = true;
@@ -709,7 +764,7 @@ void LjNd::evaluate(int prec, const void* x, const void* d, double t, double* e,
     else minim_amd::launch_allpairs<float>(nDim, x, d, t, N, sigma, epsilon, mode, g, ws.rs(), s);
   } else {
     Impl& I = *impl_;
-    if ((N + kBlock - 1) / kBlock > minim_amd::kMaxRedBlocks)
+    if (cut_blocks(N) > minim_amd::kMaxRedBlocks)
       throw std::invalid_argument("LjNd: too many particles for one launch");
     const double src6 = std::pow(sigma / cutoff, 6);
     const double eshift = 4 * epsilon * (src6 * src6 - src6);
