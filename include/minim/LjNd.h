@@ -45,6 +45,8 @@ class LjNd : public NewPotential<LjNd> {
   void init(const vector<double>& coords) override;
   void evaluate(int prec, const void* x, const void* d, double t, double* e, void* g,
                 void* stream) const override;
+  void evaluateAsync(int prec, const void* x, const void* d, double t, bool wantE, double* e_dev, void* g,
+                     void* stream) const override;
   double timeKernel(int prec, const void* x, bool wantE, void* g, int reps, void* stream) const override;
   int gradientDeferred(int prec, const void* x, void* g, void* stream) const override;
   void redoGradient(int prec, const void* x, void* g, void* stream) const override;
@@ -60,6 +62,8 @@ class LjNd : public NewPotential<LjNd> {
 
  private:
   std::shared_ptr<Impl> impl_;  // device neighbour-list state (rebuilt lazily)
+  void launch(int prec, const void* x, const void* d, double t, bool wantE, double* eDev, void* g,
+              void* stream) const;
 };
 
 class Lj2d : public LjNd {

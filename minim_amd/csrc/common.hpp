@@ -86,6 +86,9 @@ __device__ inline void block_sum(double (&v)[K], double* lds) {
 struct RedScratch {
   double* partials;  // [kMaxDots][kMaxRedBlocks], value k of block b at k * gridDim + b
   double* result;    // [kMaxDots]
+  double* mirror = nullptr;  // the same values in pinned host memory, for Workspace::fetch
+  // The same scratch with results from slot k on.
+  RedScratch from(int k) const { return {partials, result + k, mirror ? mirror + k : nullptr}; }
 };
 
 // All threads of the (1-D) grid must call this; v is each thread's contribution.

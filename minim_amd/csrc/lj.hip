@@ -510,7 +510,7 @@ int launch_allpairs_d(const T* x, const T* d, T t, int N, T sig6, T eps, int mod
 
 template <typename T>
 void launch_allpairs(int D, const void* x, const void* d, double t, int N, double sigma, double eps, int mode, void* g,
-                     RedScratch rs, hipStream_t s) {
+                     RedScratch rs, hipStream_t s, double* eDev = nullptr) {
   if (N < 1) throw std::invalid_argument("LjNd: no particles");
   if ((N + kBlock - 1) / kBlock > kMaxRedBlocks)
     throw std::invalid_argument("LjNd: too many particles for the all-pairs kernel");
@@ -527,7 +527,7 @@ void launch_allpairs(int D, const void* x, const void* d, double t, int N, doubl
     default: throw std::invalid_argument("LjNd: nDim must be 1..4 on the device path");
   }
   MINIM_HIP_CHECK(hipGetLastError());
-  launch_finalize(rs, 1, nb, s);
+  launch_finalize(rs, 1, nb, s, 0, (mode & 1) ? eDev : nullptr);
 }
 
 }  // namespace
@@ -752,16 +752,18 @@ void rebuild_list(LjNd::Impl& I, int prec, const void* x, const void* d, double 
 }
 }  // namespace
 
-void LjNd::evaluate(int prec, const void* x, const void* d, double t, double* e, void* g, void* stream) const {
+// Energy (result slot 0, and eDev when given) and gradient, without waiting for
+// them: except in cutoff mode, where the list check is read.
+void LjNd::launch(int prec, const void* x, const void* d, double t, bool wantE, double* eDev, void* g,
+                  void* stream) const {
   if (!impl_) throw std::runtime_error("LjNd: not initialised (construct a State first).");
   hipStream_t s = static_cast<hipStream_t>(stream);
   auto& ws = minim_amd::Workspace::current();
-  const int mode = (e ? 1 : 0) | (g ? 2 : 0);
-  if (!mode) return;
+  const int mode = (wantE ? 1 : 0) | (g ? 2 : 0);
   const int N = nParticle;
   if (cutoff <= 0) {
-    if (prec == FP64) minim_amd::launch_allpairs<double>(nDim, x, d, t, N, sigma, epsilon, mode, g, ws.rs(), s);
-    else minim_amd::launch_allpairs<float>(nDim, x, d, t, N, sigma, epsilon, mode, g, ws.rs(), s);
+    if (prec == FP64) minim_amd::launch_allpairs<double>(nDim, x, d, t, N, sigma, epsilon, mode, g, ws.rs(), s, eDev);
+    else minim_amd::launch_allpairs<float>(nDim, x, d, t, N, sigma, epsilon, mode, g, ws.rs(), s, eDev);
   } else {
     Impl& I = *impl_;
     if (cut_blocks(N) > minim_amd::kMaxRedBlocks)
@@ -770,7 +772,7 @@ void LjNd::evaluate(int prec, const void* x, const void* d, double t, double* e,
     const double eshift = 4 * epsilon * (src6 * src6 - src6);
     auto launch_force = [&]() {
       launch_cut(I, prec, x, d, t, N, sigma, epsilon, eshift, mode, g, ws.rs(), s);
-      minim_amd::launch_finalize(ws.rs(), 2, cut_blocks(N), s);
+      minim_amd::launch_finalize(ws.rs(), 2, cut_blocks(N), s, 0, wantE ? eDev : nullptr);
     };
     if (!I.built) rebuild_list(I, prec, x, d, t, N, s);
     launch_force();
@@ -779,18 +781,26 @@ void LjNd::evaluate(int prec, const void* x, const void* d, double t, double* e,
     if (r[1] > 0) {
       rebuild_list(I, prec, x, d, t, N, s);
       launch_force();
-      ws.fetch(s, 2, r);
     }
-    if (g) constrainDevice(prec, x, g, (size_t)N * nDim, stream);
-    if (e) *e = r[0];
-    return;
   }
   if (g) constrainDevice(prec, x, g, (size_t)N * nDim, stream);
+}
+
+void LjNd::evaluate(int prec, const void* x, const void* d, double t, double* e, void* g, void* stream) const {
+  if (!impl_) throw std::runtime_error("LjNd: not initialised (construct a State first).");
+  if (!e && !g) return;
+  launch(prec, x, d, t, e != nullptr, nullptr, g, stream);
   if (e) {
     double r[1];
-    ws.fetch(s, 1, r);
+    minim_amd::Workspace::current().fetch(static_cast<hipStream_t>(stream), 1, r);
     *e = r[0];
   }
+}
+
+void LjNd::evaluateAsync(int prec, const void* x, const void* d, double t, bool wantE, double* e_dev, void* g,
+                         void* stream) const {
+  if (!impl_) throw std::runtime_error("LjNd: not initialised (construct a State first).");
+  if (wantE || g) launch(prec, x, d, t, wantE, e_dev, g, stream);
 }
 
 // Cutoff mode: the force pass without the host synchronisation of the list
@@ -806,7 +816,7 @@ int LjNd::gradientDeferred(int prec, const void* x, void* g, void* stream) const
   const double src6 = std::pow(sigma / cutoff, 6);
   const double eshift = 4 * epsilon * (src6 * src6 - src6);
   launch_cut(I, prec, x, nullptr, 0.0, N, sigma, epsilon, eshift, 2, g, ws.rs(), s);
-  minim_amd::launch_finalize(ws.rs(), 2, cut_blocks(N), s, 1, ws.device_result() + minim_amd::kDeferSlot);
+  minim_amd::launch_finalize(ws.rs(), 2, cut_blocks(N), s, 1, ws.rs().mirror + minim_amd::kDeferSlot);
   constrainDevice(prec, x, g, (size_t)N * nDim, stream);
   return minim_amd::kDeferSlot;
 }

@@ -594,7 +594,7 @@ void Lbfgs::iteration(State& state) {
   const bool defer = fused && state.pot->stepDefersGradient();
   constexpr int kStash = 48;
   minim_amd::RedScratch rd = ws.rs();
-  if (spec) rd.result += kStash;
+  if (spec) rd = rd.from(kStash);
   minim_amd::launch_direction(a, prec, rd, s);
   std::vector<double> dres(1 + a.ndot);
   double ddPre = 0;
@@ -907,7 +907,7 @@ void Fire::iteration(State& state) {
     const void* pb[3] = {I.g.data(), I.g.data(), I.v.data()};
     constexpr int kStash = 48;  // with the largest force in slot 0, the dots go to [48, 51)
     minim_amd::RedScratch rd = ws.rs();
-    if (_maxForceDim > 0) rd.result += kStash;
+    if (_maxForceDim > 0) rd = rd.from(kStash);
     minim_amd::launch_dots(I.prec, pa, pb, 3, I.n, rd, s);
     std::array<double, minim_amd::kMaxDots> q;
     int nfetch = 3;

@@ -935,7 +935,7 @@ template <typename T>
 void volproj_t(const PFArgs& a, void* v, size_t nsite, bool norm, RedScratch rs, hipStream_t s) {
   T* u = static_cast<T*>(v);
   const int nb = grid_blocks(nsite, 4, 2048);
-  RedScratch slot{rs.partials, rs.result + kPFVolSlot};
+  const RedScratch slot = rs.from(kPFVolSlot);
   switch (a.nf) {
     case 2: pf_volproj_reduce_kernel<T, 2><<<nb, kBlock, 0, s>>>(a, u, nsite, slot); break;
     case 3: pf_volproj_reduce_kernel<T, 3><<<nb, kBlock, 0, s>>>(a, u, nsite, slot); break;
@@ -952,7 +952,7 @@ void volproj_t(const PFArgs& a, void* v, size_t nsite, bool norm, RedScratch rs,
       case 4: pf_volproj_apply_kernel<T, 4, true><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, rs); break;
       default: pf_volproj_apply_kernel<T, 0, true><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, rs); break;
     }
-    launch_finalize(RedScratch{rs.partials, rs.result + 1}, 1, nb, s);
+    launch_finalize(rs.from(1), 1, nb, s);
   } else {
     switch (a.nf) {
       case 2: pf_volproj_apply_kernel<T, 2, false><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, rs); break;

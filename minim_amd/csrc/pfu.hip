@@ -619,7 +619,7 @@ __global__ __launch_bounds__(kBlock) void pfu_volumes_kernel(PFUArgs u, const T*
 // volCoef * volDiff per fluid, and (with the energy) the term's energy added to
 // the elements' (:295-300).  One thread.
 __global__ void pfu_volfix_kernel(PFUArgs u, const double* __restrict__ vol, double* __restrict__ energy,
-                                  int want_energy, double* eOut) {
+                                  double* mirror, int want_energy, double* eOut) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   double e = want_energy ? energy[0] : 0.0;
   for (int k = 0; k < u.nf; k++) {
@@ -628,6 +628,7 @@ __global__ void pfu_volfix_kernel(PFUArgs u, const double* __restrict__ vol, dou
     u.volg[k] = u.vol_coef * diff;
   }
   if (want_energy) energy[0] = e;
+  if (want_energy && mirror) mirror[0] = e;
   if (eOut) *eOut = e;
 }
 
@@ -701,14 +702,14 @@ void eval_t(const PFUArgs& u, const PFArgs& con, int mode, const void* x, const 
   MINIM_HIP_CHECK(hipGetLastError());
   launch_finalize(rs, 1, nb, s, 0, (mode & 1) && !u.volfix ? eOut : nullptr);
   if (u.volfix) {
-    RedScratch slot{rs.partials, rs.result + kPFVolSlot};
+    const RedScratch slot = rs.from(kPFVolSlot);
     const int nbv = grid_blocks(u.ngrid, 4, 2048);
     if (mode & 4)
       pfu_volumes_kernel<T, T, true><<<nbv, kBlock, 0, s>>>(u, xx, dd, tt, slot);
     else
       pfu_volumes_kernel<T, T, false><<<nbv, kBlock, 0, s>>>(u, xx, dd, tt, slot);
     launch_finalize(slot, kPFMaxFluid, nbv, s);
-    pfu_volfix_kernel<<<1, 64, 0, s>>>(u, rs.result + kPFVolSlot, rs.result, (mode & 1) ? 1 : 0,
+    pfu_volfix_kernel<<<1, 64, 0, s>>>(u, rs.result + kPFVolSlot, rs.result, rs.mirror, (mode & 1) ? 1 : 0,
                                        (mode & 1) ? eOut : nullptr);
     if (mode & 2) pfu_volgrad_kernel<T, T, false><<<grid_blocks(nd, 4, 4096), kBlock, 0, s>>>(u, xx, dd, tt, gg);
     MINIM_HIP_CHECK(hipGetLastError());

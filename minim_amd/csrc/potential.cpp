@@ -399,9 +399,13 @@ void Potential::evaluateAsync(int prec, const void* x, const void* d, double t, 
   if (wantE) {
     // the value goes where the library's own potentials leave it: e_dev, or
     // the calling thread's reduction result slot 0
-    double* dst = e_dev ? e_dev : minim_amd::Workspace::current().device_result();
-    MINIM_HIP_CHECK(hipMemcpyAsync(dst, &e, sizeof(double), hipMemcpyHostToDevice, static_cast<hipStream_t>(stream)));
-    MINIM_HIP_CHECK(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (!e_dev) {
+      minim_amd::Workspace::current().put(s, 0, e);
+      return;
+    }
+    MINIM_HIP_CHECK(hipMemcpyAsync(e_dev, &e, sizeof(double), hipMemcpyHostToDevice, s));
+    MINIM_HIP_CHECK(hipStreamSynchronize(s));
   }
 }
 

@@ -36,7 +36,8 @@ void DeviceBuffer::reset(size_t bytes) {
 namespace {
 // One block per reduced value: partials of value k are contiguous.
 __global__ __launch_bounds__(kBlock) void finalize_kernel(const double* __restrict__ partials, int nb,
-                                                          double* __restrict__ result, int dupK, double* dupDst) {
+                                                          double* __restrict__ result, double* mirror, int dupK,
+                                                          double* dupDst) {
   __shared__ double lds[kBlock / kWave];
   const int k = blockIdx.x;
   const double* p = partials + (size_t)k * nb;
@@ -45,6 +46,7 @@ __global__ __launch_bounds__(kBlock) void finalize_kernel(const double* __restri
   block_sum<1>(v, lds);
   if (threadIdx.x == 0) {
     result[k] = v[0];
+    if (mirror) mirror[k] = v[0];
     if (k == dupK) *dupDst = v[0];
   }
 }
@@ -54,7 +56,7 @@ void launch_finalize(RedScratch rs, int K, int nb, hipStream_t s, int dupK, doub
   if (K < 1 || K > kMaxDots || nb < 1 || nb > kMaxRedBlocks)
     throw std::invalid_argument("reduction shape out of range");
   if (!dupDst) dupK = -1;
-  finalize_kernel<<<K, kBlock, 0, s>>>(rs.partials, nb, rs.result, dupK, dupDst);
+  finalize_kernel<<<K, kBlock, 0, s>>>(rs.partials, nb, rs.result, rs.mirror, dupK, dupDst);
   MINIM_HIP_CHECK(hipGetLastError());
 }
 
@@ -65,7 +67,10 @@ Workspace::Workspace() {
   char* base = static_cast<char*>(mem_.get());
   rs_.partials = reinterpret_cast<double*>(base);
   rs_.result = reinterpret_cast<double*>(base + partial_bytes);
-  MINIM_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_), result_bytes, hipHostMallocDefault));
+  MINIM_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_), result_bytes, hipHostMallocCoherent));
+  void* dev = nullptr;
+  MINIM_HIP_CHECK(hipHostGetDevicePointer(&dev, host_, 0));
+  rs_.mirror = static_cast<double*>(dev);
 }
 
 Workspace::~Workspace() {
@@ -86,9 +91,14 @@ Workspace& Workspace::current() {
 }
 
 void Workspace::fetch(hipStream_t s, int k, double* out) {
-  MINIM_HIP_CHECK(hipMemcpyAsync(host_, rs_.result, sizeof(double) * k, hipMemcpyDeviceToHost, s));
   MINIM_HIP_CHECK(hipStreamSynchronize(s));
   for (int i = 0; i < k; i++) out[i] = host_[i];
+}
+
+void Workspace::put(hipStream_t s, int slot, double value) {
+  MINIM_HIP_CHECK(hipMemcpyAsync(rs_.result + slot, &value, sizeof(double), hipMemcpyHostToDevice, s));
+  MINIM_HIP_CHECK(hipStreamSynchronize(s));
+  host_[slot] = value;
 }
 
 namespace {

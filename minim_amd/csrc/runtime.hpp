@@ -58,14 +58,17 @@ class Workspace {
   Workspace(const Workspace&) = delete;
   Workspace& operator=(const Workspace&) = delete;
   RedScratch rs() const { return rs_; }
-  // Copy result[0..k) to host (synchronising stream s) into out.
+  // Wait for stream s and copy result[0..k) into out.  Whatever writes a result
+  // slot on the device also writes its mirror in pinned host memory, so no copy
+  // is launched.
   void fetch(hipStream_t s, int k, double* out);
-  double* device_result() const { return rs_.result; }
+  // A result slot set by the host, ordered after the work on stream s.
+  void put(hipStream_t s, int slot, double value);
 
  private:
   Workspace();
   RedScratch rs_{};
-  double* host_ = nullptr;
+  double* host_ = nullptr;  // the mirror, as the host sees it
   DeviceBuffer mem_;
 };
 

@@ -478,7 +478,7 @@ __global__ __launch_bounds__(kBlock) void group_norm_max_kernel(const T* __restr
 }
 
 __global__ __launch_bounds__(kBlock) void max_sqrt_finalize_kernel(const double* __restrict__ partial, int nb,
-                                                                   double* __restrict__ result) {
+                                                                   double* __restrict__ result, double* mirror) {
   double m = 0.0;
   for (int b = threadIdx.x; b < nb; b += kBlock) m = nan_max(m, partial[b]);
   for (int off = kWave / 2; off > 0; off >>= 1) m = nan_max(m, __shfl_xor(m, off, kWave));
@@ -488,6 +488,7 @@ __global__ __launch_bounds__(kBlock) void max_sqrt_finalize_kernel(const double*
   if (threadIdx.x == 0) {
     for (int w = 1; w < kBlock / kWave; w++) m = nan_max(m, lds[w]);
     result[0] = sqrt(m);
+    if (mirror) mirror[0] = sqrt(m);
   }
 }
 
@@ -651,7 +652,7 @@ void launch_group_norm_max(int prec, const void* v, size_t n, int dim, RedScratc
   if (prec == F64) group_norm_max_kernel<double><<<nb, kBlock, 0, s>>>((const double*)v, ngroup, dim, rs.partials);
   else group_norm_max_kernel<float><<<nb, kBlock, 0, s>>>((const float*)v, ngroup, dim, rs.partials);
   MINIM_HIP_CHECK(hipGetLastError());
-  max_sqrt_finalize_kernel<<<1, kBlock, 0, s>>>(rs.partials, nb, rs.result);
+  max_sqrt_finalize_kernel<<<1, kBlock, 0, s>>>(rs.partials, nb, rs.result, rs.mirror);
   MINIM_HIP_CHECK(hipGetLastError());
 }
 
