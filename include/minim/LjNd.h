@@ -50,6 +50,8 @@ class LjNd : public NewPotential<LjNd> {
   double timeKernel(int prec, const void* x, bool wantE, void* g, int reps, void* stream) const override;
   int gradientDeferred(int prec, const void* x, void* g, void* stream) const override;
   void redoGradient(int prec, const void* x, void* g, void* stream) const override;
+  bool fusesFire(int dim) const override;
+  void fireGradient(int prec, const void* x, void* g, const void* v, int dim, bool again, void* stream) const override;
 
   // Statistics of the neighbour list (cutoff mode) of this object's device
   // state: a State evaluates its own copy of the potential (state.pot).

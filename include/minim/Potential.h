@@ -217,6 +217,13 @@ class Potential {
   // next fetch), or -1 when the gradient is complete (the default: evaluate).
   virtual int gradientDeferred(int prec, const void* x, void* g, void* stream) const;
   virtual void redoGradient(int prec, const void* x, void* g, void* stream) const;
+  // FIRE's gradient with the sums it needs in the same pass: result slots 0 to 5
+  // hold g.g, v.g, v.v, two values that are nonzero when the gradient must be
+  // evaluated again (again: it is this evaluation), and the largest norm over
+  // groups of dim components of g (0 for dim 0).  Only where fusesFire(dim),
+  // which also says that steps need no constraint.
+  virtual bool fusesFire(int) const { return false; }
+  virtual void fireGradient(int, const void*, void*, const void*, int, bool, void*) const {}
   // True when constrainDevice does more than the per-site projection:
   // constraints that couple all DOFs (PhaseField's fixed total volumes,
   // PhaseField.cpp:614-658), normal constraints, or the constraints of a

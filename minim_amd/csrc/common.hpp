@@ -105,8 +105,21 @@ __device__ inline void grid_sum_store(double (&v)[K], RedScratch rs) {
 
 // Second stage: result[k] = sum over the nb partials of value k, in a fixed
 // order (stream-ordered after the producing kernel).  With dupDst, value dupK
-// is also written there (a caller's device slot: no copy launch after).
-void launch_finalize(RedScratch rs, int K, int nb, hipStream_t s, int dupK = -1, double* dupDst = nullptr);
+// is also written there (a caller's device slot: no copy launch after).  Value
+// maxK, if any, is the square root of the largest partial instead (a NaN wins).
+void launch_finalize(RedScratch rs, int K, int nb, hipStream_t s, int dupK = -1, double* dupDst = nullptr,
+                     int maxK = -1);
+
+// NaN-propagating maximum
+__device__ inline double nan_max(double a, double b) { return (b > a || b != b) ? b : a; }
+// Block-wide nan_max; valid in thread 0.  lds must hold kBlock/kWave doubles.
+__device__ inline double block_max(double m, double* lds) {
+  for (int off = kWave / 2; off > 0; off >>= 1) m = nan_max(m, __shfl_xor(m, off, kWave));
+  if (threadIdx.x % kWave == 0) lds[threadIdx.x / kWave] = m;
+  __syncthreads();
+  for (int w = 0; w < kBlock / kWave; w++) m = nan_max(m, lds[w]);
+  return m;
+}
 
 // MI355X dispatches consecutive workgroups round-robin over its 8 XCDs, each
 // with a private L2.  Remap the hardware block id so that every XCD receives a

@@ -162,6 +162,12 @@ __global__ __launch_bounds__(kBlock) void lj_cell_index_kernel(const T* __restri
   atomicAdd(&count[id], 1);
 }
 
+// Zero cell counts and overflow flag.
+__global__ __launch_bounds__(kBlock) void lj_clear_kernel(int* __restrict__ count, int ncell, int* __restrict__ flag) {
+  for (int c = blockIdx.x * kBlock + threadIdx.x; c < ncell; c += gridDim.x * kBlock) count[c] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
+}
+
 // Exclusive scan of cell counts by a single block (cell counts are small).
 __global__ __launch_bounds__(kBlock) void lj_scan_kernel(const int* __restrict__ count, int* __restrict__ start,
                                                          int* __restrict__ cursor, int ncell) {
@@ -200,32 +206,46 @@ __global__ __launch_bounds__(kBlock) void lj_fill_kernel(const int* __restrict__
   order[pos] = i;
 }
 
+// A coordinate wrapped into [0, L), as the cell index takes it.
+__device__ __forceinline__ double wrap_box(double v, double L) { return v - L * floor(v / L); }
+
 // Sort each cell's members by particle id so the neighbour order is
 // reproducible: one wavefront per cell; with up to 64 members each lane
 // holds one and computes its rank by comparing with the others (ids are
 // distinct, so the ranks are a permutation); larger cells are sorted by one
-// lane with an insertion sort.
-__global__ __launch_bounds__(kBlock) void lj_sort_cells_kernel(const int* __restrict__ start, int* __restrict__ order,
-                                                               int ncell) {
+// lane with an insertion sort.  The members' positions go out in that order,
+// wrapped into the box, each with its particle id: xc[p] = (x, y, z, j) (FP64,
+// the list is built in FP64 in either precision), so that the list build reads
+// one contiguous 32-byte entry per candidate instead of an index and then three
+// scattered coordinates.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void lj_sort_cells_kernel(const T* __restrict__ x, BoxArgs b,
+                                                               const int* __restrict__ start, int* order, int ncell,
+                                                               double4* __restrict__ xc) {
   const int lane = threadIdx.x % kWave;
   const int c = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
   if (c >= ncell) return;  // uniform over the wavefront
   const int lo = start[c], hi = start[c + 1], k = hi - lo;
+  auto put = [&](int p, int j) {
+    xc[p] = make_double4(wrap_box((double)x[(size_t)j * 3], b.L[0]), wrap_box((double)x[(size_t)j * 3 + 1], b.L[1]),
+                         wrap_box((double)x[(size_t)j * 3 + 2], b.L[2]), (double)j);
+  };
   if (k <= kWave) {
     const int v = lane < k ? order[lo + lane] : INT_MAX;
     int rank = 0;
     for (int q = 0; q < k; q++) rank += __shfl(v, q, kWave) < v ? 1 : 0;
-    if (lane < k) order[lo + rank] = v;
+    if (lane < k) put(lo + rank, v);
   } else if (lane == 0) {
     for (int a = lo + 1; a < hi; a++) {
       int v = order[a];
-      int b = a - 1;
-      while (b >= lo && order[b] > v) {
-        order[b + 1] = order[b];
-        b--;
+      int q = a - 1;
+      while (q >= lo && order[q] > v) {
+        order[q + 1] = order[q];
+        q--;
       }
-      order[b + 1] = v;
+      order[q + 1] = v;
     }
+    for (int p = lo; p < hi; p++) put(p, order[p]);
   }
 }
 
@@ -251,30 +271,10 @@ __device__ inline void pad_list(int i, int cnt, int maxn, int* __restrict__ nn, 
   for (int k = n; k % kListPad != 0; k++) nbr[nbr_at(i, k, maxn)] = i;
 }
 
-// A coordinate wrapped into [0, L), as the cell index takes it.
-__device__ __forceinline__ double wrap_box(double v, double L) { return v - L * floor(v / L); }
-
-// Positions in cell order, wrapped into the box, each with its particle id:
-// xc[p] = (x, y, z, j) for j = order[p] (FP64, the list is built in FP64 in
-// either precision), so that the list build reads one contiguous 32-byte
-// entry per candidate instead of an index and then three scattered
-// coordinates.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void lj_gather_cells_kernel(const T* __restrict__ x, int N, BoxArgs b,
-                                                                 const int* __restrict__ order,
-                                                                 double4* __restrict__ xc) {
-  const int p = blockIdx.x * kBlock + threadIdx.x;
-  if (p >= N) return;
-  const int j = order[p];
-  xc[p] = make_double4(wrap_box((double)x[(size_t)j * 3], b.L[0]), wrap_box((double)x[(size_t)j * 3 + 1], b.L[1]),
-                       wrap_box((double)x[(size_t)j * 3 + 2], b.L[2]), (double)j);
-}
-
 // Full Verlet list: neighbour k of particle i at nbr[nbr_at(i, k, maxn)].  The 27
 // cells around i's cell are visited in a fixed order and each cell's members
 // in particle-id order (lj_sort_cells_kernel), so the list -- and with it the
 // order in which the force pass sums pairs -- does not depend on scheduling.
-// Candidates are read U at a time, all loads issued before any is used.
 // With at least 3 cells of side >= rc + skin along each axis, the image of a
 // neighbour cell that lies within the list radius is the one its index wrap
 // implies, so each candidate needs no minimum-image rounding: i's wrapped
@@ -282,23 +282,32 @@ __global__ __launch_bounds__(kBlock) void lj_gather_cells_kernel(const T* __rest
 // list radius widened by 1e-12 of itself, so no pair the minimum-image test
 // keeps is lost to rounding; a pair kept in excess lies beyond the cutoff
 // (or at it, for skin 0) and the force pass, which tests the cutoff itself,
-// skips it.  Threads take the particles in cell order (thread p builds the
-// list of particle xc[p].w), so the lanes of a wavefront lie in a few cells
-// and read the same candidates instead of gathering from two dozen cells.
+// skips it.
+//
+// Q lanes per particle, each testing every Q-th candidate; a ballot gives the
+// kept ones consecutive entries in candidate order.  Cells that are neighbours
+// in z are neighbours in memory, so away from the z faces the three are one run.
+// Particles are taken in cell order (those of xc), so that a wavefront's
+// lanes read the same candidates.  Bound by the latency of the candidate loads
+// where there are few wavefronts and by the scattered writes of the list where
+// there are many (32,768 particles: 60 us, one lane per particle 150).
+template <int Q>
 __global__ __launch_bounds__(kBlock) void lj_build_list_kernel(int N, BoxArgs b, const int* __restrict__ cell,
                                                                const int* __restrict__ start,
                                                                const double4* __restrict__ xc, int maxn,
                                                                int* __restrict__ nn, int* __restrict__ nbr,
                                                                int* __restrict__ overflow) {
-  constexpr int U = 4;
-  const int pi = blockIdx.x * kBlock + threadIdx.x;
+  constexpr int U = 2;  // candidates requested per lane before any is used
+  const int pi = (blockIdx.x * kBlock + threadIdx.x) / Q, sub = threadIdx.x % Q;
   if (pi >= N) return;
+  const int first = (threadIdx.x % kWave) / Q * Q;  // this particle's lanes in the wavefront
   const double4 vi = xc[pi];
   const int i = (int)vi.w;
   const double xw0 = vi.x, xw1 = vi.y, xw2 = vi.z;
   const double rl2 = b.rlist2 * (1.0 + 1e-12);
   const int c = cell[i];
   const int cz = c % b.nc[2], cy = (c / b.nc[2]) % b.nc[1], cx = c / (b.nc[1] * b.nc[2]);
+  const bool inner = cz > 0 && cz < b.nc[2] - 1;
   int cnt = 0;
   for (int dx = -1; dx <= 1; dx++) {
     const int ux = cx + dx;
@@ -309,33 +318,34 @@ __global__ __launch_bounds__(kBlock) void lj_build_list_kernel(int N, BoxArgs b,
       const int uy = cy + dy;
       const int ay = uy < 0 ? uy + b.nc[1] : (uy >= b.nc[1] ? uy - b.nc[1] : uy);
       const double xi1 = uy < 0 ? xw1 + b.L[1] : (uy >= b.nc[1] ? xw1 - b.L[1] : xw1);
-      for (int dz = -1; dz <= 1; dz++) {
+      const int row = (ax * b.nc[1] + ay) * b.nc[2];
+      for (int dz = inner ? 1 : -1; dz <= 1; dz++) {
         const int uz = cz + dz;
         const int az = uz < 0 ? uz + b.nc[2] : (uz >= b.nc[2] ? uz - b.nc[2] : uz);
         const double xi2 = uz < 0 ? xw2 + b.L[2] : (uz >= b.nc[2] ? xw2 - b.L[2] : xw2);
-        const int cc = (ax * b.nc[1] + ay) * b.nc[2] + az;
-        const int p1 = start[cc + 1];
-        for (int p0 = start[cc]; p0 < p1; p0 += U) {
+        const int p1 = start[row + az + 1];
+        for (int p0 = start[row + (inner ? cz - 1 : az)]; p0 < p1; p0 += U * Q) {
           double4 v[U];
 #pragma unroll
-          for (int u = 0; u < U; u++) v[u] = xc[min(p0 + u, p1 - 1)];
+          for (int u = 0; u < U; u++) v[u] = xc[min(p0 + u * Q + sub, p1 - 1)];
 #pragma unroll
           for (int u = 0; u < U; u++) {
-            if (p0 + u >= p1) break;
             const int j = (int)v[u].w;
-            if (j == i) continue;
             const double r0 = xi0 - v[u].x, r1 = xi1 - v[u].y, r2 = xi2 - v[u].z;
-            if (r0 * r0 + r1 * r1 + r2 * r2 < rl2) {
-              if (cnt < maxn) nbr[nbr_at(i, cnt, maxn)] = j;
-              cnt++;
-            }
+            const bool keep = p0 + u * Q + sub < p1 && j != i && r0 * r0 + r1 * r1 + r2 * r2 < rl2;
+            const unsigned long long all = (__ballot(keep) >> first) & ((1ull << Q) - 1);
+            const int at = cnt + __popcll(all & ((1ull << sub) - 1));
+            if (keep && at < maxn) nbr[nbr_at(i, at, maxn)] = j;
+            cnt += __popcll(all);
           }
         }
       }
     }
   }
-  pad_list(i, cnt, maxn, nn, nbr);
-  if (cnt > maxn) atomicMax(overflow, cnt);
+  if (sub == 0) {
+    pad_list(i, cnt, maxn, nn, nbr);
+    if (cnt > maxn) atomicMax(overflow, cnt);
+  }
 }
 
 // Small boxes (fewer than 3 cells along a side): list by brute force.
@@ -402,7 +412,9 @@ struct Pos3 {
 // skin/2 since the list was built (reduction slot 1): when any has, the caller
 // rebuilds the list and evaluates again.  Blocks are spread over the XCDs in
 // contiguous ranges, so each L2 holds the positions of one spatially coherent
-// range of particles.  MODE bit 1 energy, bit 2 gradient.
+// range of particles.  MODE bit 1 energy, bit 2 gradient, bit 4 (with 2) FIRE's
+// sums.  Reduction rows: energy, moved, list overflow; or g.g, v.g, v.v, moved,
+// list overflow, largest |g_i|^2.
 //
 // Bound by VALU issue, about 40 instructions per entry: the reciprocal by
 // Newton's iteration, fused products, constant factors and the energy shift
@@ -415,10 +427,11 @@ template <typename T, int P, int U, int MODE>
 __global__ __launch_bounds__(kBlock) void lj_cut_kernel(const T* __restrict__ x, int N, BoxArgs b, T sig2, double eps,
                                                         double eshift, const int* __restrict__ nn,
                                                         const int* __restrict__ nbr, int maxn,
-                                                        const double* __restrict__ xbuild, T* __restrict__ g,
-                                                        RedScratch rs) {
+                                                        const double* __restrict__ xbuild,
+                                                        const int* __restrict__ overflow, const T* __restrict__ v,
+                                                        T* __restrict__ g, RedScratch rs) {
   static_assert(kListPad % (P * U) == 0, "whole chunks");
-  constexpr bool WE = MODE & 1, WG = MODE & 2;
+  constexpr bool WE = MODE & 1, WG = MODE & 2, WS = MODE & 4;
   const int tid = xcd_logical_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   const int i = tid / P, sub = tid % P;
   auto at = [&](unsigned j) {
@@ -426,6 +439,7 @@ __global__ __launch_bounds__(kBlock) void lj_cut_kernel(const T* __restrict__ x,
     return *reinterpret_cast<const Pos3<T>*>(reinterpret_cast<const char*>(x) + j * (unsigned)sizeof(Pos3<T>));
   };
   double ei = 0.0, moved = 0.0;
+  double gg = 0.0, vg = 0.0, vv = 0.0;
   if (i < N) {
     const Pos3<T> xi = at(i);
     const T L0 = (T)b.L[0], L1 = (T)b.L[1], L2 = (T)b.L[2];
@@ -482,12 +496,30 @@ __global__ __launch_bounds__(kBlock) void lj_cut_kernel(const T* __restrict__ x,
       if (WG) {
         const T f = (T)(-24 * eps);
 #pragma unroll
-        for (int k = 0; k < 3; k++) g[(size_t)i * 3 + k] = f * gi[k];
+        for (int k = 0; k < 3; k++) {
+          const T gk = f * gi[k];
+          g[(size_t)i * 3 + k] = gk;
+          if (WS) {
+            const double gd = (double)gk, vd = (double)v[(size_t)i * 3 + k];
+            gg += gd * gd;
+            vg += vd * gd;
+            vv += vd * vd;
+          }
+        }
       }
     }
   }
-  double acc[2] = {ei, moved};
-  grid_sum_store<2>(acc, rs);
+  const double over = blockIdx.x == 0 && threadIdx.x == 0 ? (double)*overflow : 0.0;
+  if constexpr (WS) {
+    __shared__ double lds[kBlock / kWave];
+    const double m = block_max(gg, lds);  // a lane holds one particle
+    if (threadIdx.x == 0) rs.partials[(size_t)5 * gridDim.x + blockIdx.x] = m;
+    double acc[5] = {gg, vg, vv, moved, over};
+    grid_sum_store<5>(acc, rs);
+  } else {
+    double acc[3] = {ei, moved, over};
+    grid_sum_store<3>(acc, rs);
+  }
 }
 
 template <typename T, int D>
@@ -650,7 +682,7 @@ int cut_blocks(int N) { return (int)(((size_t)N * cut_lanes(N) + kBlock - 1) / k
 
 template <typename T>
 void launch_cut_t(LjNd::Impl& I, const T* x, const T* d, T t, int N, double sigma, double eps, double eshift, int mode,
-                  T* g, minim_amd::RedScratch rs, hipStream_t s) {
+                  T* g, minim_amd::RedScratch rs, hipStream_t s, const T* v) {
   if (d) {
     const size_t n = 3 * (size_t)N;
     if (I.xtrial.bytes() < n * sizeof(double)) I.xtrial.reset(n * sizeof(double));
@@ -662,9 +694,11 @@ void launch_cut_t(LjNd::Impl& I, const T* x, const T* d, T t, int N, double sigm
     constexpr int P = decltype(lanes)::value, U = decltype(unroll)::value;
     auto run = [&](auto kernel) {
       kernel<<<cut_blocks(N), kBlock, 0, s>>>(x, N, I.box, (T)(sigma * sigma), eps, eshift, (const int*)I.nn.get(),
-                                              (const int*)I.nbr.get(), I.maxn, (const double*)I.xbuild.get(), g, rs);
+                                              (const int*)I.nbr.get(), I.maxn, (const double*)I.xbuild.get(),
+                                              (const int*)I.flag.get(), v, g, rs);
     };
-    if (mode == 1) run(minim_amd::lj_cut_kernel<T, P, U, 1>);
+    if (v) run(minim_amd::lj_cut_kernel<T, P, U, 6>);
+    else if (mode == 1) run(minim_amd::lj_cut_kernel<T, P, U, 1>);
     else if (mode == 2) run(minim_amd::lj_cut_kernel<T, P, U, 2>);
     else run(minim_amd::lj_cut_kernel<T, P, U, 3>);
   };
@@ -679,77 +713,92 @@ void launch_cut_t(LjNd::Impl& I, const T* x, const T* d, T t, int N, double sigm
 }
 
 void launch_cut(LjNd::Impl& I, int prec, const void* x, const void* d, double t, int N, double sigma, double epsilon,
-                double eshift, int mode, void* g, minim_amd::RedScratch rs, hipStream_t s) {
+                double eshift, int mode, void* g, minim_amd::RedScratch rs, hipStream_t s, const void* v = nullptr) {
   if (prec == FP64)
-    launch_cut_t(I, (const double*)x, (const double*)d, t, N, sigma, epsilon, eshift, mode, (double*)g, rs, s);
+    launch_cut_t(I, (const double*)x, (const double*)d, t, N, sigma, epsilon, eshift, mode, (double*)g, rs, s,
+                 (const double*)v);
   else
-    launch_cut_t(I, (const float*)x, (const float*)d, (float)t, N, sigma, epsilon, eshift, mode, (float*)g, rs, s);
+    launch_cut_t(I, (const float*)x, (const float*)d, (float)t, N, sigma, epsilon, eshift, mode, (float*)g, rs, s,
+                 (const float*)v);
   MINIM_HIP_CHECK(hipGetLastError());
 }
 
-// (Re)builds the Verlet list at the evaluated positions x (+ t*d).
+// Lanes per particle of the list build: 16 while one wavefront per four
+// particles leaves room, then 8 (whole rebuild with its evaluation at 4,096
+// particles: 207 us with one lane, 102 with 8, 88 with 16; at 32,768: 215, 127,
+// 131; at 262,144: 429, 385, 423).
+int build_lanes(int N) { return N <= 16384 ? 16 : 8; }
+
+// (Re)builds the Verlet list at the evaluated positions x (+ t*d), without
+// waiting for it: the force pass reports a list that outgrew its rows (its
+// reduction row after the moved particles), and grow_list makes room.
 void rebuild_list(LjNd::Impl& I, int prec, const void* x, const void* d, double t, int N, hipStream_t s) {
   const int nb = (N + kBlock - 1) / kBlock;
   // Build at the evaluated positions: materialise x + t*d when needed.
-  DeviceBuffer tmp;
   const void* xb = x;
   if (d) {
-    tmp.reset(3 * (size_t)N * minim_amd::prec_bytes(prec));
-    minim_amd::device_copy(tmp.get(), x, 3 * (size_t)N * minim_amd::prec_bytes(prec), s);
-    minim_amd::launch_axpy(prec, tmp.get(), d, t, 3 * (size_t)N, s);
-    xb = tmp.get();
+    if (I.xtrial.bytes() < 3 * sizeof(double) * (size_t)N) I.xtrial.reset(3 * sizeof(double) * (size_t)N);
+    minim_amd::device_copy(I.xtrial.get(), x, 3 * (size_t)N * minim_amd::prec_bytes(prec), s);
+    minim_amd::launch_axpy(prec, I.xtrial.get(), d, t, 3 * (size_t)N, s);
+    xb = I.xtrial.get();
   }
-  for (int attempt = 0; attempt < 2; attempt++) {
-    MINIM_HIP_CHECK(hipMemsetAsync(I.flag.get(), 0, sizeof(int), s));
+  int* count = (int*)I.count.get();
+  int* flag = (int*)I.flag.get();
+  auto go = [&](auto tag) {
+    using T = decltype(tag);
+    const T* xx = (const T*)xb;
+    double* xbuild = (double*)I.xbuild.get();
     if (I.cellMode) {
-      MINIM_HIP_CHECK(hipMemsetAsync(I.count.get(), 0, sizeof(int) * I.ncell, s));
       constexpr int kCellsPerBlock = kBlock / minim_amd::kWave;  // one wavefront per cell
       const int nbc = (I.ncell + kCellsPerBlock - 1) / kCellsPerBlock;
-      if (prec == FP64)
-        minim_amd::lj_cell_index_kernel<double><<<nb, kBlock, 0, s>>>((const double*)xb, N, I.box, (int*)I.cell.get(),
-                                                                      (int*)I.count.get(), (double*)I.xbuild.get());
-      else
-        minim_amd::lj_cell_index_kernel<float><<<nb, kBlock, 0, s>>>((const float*)xb, N, I.box, (int*)I.cell.get(),
-                                                                     (int*)I.count.get(), (double*)I.xbuild.get());
-      minim_amd::lj_scan_kernel<<<1, kBlock, 0, s>>>((const int*)I.count.get(), (int*)I.start.get(),
-                                                     (int*)I.cursor.get(), I.ncell);
-      minim_amd::lj_fill_kernel<<<nb, kBlock, 0, s>>>((const int*)I.cell.get(), N, (const int*)I.start.get(),
-                                                      (int*)I.cursor.get(), (int*)I.order.get());
-      minim_amd::lj_sort_cells_kernel<<<nbc, kBlock, 0, s>>>((const int*)I.start.get(), (int*)I.order.get(), I.ncell);
       if (I.xcell.bytes() < sizeof(double4) * (size_t)N) I.xcell.reset(sizeof(double4) * (size_t)N);
       double4* xc = static_cast<double4*>(I.xcell.get());
-      if (prec == FP64) {
-        minim_amd::lj_gather_cells_kernel<double><<<nb, kBlock, 0, s>>>((const double*)xb, N, I.box,
-                                                                         (const int*)I.order.get(), xc);
-      } else {
-        minim_amd::lj_gather_cells_kernel<float><<<nb, kBlock, 0, s>>>((const float*)xb, N, I.box,
-                                                                        (const int*)I.order.get(), xc);
-      }
-      minim_amd::lj_build_list_kernel<<<nb, kBlock, 0, s>>>(N, I.box, (const int*)I.cell.get(),
-                                                             (const int*)I.start.get(), xc, I.maxn, (int*)I.nn.get(),
-                                                             (int*)I.nbr.get(), (int*)I.flag.get());
+      minim_amd::lj_clear_kernel<<<minim_amd::grid_blocks(I.ncell), kBlock, 0, s>>>(count, I.ncell, flag);
+      minim_amd::lj_cell_index_kernel<T><<<nb, kBlock, 0, s>>>(xx, N, I.box, (int*)I.cell.get(), count, xbuild);
+      minim_amd::lj_scan_kernel<<<1, kBlock, 0, s>>>(count, (int*)I.start.get(), (int*)I.cursor.get(), I.ncell);
+      minim_amd::lj_fill_kernel<<<nb, kBlock, 0, s>>>((const int*)I.cell.get(), N, (const int*)I.start.get(),
+                                                      (int*)I.cursor.get(), (int*)I.order.get());
+      minim_amd::lj_sort_cells_kernel<T><<<nbc, kBlock, 0, s>>>(xx, I.box, (const int*)I.start.get(),
+                                                                (int*)I.order.get(), I.ncell, xc);
+      auto build = [&](auto kernel, int lanes) {
+        kernel<<<(int)(((size_t)N * lanes + kBlock - 1) / kBlock), kBlock, 0, s>>>(
+            N, I.box, (const int*)I.cell.get(), (const int*)I.start.get(), xc, I.maxn, (int*)I.nn.get(),
+            (int*)I.nbr.get(), flag);
+      };
+      if (build_lanes(N) == 16) build(minim_amd::lj_build_list_kernel<16>, 16);
+      else build(minim_amd::lj_build_list_kernel<8>, 8);
     } else {
-      if (prec == FP64)
-        minim_amd::lj_build_list_brute_kernel<double><<<nb, kBlock, 0, s>>>(
-            (const double*)xb, N, I.box, I.maxn, (int*)I.nn.get(), (int*)I.nbr.get(), (int*)I.flag.get(),
-            (double*)I.xbuild.get());
-      else
-        minim_amd::lj_build_list_brute_kernel<float><<<nb, kBlock, 0, s>>>(
-            (const float*)xb, N, I.box, I.maxn, (int*)I.nn.get(), (int*)I.nbr.get(), (int*)I.flag.get(),
-            (double*)I.xbuild.get());
+      minim_amd::lj_clear_kernel<<<1, kBlock, 0, s>>>(count, 0, flag);
+      minim_amd::lj_build_list_brute_kernel<T><<<nb, kBlock, 0, s>>>(xx, N, I.box, I.maxn, (int*)I.nn.get(),
+                                                                     (int*)I.nbr.get(), flag, xbuild);
     }
     MINIM_HIP_CHECK(hipGetLastError());
-    int over = 0;
-    MINIM_HIP_CHECK(hipMemcpyAsync(&over, I.flag.get(), sizeof(int), hipMemcpyDeviceToHost, s));
-    MINIM_HIP_CHECK(hipStreamSynchronize(s));
-    if (over == 0) break;
-    if (attempt == 1) throw std::runtime_error("LjNd: neighbour list overflow");
-    I.maxn = (over + 2 * minim_amd::kListPad - 1) / minim_amd::kListPad * minim_amd::kListPad;
-    I.nbr.reset(sizeof(int) * minim_amd::nbr_elems(N, I.maxn));
-  }
+  };
+  if (prec == FP64) go(0.0);
+  else go(0.0f);
   I.built = true;
   I.builds++;
 }
+
+// Rows for lists of up to longest entries; the list is built again after.
+void grow_list(LjNd::Impl& I, int N, int longest) {
+  I.maxn = (longest + 2 * minim_amd::kListPad - 1) / minim_amd::kListPad * minim_amd::kListPad;
+  I.nbr.reset(sizeof(int) * minim_amd::nbr_elems(N, I.maxn));
+  I.builds--;
+}
+
+// rebuild_list, waiting until it is known that the lists fit.
+void rebuild_list_checked(LjNd::Impl& I, int prec, const void* x, int N, hipStream_t s) {
+  for (;;) {
+    rebuild_list(I, prec, x, nullptr, 0.0, N, s);
+    int over = 0;
+    MINIM_HIP_CHECK(hipMemcpyAsync(&over, I.flag.get(), sizeof(int), hipMemcpyDeviceToHost, s));
+    MINIM_HIP_CHECK(hipStreamSynchronize(s));
+    if (over == 0) return;
+    grow_list(I, N, over);
+  }
+}
+
 }  // namespace
 
 // Energy (result slot 0, and eDev when given) and gradient, without waiting for
@@ -770,17 +819,16 @@ void LjNd::launch(int prec, const void* x, const void* d, double t, bool wantE, 
       throw std::invalid_argument("LjNd: too many particles for one launch");
     const double src6 = std::pow(sigma / cutoff, 6);
     const double eshift = 4 * epsilon * (src6 * src6 - src6);
-    auto launch_force = [&]() {
+    bool build = !I.built;
+    for (;;) {
+      if (build) rebuild_list(I, prec, x, d, t, N, s);
       launch_cut(I, prec, x, d, t, N, sigma, epsilon, eshift, mode, g, ws.rs(), s);
-      minim_amd::launch_finalize(ws.rs(), 2, cut_blocks(N), s, 0, wantE ? eDev : nullptr);
-    };
-    if (!I.built) rebuild_list(I, prec, x, d, t, N, s);
-    launch_force();
-    double r[2];
-    ws.fetch(s, 2, r);  // energy, particles moved more than skin/2 since the list was built
-    if (r[1] > 0) {
-      rebuild_list(I, prec, x, d, t, N, s);
-      launch_force();
+      minim_amd::launch_finalize(ws.rs(), 3, cut_blocks(N), s, 0, wantE ? eDev : nullptr);
+      double r[3];  // energy, particles moved more than skin/2 since the list was built, its overflow
+      ws.fetch(s, 3, r);
+      if (r[1] == 0 && r[2] == 0) break;
+      if (r[2] > 0) grow_list(I, N, (int)r[2]);
+      build = true;
     }
   }
   if (g) constrainDevice(prec, x, g, (size_t)N * nDim, stream);
@@ -812,11 +860,11 @@ int LjNd::gradientDeferred(int prec, const void* x, void* g, void* stream) const
   auto& ws = minim_amd::Workspace::current();
   Impl& I = *impl_;
   const int N = nParticle;
-  if (!I.built) rebuild_list(I, prec, x, nullptr, 0.0, N, s);
+  if (!I.built) rebuild_list_checked(I, prec, x, N, s);
   const double src6 = std::pow(sigma / cutoff, 6);
   const double eshift = 4 * epsilon * (src6 * src6 - src6);
   launch_cut(I, prec, x, nullptr, 0.0, N, sigma, epsilon, eshift, 2, g, ws.rs(), s);
-  minim_amd::launch_finalize(ws.rs(), 2, cut_blocks(N), s, 1, ws.rs().mirror + minim_amd::kDeferSlot);
+  minim_amd::launch_finalize(ws.rs(), 3, cut_blocks(N), s, 1, ws.rs().mirror + minim_amd::kDeferSlot);
   constrainDevice(prec, x, g, (size_t)N * nDim, stream);
   return minim_amd::kDeferSlot;
 }
@@ -827,12 +875,36 @@ void LjNd::redoGradient(int prec, const void* x, void* g, void* stream) const {
   hipStream_t s = static_cast<hipStream_t>(stream);
   auto& ws = minim_amd::Workspace::current();
   const int N = nParticle;
-  rebuild_list(*impl_, prec, x, nullptr, 0.0, N, s);
+  rebuild_list_checked(*impl_, prec, x, N, s);
   const double src6 = std::pow(sigma / cutoff, 6);
   const double eshift = 4 * epsilon * (src6 * src6 - src6);
   launch_cut(*impl_, prec, x, nullptr, 0.0, N, sigma, epsilon, eshift, 2, g, ws.rs(), s);
-  minim_amd::launch_finalize(ws.rs(), 2, cut_blocks(N), s);
+  minim_amd::launch_finalize(ws.rs(), 3, cut_blocks(N), s);
   constrainDevice(prec, x, g, (size_t)N * nDim, stream);
+}
+
+// Cutoff mode without constraints: the force pass has each particle's force in
+// registers, so that FIRE's dots and largest force need no pass of their own.
+bool LjNd::fusesFire(int dim) const {
+  return cutoff > 0 && constraints.empty() && (dim == 0 || dim == 3) &&
+         cut_blocks(nParticle) <= minim_amd::kMaxRedBlocks;
+}
+
+void LjNd::fireGradient(int prec, const void* x, void* g, const void* v, int, bool again, void* stream) const {
+  if (!impl_) throw std::runtime_error("LjNd: not initialised (construct a State first).");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  auto& ws = minim_amd::Workspace::current();
+  Impl& I = *impl_;
+  const int N = nParticle;
+  if (again) {
+    // a list that was built for the last evaluation may have outgrown its rows
+    double r[5];
+    ws.fetch(s, 5, r);
+    if (r[4] > 0) grow_list(I, N, (int)r[4]);
+  }
+  if (again || !I.built) rebuild_list(I, prec, x, nullptr, 0.0, N, s);
+  launch_cut(I, prec, x, nullptr, 0.0, N, sigma, epsilon, 0.0, 2, g, ws.rs(), s, v);
+  minim_amd::launch_finalize(ws.rs(), 6, cut_blocks(N), s, -1, nullptr, 5);
 }
 
 // Average duration (ms) of reps launches of the force kernel (cutoff mode:
@@ -860,7 +932,7 @@ double LjNd::timeKernel(int prec, const void* x, bool wantE, void* g, int reps, 
       minim_amd::launch_allpairs<float>(nDim, x, nullptr, 0.0, N, sigma, epsilon, mode, g, ws.rs(), s);
     }
   };
-  if (cutoff > 0 && !impl_->built) rebuild_list(*impl_, prec, x, nullptr, 0.0, N, s);
+  if (cutoff > 0 && !impl_->built) rebuild_list_checked(*impl_, prec, x, N, s);
   launch();
   hipEvent_t e0, e1;
   MINIM_HIP_CHECK(hipEventCreate(&e0));

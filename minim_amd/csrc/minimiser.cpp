@@ -886,6 +886,28 @@ void Fire::iteration(State& state) {
     I.a = _aStart;
     I.dt = I.dt * _fDec;
   }
+  if (linesearch != "backtracking" && state.pot->fusesFire(_maxForceDim)) {
+    minim_amd::launch_fire_move(I.prec, mode, I.v.data(), I.g.data(), state.deviceCoords(), f1, f2, I.dt, I.n, s);
+    state.invalidateHost();
+    I.ec.valid = false;
+    stats.nGradient++;
+    double q[6];
+    bool again = false;
+    do {
+      state.pot->fireGradient(I.prec, state.deviceCoords(), I.g.data(), I.v.data(), _maxForceDim, again,
+                              state.stream());
+      ws.fetch(s, 6, q);
+      again = q[3] > 0 || q[4] > 0;
+    } while (again);
+    I.gNorm = std::sqrt(q[0]);
+    I.vg = q[1];
+    I.vv = q[2];
+    I.haveDots = true;
+    if (_maxForceDim > 0) I.gMax = q[5];
+    if (I.prec == FP32) stats.iterFP32++;
+    else stats.iterFP64++;
+    return;
+  }
   minim_amd::launch_fire_update(I.prec, mode, I.v.data(), I.g.data(), I.step.data(), f1, f2, I.dt, I.n, s);
   state.pot->constrainDevice(I.prec, I.prec == state.precision() ? state.deviceCoords() : nullptr, I.step.data(),
                              I.n, state.stream());

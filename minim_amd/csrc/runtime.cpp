@@ -37,13 +37,18 @@ namespace {
 // One block per reduced value: partials of value k are contiguous.
 __global__ __launch_bounds__(kBlock) void finalize_kernel(const double* __restrict__ partials, int nb,
                                                           double* __restrict__ result, double* mirror, int dupK,
-                                                          double* dupDst) {
+                                                          double* dupDst, int maxK) {
   __shared__ double lds[kBlock / kWave];
   const int k = blockIdx.x;
   const double* p = partials + (size_t)k * nb;
   double v[1] = {0.0};
-  for (int b = threadIdx.x; b < nb; b += kBlock) v[0] += p[b];
-  block_sum<1>(v, lds);
+  if (k == maxK) {
+    for (int b = threadIdx.x; b < nb; b += kBlock) v[0] = nan_max(v[0], p[b]);
+    v[0] = sqrt(block_max(v[0], lds));
+  } else {
+    for (int b = threadIdx.x; b < nb; b += kBlock) v[0] += p[b];
+    block_sum<1>(v, lds);
+  }
   if (threadIdx.x == 0) {
     result[k] = v[0];
     if (mirror) mirror[k] = v[0];
@@ -52,11 +57,11 @@ __global__ __launch_bounds__(kBlock) void finalize_kernel(const double* __restri
 }
 }  // namespace
 
-void launch_finalize(RedScratch rs, int K, int nb, hipStream_t s, int dupK, double* dupDst) {
+void launch_finalize(RedScratch rs, int K, int nb, hipStream_t s, int dupK, double* dupDst, int maxK) {
   if (K < 1 || K > kMaxDots || nb < 1 || nb > kMaxRedBlocks)
     throw std::invalid_argument("reduction shape out of range");
   if (!dupDst) dupK = -1;
-  finalize_kernel<<<K, kBlock, 0, s>>>(rs.partials, nb, rs.result, rs.mirror, dupK, dupDst);
+  finalize_kernel<<<K, kBlock, 0, s>>>(rs.partials, nb, rs.result, rs.mirror, dupK, dupDst, maxK);
   MINIM_HIP_CHECK(hipGetLastError());
 }
 

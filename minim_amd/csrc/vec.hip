@@ -452,8 +452,18 @@ __global__ __launch_bounds__(kBlock) void fire_kernel(int mode, T* __restrict__ 
   }
 }
 
-// NaN-propagating maximum
-__device__ inline double nan_max(double a, double b) { return (b > a || b != b) ? b : a; }
+// fire_kernel and x += step in one pass, the step not kept.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void fire_move_kernel(int mode, T* __restrict__ v, const T* __restrict__ g,
+                                                           T* __restrict__ x, T f1, T f2, T dt, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
+    const T t2 = f2 * g[i];
+    const T nv = mode == 1 ? f1 * v[i] - t2 : t2;
+    v[i] = nv;
+    const T step = dt * nv;
+    x[i] = x[i] + step;
+  }
+}
 
 template <typename T>
 __global__ __launch_bounds__(kBlock) void group_norm_max_kernel(const T* __restrict__ v, size_t ngroup, int dim,
@@ -467,29 +477,9 @@ __global__ __launch_bounds__(kBlock) void group_norm_max_kernel(const T* __restr
     }
     m = nan_max(m, s);
   }
-  for (int off = kWave / 2; off > 0; off >>= 1) m = nan_max(m, __shfl_xor(m, off, kWave));
   __shared__ double lds[kBlock / kWave];
-  if (threadIdx.x % kWave == 0) lds[threadIdx.x / kWave] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kBlock / kWave; w++) m = nan_max(m, lds[w]);
-    partial[blockIdx.x] = m;
-  }
-}
-
-__global__ __launch_bounds__(kBlock) void max_sqrt_finalize_kernel(const double* __restrict__ partial, int nb,
-                                                                   double* __restrict__ result, double* mirror) {
-  double m = 0.0;
-  for (int b = threadIdx.x; b < nb; b += kBlock) m = nan_max(m, partial[b]);
-  for (int off = kWave / 2; off > 0; off >>= 1) m = nan_max(m, __shfl_xor(m, off, kWave));
-  __shared__ double lds[kBlock / kWave];
-  if (threadIdx.x % kWave == 0) lds[threadIdx.x / kWave] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kBlock / kWave; w++) m = nan_max(m, lds[w]);
-    result[0] = sqrt(m);
-    if (mirror) mirror[0] = sqrt(m);
-  }
+  m = block_max(m, lds);
+  if (threadIdx.x == 0) partial[blockIdx.x] = m;
 }
 
 int bucket(int k) {
@@ -652,8 +642,7 @@ void launch_group_norm_max(int prec, const void* v, size_t n, int dim, RedScratc
   if (prec == F64) group_norm_max_kernel<double><<<nb, kBlock, 0, s>>>((const double*)v, ngroup, dim, rs.partials);
   else group_norm_max_kernel<float><<<nb, kBlock, 0, s>>>((const float*)v, ngroup, dim, rs.partials);
   MINIM_HIP_CHECK(hipGetLastError());
-  max_sqrt_finalize_kernel<<<1, kBlock, 0, s>>>(rs.partials, nb, rs.result, rs.mirror);
-  MINIM_HIP_CHECK(hipGetLastError());
+  launch_finalize(rs, 1, nb, s, -1, nullptr, 0);
 }
 
 void launch_fire_update(int prec, int mode, void* v, const void* g, void* step, double f1, double f2,
@@ -664,6 +653,17 @@ void launch_fire_update(int prec, int mode, void* v, const void* g, void* step, 
   else
     fire_kernel<float><<<nb, kBlock, 0, s>>>(mode, (float*)v, (const float*)g, (float*)step, (float)f1, (float)f2,
                                              (float)dt, n);
+  MINIM_HIP_CHECK(hipGetLastError());
+}
+
+void launch_fire_move(int prec, int mode, void* v, const void* g, void* x, double f1, double f2, double dt, size_t n,
+                      hipStream_t s) {
+  const int nb = grid_blocks(n, 1, 4096);
+  if (prec == F64)
+    fire_move_kernel<double><<<nb, kBlock, 0, s>>>(mode, (double*)v, (const double*)g, (double*)x, f1, f2, dt, n);
+  else
+    fire_move_kernel<float><<<nb, kBlock, 0, s>>>(mode, (float*)v, (const float*)g, (float*)x, (float)f1, (float)f2,
+                                                  (float)dt, n);
   MINIM_HIP_CHECK(hipGetLastError());
 }
 

@@ -77,6 +77,10 @@ void launch_convert(int prec_dst, void* dst, int prec_src, const void* src, size
 void launch_fire_update(int prec, int mode, void* v, const void* g, void* step, double f1, double f2,
                         double dt, size_t n, hipStream_t s);
 
+// The same velocity update with x = x + dt*v, the step not stored.
+void launch_fire_move(int prec, int mode, void* v, const void* g, void* x, double f1, double f2, double dt, size_t n,
+                      hipStream_t s);
+
 // x = x + step (element-wise); used where the step vector is explicit
 void launch_add(int prec, void* x, const void* step, size_t n, hipStream_t s);
 

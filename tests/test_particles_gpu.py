@@ -540,3 +540,63 @@ def test_bah_mixed_evaluation_and_minimisation(gpu):
     # of 1e-6 its energy is pinned only to about 1e-5 of the initial energy,
     # and the two schedules stop at different points of that valley.
     assert abs(out["mixed"] - out["fp64"]) <= 1e-5 * abs(o.energy(x0))
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("side", [7, 20, 25, 26, 33, 41])
+def test_lj_cutoff_lanes_vs_lattice_sum(gpu, side, prec):
+    """Cutoff mode at particle counts on either side of each choice of lanes
+    per particle, force pass (16, 8, 4, 2 and 1) and list build (16 and 8):
+    energy and gradient of a jittered lattice against the FP64 sum over lattice
+    shifts.  FP32: a pair keeps an absolute error of one ulp of the box per
+    component, and the pair force's relative change is at most 14 times the
+    distance's (r > 0.75): 14 * 2^-23 * side / 0.75 per pair, a few pairs of
+    which dominate a particle."""
+    import torch
+
+    m = gpu
+    print("case lj lanes", side, prec, flush=True)
+    a, rc = 0.85 ** (-1 / 3), 2.5
+    k = np.arange(side) * a
+    x = np.stack(np.meshgrid(k, k, k, indexing="ij"), -1).reshape(-1, 3)
+    x = r32((x + np.random.default_rng(side).uniform(-0.1, 0.1, x.shape)).reshape(-1))
+    p = torch.tensor(x, device="cuda").reshape(side, side, side, 3)
+    go, eo, L = torch.zeros_like(p), 0.0, side * a
+    # a pair within the cutoff is at most three lattice steps apart along each axis
+    for s in np.stack(np.meshgrid(*[range(-3, 4)] * 3), -1).reshape(-1, 3):
+        if not s.any():
+            continue
+        dx = p - torch.roll(p, s.tolist(), (0, 1, 2))
+        dx = dx - L * torch.round(dx / L)
+        r2 = (dx * dx).sum(-1)
+        near = r2 < rc * rc
+        i6 = torch.where(near, r2, 1.0) ** -3
+        eo += 0.5 * float(torch.where(near, 4 * (i6 * i6 - i6) - 4 * (rc ** -12 - rc ** -6), 0.0).sum())
+        go += dx * torch.where(near, -24 * (2 * i6 * i6 - i6) / r2, 0.0)[..., None]
+    xd = torch.tensor(x, dtype=torch.float64 if prec == "fp64" else torch.float32, device="cuda")
+    h = m.Lj3d().setCutoff(rc, [L] * 3, 0.3).handle(x)
+    g = torch.empty_like(xd)
+    e = m.potential_eval(h, prec, xd.data_ptr(), xd.numel(), g_ptr=g.data_ptr())
+    tol = 1e-12 if prec == "fp64" else 14 * 2.0 ** -23 * side / 0.75
+    assert abs(e - eo) <= tol * abs(eo)
+    assert float((g.double() - go.reshape(-1)).norm()) <= tol * float(go.norm())
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_lj_list_longer_than_its_rows(gpu, prec):
+    """A system so dense that a list outgrows its rows at first (343 particles
+    in a box of 6 sigma, more than 128 neighbours): the list is built again with
+    longer rows and the evaluation repeated, in cell mode off (fewer than three
+    cells a side) and on (a dense corner of a larger box)."""
+    m = gpu
+    rng = np.random.default_rng(5)
+    for L, spread in ((6.0, 6.0), (12.0, 6.0)):
+        k = np.arange(7)
+        x = np.stack(np.meshgrid(k, k, k, indexing="ij"), -1).reshape(-1, 3) * (spread / 7)
+        x = r32((x + rng.uniform(-0.02, 0.02, x.shape)).reshape(-1))
+        o = OracleLJPBC(len(x) // 3, L, 2.5)
+        s = m.State(m.Lj3d().setCutoff(2.5, [L] * 3, 0.3), x, prec)
+        e, g = s.energyGradient(x)
+        tol = 1e-12 if prec == "fp64" else 1e-4
+        assert abs(e - o.energy(x)) <= tol * abs(o.energy(x)) + tol
+        assert rel_err(g, o.gradient(x)) <= tol
