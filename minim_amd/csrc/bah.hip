@@ -754,6 +754,7 @@ void launch_bah(const BarAndHinge::Dev& dv, int prec, int pv, const void* x, con
                 bool wantE, void* g, bool mask, minim_amd::RedScratch rs, hipStream_t s, double* eDev = nullptr,
                 int parts = minim_amd::kAllParts) {
   const auto& a = dv.args;
+  rs = rs.only(0, eDev);
   if (pv != prec && !(prec == FP64 && pv == FP32))
     throw std::invalid_argument("BarAndHinge: FP32 coordinates with FP64 vectors are not supported.");
   // the same blocks with and without the gradient: the energy is the same bit for bit
@@ -773,7 +774,7 @@ void launch_bah(const BarAndHinge::Dev& dv, int prec, int pv, const void* x, con
   if (prec == FP64 && pv == FP64) go(0.0, 0.0);
   else if (prec == FP64) go(0.0, 0.0f);
   else go(0.0f, 0.0f);
-  if (wantE) minim_amd::launch_finalize(rs, 1, nb, s, 0, eDev);
+  if (wantE) minim_amd::launch_finalize(rs, 1, nb, s);
 }
 }  // namespace
 

@@ -23,6 +23,7 @@ constexpr int kBlock = 256;          // threads per block (4 wavefronts of 64)
 constexpr int kWave = 64;
 constexpr int kMaxRedBlocks = 8192;  // upper bound on blocks of any reducing launch
 constexpr int kMaxDots = 96;         // upper bound on values reduced by one launch
+constexpr int kSelfBlocks = kWave;    // largest launch that finishes its own reduction
 // Result slot of a deferred validity flag (Potential::gradientDeferred): the
 // last one, written by that launch and read by the caller's next fetch.
 constexpr int kDeferSlot = kMaxDots - 1;
@@ -78,25 +79,98 @@ __device__ inline void block_sum(double (&v)[K], double* lds) {
 // Scratch for cross-block reductions: K rows of per-block partials and the
 // final result (device).
 //
-// Two stages, no fences and no atomics: each block of the producing kernel
-// writes its K partial sums (grid_sum_store), then a small kernel with one
-// block per value sums the partials in block order (launch_finalize).  A
-// "last block finishes the sum" scheme would need a device-scope fence in
-// every block, which on CDNA3/4 writes back the whole L2 each time.
+// Many blocks: two stages, no fences and no atomics.  Each block of the
+// producing kernel writes its K partial sums (grid_sum_store), then a small
+// kernel with one block per value sums the partials in block order
+// (launch_finalize).  A "last block finishes the sum" scheme with a device-scope
+// fence in every block writes back the whole L2 each time on CDNA3/4.
+//
+// Kernels compiled with grid_sum_store<K, true>, for up to kSelfBlocks blocks: the
+// last block to arrive does finish the sum, in the same order, in place of
+// launch_finalize.  It needs no fence, because the partials themselves bypass the
+// L2 (relaxed device-scope atomics): a block waits for its own partials to be
+// stored, then counts itself.  It saves a launch (128 x 128 field, 16 blocks:
+// energy and gradient 9.4 -> 7.2 us), but the blocks are counted one after the
+// other (at 512 blocks an evaluation took 1.5 to 2 us longer than with the second
+// launch), and the 23 sums of a Gram pass take as long as the launch they save.
 struct RedScratch {
   double* partials;  // [kMaxDots][kMaxRedBlocks], value k of block b at k * gridDim + b
   double* result;    // [kMaxDots]
-  double* mirror = nullptr;  // the same values in pinned host memory, for Workspace::fetch
+  double* mirror = nullptr;   // the same values in pinned host memory, for Workspace::fetch
+  unsigned* ticket = nullptr; // arrivals of this launch (zero before and after), or null: two stages only
+  double* few = nullptr;      // its partials, [kMaxDots][kSelfBlocks]
+  double* copy = nullptr;     // value copyK goes there too (a caller's device slot)
+  int copyK = -1;
   // The same scratch with results from slot k on.
-  RedScratch from(int k) const { return {partials, result + k, mirror ? mirror + k : nullptr}; }
+  RedScratch from(int k) const {
+    RedScratch r = *this;
+    r.result += k;
+    if (mirror) r.mirror += k;
+    return r;
+  }
+  // ... with value k also written to dst (none if null).
+  RedScratch copying(int k, double* dst) const {
+    RedScratch r = *this;
+    r.copy = dst;
+    r.copyK = dst ? k : -1;
+    return r;
+  }
+  // ... to dst alone: nothing fetches it (a store to host memory holds the end of
+  // the kernel up by about 0.5 us).
+  RedScratch only(int k, double* dst) const {
+    RedScratch r = copying(k, dst);
+    if (dst) r.mirror = nullptr;
+    return r;
+  }
 };
 
-// All threads of the (1-D) grid must call this; v is each thread's contribution.
+// The last block's part: v (thread 0) are this block's partial sums.
 template <int K>
+__device__ inline void finish_in_kernel(double (&v)[K], const RedScratch& rs) {
+  __shared__ bool last;
+  const int nb = gridDim.x;
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 0; k < K; k++)
+      __hip_atomic_store(&rs.few[(size_t)k * nb + blockIdx.x], v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(rs.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)nb - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  // one lane per partial, as finalize_kernel; each wave takes every fourth value
+  constexpr int W = kBlock / kWave, J = (K + W - 1) / W;
+  const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
+  double s[J];
+#pragma unroll
+  for (int j = 0; j < J; j++) {
+    const int k = wid + j * W;
+    s[j] = k < K && lane < nb ? __hip_atomic_load(&rs.few[(size_t)k * nb + lane], __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT)
+                              : 0.0;
+  }
+  wave_sum(s);
+  if (lane == 0) {
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+      const int k = wid + j * W;
+      if (k >= K) break;
+      rs.result[k] = s[j];
+      if (rs.mirror) rs.mirror[k] = s[j];
+      if (k == rs.copyK) *rs.copy = s[j];
+    }
+  }
+  if (threadIdx.x == 0) __hip_atomic_store(rs.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// All threads of the (1-D) grid must call this; v is each thread's contribution.
+template <int K, bool SELF = false>
 __device__ inline void grid_sum_store(double (&v)[K], RedScratch rs) {
   __shared__ double lds[(kBlock / kWave) * (K > 0 ? K : 1)];
   block_sum<K>(v, lds);
-  if (threadIdx.x == 0) {
+  if constexpr (SELF) {
+    finish_in_kernel(v, rs);
+  } else if (threadIdx.x == 0) {
     const size_t nb = gridDim.x;
 #pragma unroll
     for (int k = 0; k < K; k++) rs.partials[(size_t)k * nb + blockIdx.x] = v[k];
@@ -104,11 +178,9 @@ __device__ inline void grid_sum_store(double (&v)[K], RedScratch rs) {
 }
 
 // Second stage: result[k] = sum over the nb partials of value k, in a fixed
-// order (stream-ordered after the producing kernel).  With dupDst, value dupK
-// is also written there (a caller's device slot: no copy launch after).  Value
-// maxK, if any, is the square root of the largest partial instead (a NaN wins).
-void launch_finalize(RedScratch rs, int K, int nb, hipStream_t s, int dupK = -1, double* dupDst = nullptr,
-                     int maxK = -1);
+// order (stream-ordered after the producing kernel).  Value maxK, if any, is the
+// square root of the largest partial instead (a NaN wins).
+void launch_finalize(RedScratch rs, int K, int nb, hipStream_t s, int maxK = -1);
 
 // NaN-propagating maximum
 __device__ inline double nan_max(double a, double b) { return (b > a || b != b) ? b : a; }

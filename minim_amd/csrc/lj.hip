@@ -550,6 +550,7 @@ void launch_allpairs(int D, const void* x, const void* d, double t, int N, doubl
   const T* dd = (const T*)d;
   T* gg = (T*)g;
   const T sig6 = (T)std::pow(sigma, 6), tt = (T)t, ee = (T)eps;
+  rs = rs.only(0, (mode & 1) ? eDev : nullptr);
   int nb = 0;
   switch (D) {
     case 1: nb = launch_allpairs_d<T, 1>(xx, dd, tt, N, sig6, ee, mode, gg, rs, s); break;
@@ -559,7 +560,7 @@ void launch_allpairs(int D, const void* x, const void* d, double t, int N, doubl
     default: throw std::invalid_argument("LjNd: nDim must be 1..4 on the device path");
   }
   MINIM_HIP_CHECK(hipGetLastError());
-  launch_finalize(rs, 1, nb, s, 0, (mode & 1) ? eDev : nullptr);
+  launch_finalize(rs, 1, nb, s);
 }
 
 }  // namespace
@@ -822,8 +823,9 @@ void LjNd::launch(int prec, const void* x, const void* d, double t, bool wantE, 
     bool build = !I.built;
     for (;;) {
       if (build) rebuild_list(I, prec, x, d, t, N, s);
-      launch_cut(I, prec, x, d, t, N, sigma, epsilon, eshift, mode, g, ws.rs(), s);
-      minim_amd::launch_finalize(ws.rs(), 3, cut_blocks(N), s, 0, wantE ? eDev : nullptr);
+      const minim_amd::RedScratch rs = ws.rs().copying(0, wantE ? eDev : nullptr);
+      launch_cut(I, prec, x, d, t, N, sigma, epsilon, eshift, mode, g, rs, s);
+      minim_amd::launch_finalize(rs, 3, cut_blocks(N), s);
       double r[3];  // energy, particles moved more than skin/2 since the list was built, its overflow
       ws.fetch(s, 3, r);
       if (r[1] == 0 && r[2] == 0) break;
@@ -863,8 +865,10 @@ int LjNd::gradientDeferred(int prec, const void* x, void* g, void* stream) const
   if (!I.built) rebuild_list_checked(I, prec, x, N, s);
   const double src6 = std::pow(sigma / cutoff, 6);
   const double eshift = 4 * epsilon * (src6 * src6 - src6);
-  launch_cut(I, prec, x, nullptr, 0.0, N, sigma, epsilon, eshift, 2, g, ws.rs(), s);
-  minim_amd::launch_finalize(ws.rs(), 3, cut_blocks(N), s, 1, ws.rs().mirror + minim_amd::kDeferSlot);
+  minim_amd::RedScratch rs = ws.rs();
+  rs = rs.copying(1, rs.mirror + minim_amd::kDeferSlot);
+  launch_cut(I, prec, x, nullptr, 0.0, N, sigma, epsilon, eshift, 2, g, rs, s);
+  minim_amd::launch_finalize(rs, 3, cut_blocks(N), s);
   constrainDevice(prec, x, g, (size_t)N * nDim, stream);
   return minim_amd::kDeferSlot;
 }
@@ -878,8 +882,9 @@ void LjNd::redoGradient(int prec, const void* x, void* g, void* stream) const {
   rebuild_list_checked(*impl_, prec, x, N, s);
   const double src6 = std::pow(sigma / cutoff, 6);
   const double eshift = 4 * epsilon * (src6 * src6 - src6);
-  launch_cut(*impl_, prec, x, nullptr, 0.0, N, sigma, epsilon, eshift, 2, g, ws.rs(), s);
-  minim_amd::launch_finalize(ws.rs(), 3, cut_blocks(N), s);
+  const minim_amd::RedScratch rs = ws.rs();
+  launch_cut(*impl_, prec, x, nullptr, 0.0, N, sigma, epsilon, eshift, 2, g, rs, s);
+  minim_amd::launch_finalize(rs, 3, cut_blocks(N), s);
   constrainDevice(prec, x, g, (size_t)N * nDim, stream);
 }
 
@@ -903,8 +908,9 @@ void LjNd::fireGradient(int prec, const void* x, void* g, const void* v, int, bo
     if (r[4] > 0) grow_list(I, N, (int)r[4]);
   }
   if (again || !I.built) rebuild_list(I, prec, x, nullptr, 0.0, N, s);
-  launch_cut(I, prec, x, nullptr, 0.0, N, sigma, epsilon, 0.0, 2, g, ws.rs(), s, v);
-  minim_amd::launch_finalize(ws.rs(), 6, cut_blocks(N), s, -1, nullptr, 5);
+  const minim_amd::RedScratch rs = ws.rs();
+  launch_cut(I, prec, x, nullptr, 0.0, N, sigma, epsilon, 0.0, 2, g, rs, s, v);
+  minim_amd::launch_finalize(rs, 6, cut_blocks(N), s, 5);
 }
 
 // Average duration (ms) of reps launches of the force kernel (cutoff mode:

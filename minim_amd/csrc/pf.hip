@@ -208,8 +208,8 @@ __device__ __forceinline__ void resolve_plane(PlaneIn<T, TV, NF, R, DIR>& p, T t
 
 // MODE bits: 1 = energy, 2 = gradient (+ g.g), 4 = trial point x + t*d,
 // 8 = the trial point also written to xo (an accepted line-search step and
-// the gradient there in one pass).
-template <typename T, typename TV, int NF, int DM, int MODE, int R>
+// the gradient there in one pass).  SELF: the last block finishes the sums.
+template <typename T, typename TV, int NF, int DM, int MODE, int R, bool SELF>
 __global__ __launch_bounds__(kBlock) void pf_tile_kernel(PFArgs a, TileGeom G, const T* __restrict__ x,
                                                          const TV* __restrict__ d, T t, TV* __restrict__ g,
                                                          RedScratch rs, T* __restrict__ xo) {
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(kBlock) void pf_tile_kernel(PFArgs a, TileGeom G, c
 #pragma unroll
       for (int k = 0; k < NF; k++) lds[b][th.hrow][th.hcol][k] = q.hx[k];
   }
-  grid_sum_store<2>(acc, rs);
+  grid_sum_store<2, SELF>(acc, rs);
 }
 
 // Rows per thread: the three plane copies of the own rows plus the plane in
@@ -488,6 +488,9 @@ TileGeom tile_geom_for(const PFArgs& a) {
   return G;
 }
 
+// A launch of the tiled kernel that finishes its own sums.
+bool pf_self(const RedScratch& rs, int nb) { return rs.ticket && nb <= kSelfBlocks; }
+
 template <typename T, typename TV, int NF, int DM, int MODE>
 void launch_tile(const PFArgs& a, const TileGeom& G, const void* x, const void* d, double t, void* g, RedScratch rs,
                  hipStream_t s, void* xo) {
@@ -497,8 +500,12 @@ void launch_tile(const PFArgs& a, const TileGeom& G, const void* x, const void* 
   const TV* dd = static_cast<const TV*>((MODE & 4) ? d : x);
   TV* gg = static_cast<TV*>((MODE & 2) ? g : const_cast<void*>(x));
   T* xx = static_cast<T*>((MODE & 8) ? xo : const_cast<void*>(x));
-  pf_tile_kernel<T, TV, NF, DM, MODE, R><<<G.nblocks, kBlock, 0, s>>>(a, G, static_cast<const T*>(x), dd, (T)t, gg,
-                                                                      rs, xx);
+  if (pf_self(rs, G.nblocks))
+    pf_tile_kernel<T, TV, NF, DM, MODE, R, true>
+        <<<G.nblocks, kBlock, 0, s>>>(a, G, static_cast<const T*>(x), dd, (T)t, gg, rs, xx);
+  else
+    pf_tile_kernel<T, TV, NF, DM, MODE, R, false>
+        <<<G.nblocks, kBlock, 0, s>>>(a, G, static_cast<const T*>(x), dd, (T)t, gg, rs, xx);
 }
 
 template <typename T, typename TV, int NF, int MODE>
@@ -629,6 +636,8 @@ void pf_launch_eval(const PFArgs& a, int prec, int pv, int mode, const void* x, 
                     void* g, RedScratch rs, hipStream_t s, bool finalize, void* xout, hipEvent_t evBefore,
                     hipEvent_t evAfter, double* eOut) {
   int nb;
+  const RedScratch plain = rs;
+  rs = rs.only(0, (mode & 1) ? eOut : nullptr);
   if (evBefore) MINIM_HIP_CHECK(hipEventRecord(evBefore, s));
   if (xout) {
     if (mode != 7 || a.use_ext || a.volfix)
@@ -651,9 +660,10 @@ void pf_launch_eval(const PFArgs& a, int prec, int pv, int mode, const void* x, 
   MINIM_HIP_CHECK(hipGetLastError());
   if (evAfter) MINIM_HIP_CHECK(hipEventRecord(evAfter, s));
   if (finalize) {
-    launch_finalize(rs, 2, nb, s, 0, (mode & 1) ? eOut : nullptr);
+    const bool done = !a.use_ext && a.nf <= 4 && pf_self(rs, nb);
+    if (!done) launch_finalize(rs, 2, nb, s);
     // fixed volumes: the global part of the gradient projection; g.g anew
-    if ((mode & 2) && a.volfix) pf_launch_volume_projection(a, pv, g, (size_t)a.X * a.YZ, true, rs, s);
+    if ((mode & 2) && a.volfix) pf_launch_volume_projection(a, pv, g, (size_t)a.X * a.YZ, true, plain, s);
   }
 }
 

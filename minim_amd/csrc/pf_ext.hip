@@ -946,13 +946,14 @@ void volproj_t(const PFArgs& a, void* v, size_t nsite, bool norm, RedScratch rs,
   launch_finalize(slot, K, nb, s);
   const double* sums = rs.result + kPFVolSlot;
   if (norm) {
+    const RedScratch norms = rs.from(1);
     switch (a.nf) {
-      case 2: pf_volproj_apply_kernel<T, 2, true><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, rs); break;
-      case 3: pf_volproj_apply_kernel<T, 3, true><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, rs); break;
-      case 4: pf_volproj_apply_kernel<T, 4, true><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, rs); break;
-      default: pf_volproj_apply_kernel<T, 0, true><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, rs); break;
+      case 2: pf_volproj_apply_kernel<T, 2, true><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, norms); break;
+      case 3: pf_volproj_apply_kernel<T, 3, true><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, norms); break;
+      case 4: pf_volproj_apply_kernel<T, 4, true><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, norms); break;
+      default: pf_volproj_apply_kernel<T, 0, true><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, norms); break;
     }
-    launch_finalize(rs.from(1), 1, nb, s);
+    launch_finalize(norms, 1, nb, s);
   } else {
     switch (a.nf) {
       case 2: pf_volproj_apply_kernel<T, 2, false><<<nb, kBlock, 0, s>>>(a, u, nsite, sums, rs); break;

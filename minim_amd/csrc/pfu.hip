@@ -698,9 +698,10 @@ void eval_t(const PFUArgs& u, const PFArgs& con, int mode, const void* x, const 
   T* gg = static_cast<T*>(g);
   const T tt = (T)t;
   const size_t nd = u.ngrid * u.nf;
-  const int nb = launch_elements<T>(u, con, mode, xx, dd, tt, gg, rs, s);
+  const RedScratch re = rs.only(0, (mode & 1) && !u.volfix ? eOut : nullptr);
+  const int nb = launch_elements<T>(u, con, mode, xx, dd, tt, gg, re, s);
   MINIM_HIP_CHECK(hipGetLastError());
-  launch_finalize(rs, 1, nb, s, 0, (mode & 1) && !u.volfix ? eOut : nullptr);
+  launch_finalize(re, 1, nb, s);
   if (u.volfix) {
     const RedScratch slot = rs.from(kPFVolSlot);
     const int nbv = grid_blocks(u.ngrid, 4, 2048);

@@ -906,8 +906,9 @@ std::map<std::string, vector<double>> PhaseField::energyComponents(const vector<
     minim_amd::PFCall cl{};
     cl.terms = bits[c];
     cl.raw = 1;
-    const int nb = minim_amd::pf_launch_ext(a, cl, FP64, FP64, 3, x.data(), nullptr, 0.0, g.data(), ws.rs(), s);
-    minim_amd::launch_finalize(ws.rs(), 2, nb, s);
+    const minim_amd::RedScratch rs = ws.rs();
+    const int nb = minim_amd::pf_launch_ext(a, cl, FP64, FP64, 3, x.data(), nullptr, 0.0, g.data(), rs, s);
+    minim_amd::launch_finalize(rs, 2, nb, s);
     double r[2];
     ws.fetch(s, 2, r);
     out[names[c]] = {r[0], std::sqrt(r[1])};
@@ -933,8 +934,9 @@ std::map<std::string, vector<double>> PhaseField::energyComponents(const vector<
     }
     double gg = 0;
     if (any) {
-      const int nb = minim_amd::pf_launch_ext(a, cl, FP64, FP64, 2, x.data(), nullptr, 0.0, g.data(), ws.rs(), s);
-      minim_amd::launch_finalize(ws.rs(), 2, nb, s);
+      const minim_amd::RedScratch rs = ws.rs();
+      const int nb = minim_amd::pf_launch_ext(a, cl, FP64, FP64, 2, x.data(), nullptr, 0.0, g.data(), rs, s);
+      minim_amd::launch_finalize(rs, 2, nb, s);
       double r[2];
       ws.fetch(s, 2, r);
       gg = r[1];

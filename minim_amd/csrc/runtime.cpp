@@ -36,8 +36,8 @@ void DeviceBuffer::reset(size_t bytes) {
 namespace {
 // One block per reduced value: partials of value k are contiguous.
 __global__ __launch_bounds__(kBlock) void finalize_kernel(const double* __restrict__ partials, int nb,
-                                                          double* __restrict__ result, double* mirror, int dupK,
-                                                          double* dupDst, int maxK) {
+                                                          double* __restrict__ result, double* mirror, int copyK,
+                                                          double* copy, int maxK) {
   __shared__ double lds[kBlock / kWave];
   const int k = blockIdx.x;
   const double* p = partials + (size_t)k * nb;
@@ -52,24 +52,27 @@ __global__ __launch_bounds__(kBlock) void finalize_kernel(const double* __restri
   if (threadIdx.x == 0) {
     result[k] = v[0];
     if (mirror) mirror[k] = v[0];
-    if (k == dupK) *dupDst = v[0];
+    if (k == copyK) *copy = v[0];
   }
 }
 }  // namespace
 
-void launch_finalize(RedScratch rs, int K, int nb, hipStream_t s, int dupK, double* dupDst, int maxK) {
+void launch_finalize(RedScratch rs, int K, int nb, hipStream_t s, int maxK) {
   if (K < 1 || K > kMaxDots || nb < 1 || nb > kMaxRedBlocks)
     throw std::invalid_argument("reduction shape out of range");
-  if (!dupDst) dupK = -1;
-  finalize_kernel<<<K, kBlock, 0, s>>>(rs.partials, nb, rs.result, rs.mirror, dupK, dupDst, maxK);
+  finalize_kernel<<<K, kBlock, 0, s>>>(rs.partials, nb, rs.result, rs.mirror, rs.copyK, rs.copy, maxK);
   MINIM_HIP_CHECK(hipGetLastError());
 }
 
 Workspace::Workspace() {
   const size_t partial_bytes = sizeof(double) * (size_t)kMaxRedBlocks * kMaxDots;
   const size_t result_bytes = sizeof(double) * kMaxDots;
-  mem_.reset(partial_bytes + result_bytes + 256);
+  const size_t few_bytes = sizeof(double) * (size_t)kSelfBlocks * kMaxDots * kTickets;
+  mem_.reset(partial_bytes + result_bytes + few_bytes + sizeof(unsigned) * kTickets + 256);
   char* base = static_cast<char*>(mem_.get());
+  few_ = reinterpret_cast<double*>(base + partial_bytes + result_bytes);
+  tickets_ = reinterpret_cast<unsigned*>(base + partial_bytes + result_bytes + few_bytes);
+  MINIM_HIP_CHECK(hipMemset(tickets_, 0, sizeof(unsigned) * kTickets));
   rs_.partials = reinterpret_cast<double*>(base);
   rs_.result = reinterpret_cast<double*>(base + partial_bytes);
   MINIM_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_), result_bytes, hipHostMallocCoherent));
@@ -98,6 +101,14 @@ Workspace& Workspace::current() {
 void Workspace::fetch(hipStream_t s, int k, double* out) {
   MINIM_HIP_CHECK(hipStreamSynchronize(s));
   for (int i = 0; i < k; i++) out[i] = host_[i];
+}
+
+RedScratch Workspace::rs() {
+  RedScratch r = rs_;
+  r.ticket = tickets_ + next_;
+  r.few = few_ + (size_t)next_ * kSelfBlocks * kMaxDots;
+  next_ = (next_ + 1) % kTickets;
+  return r;
 }
 
 void Workspace::put(hipStream_t s, int slot, double value) {

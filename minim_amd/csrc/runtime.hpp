@@ -57,7 +57,10 @@ class Workspace {
   ~Workspace();
   Workspace(const Workspace&) = delete;
   Workspace& operator=(const Workspace&) = delete;
-  RedScratch rs() const { return rs_; }
+  // The scratch for one launch (or several in stream order): each call hands out
+  // the next of kTickets arrival counters with its partials, so that launches on
+  // several streams do not count together.
+  RedScratch rs();
   // Wait for stream s and copy result[0..k) into out.  Whatever writes a result
   // slot on the device also writes its mirror in pinned host memory, so no copy
   // is launched.
@@ -67,7 +70,11 @@ class Workspace {
 
  private:
   Workspace();
+  static constexpr int kTickets = 16;
   RedScratch rs_{};
+  double* few_ = nullptr;
+  unsigned* tickets_ = nullptr;
+  int next_ = 0;
   double* host_ = nullptr;  // the mirror, as the host sees it
   DeviceBuffer mem_;
 };

@@ -642,7 +642,7 @@ void launch_group_norm_max(int prec, const void* v, size_t n, int dim, RedScratc
   if (prec == F64) group_norm_max_kernel<double><<<nb, kBlock, 0, s>>>((const double*)v, ngroup, dim, rs.partials);
   else group_norm_max_kernel<float><<<nb, kBlock, 0, s>>>((const float*)v, ngroup, dim, rs.partials);
   MINIM_HIP_CHECK(hipGetLastError());
-  launch_finalize(rs, 1, nb, s, -1, nullptr, 0);
+  launch_finalize(rs, 1, nb, s, 0);
 }
 
 void launch_fire_update(int prec, int mode, void* v, const void* g, void* step, double f1, double f2,
