@@ -182,6 +182,8 @@ class Lbfgs : public NewMinimiser<Lbfgs> {
                                       bool writeBack);
   struct Impl;
   std::unique_ptr<Impl> impl_;
+  struct BatchMem;
+  std::shared_ptr<BatchMem> _batchMem;  // minimiseBatch's memory; a copy has its own
 };
 
 class Fire : public NewMinimiser<Fire> {

@@ -39,6 +39,7 @@
 #include <cstring>
 #include <deque>
 #include <stdexcept>
+#include <type_traits>
 #include <vector>
 
 #include "minim/Minimiser.h"
@@ -431,26 +432,27 @@ __device__ __forceinline__ void bdir_body(const BBufs& B, const BDyn& q, const B
   }
 }
 
-// The direction pass with the number of stored pairs as a compile-time value.
-template <int BR, typename TV>
-__device__ __forceinline__ void bdir_any(const BBufs& B, const BDyn& q, const BInst& I, int lb,
-                                         double (&acc)[kKD]) {
-  switch (q.np) {
-    case 0: bdir_body<BR, 0, TV>(B, q, I, lb, acc); break;
-    case 1: bdir_body<BR, 1, TV>(B, q, I, lb, acc); break;
-    case 2: bdir_body<BR, 2, TV>(B, q, I, lb, acc); break;
-    case 3: bdir_body<BR, 3, TV>(B, q, I, lb, acc); break;
-    case 4: bdir_body<BR, 4, TV>(B, q, I, lb, acc); break;
-    case 5: bdir_body<BR, 5, TV>(B, q, I, lb, acc); break;
-    case 6: bdir_body<BR, 6, TV>(B, q, I, lb, acc); break;
-    case 7: bdir_body<BR, 7, TV>(B, q, I, lb, acc); break;
-    case 8: bdir_body<BR, 8, TV>(B, q, I, lb, acc); break;
-    case 9: bdir_body<BR, 9, TV>(B, q, I, lb, acc); break;
-    default: bdir_body<BR, 10, TV>(B, q, I, lb, acc); break;
+// f(P) with the number of stored pairs np as a compile-time value, at most PM.
+template <int PM, typename F>
+__device__ __forceinline__ void with_pairs(int np, F f) {
+  switch (np) {
+    case 0: if constexpr (PM >= 0) f(std::integral_constant<int, 0>()); break;
+    case 1: if constexpr (PM >= 1) f(std::integral_constant<int, 1>()); break;
+    case 2: if constexpr (PM >= 2) f(std::integral_constant<int, 2>()); break;
+    case 3: if constexpr (PM >= 3) f(std::integral_constant<int, 3>()); break;
+    case 4: if constexpr (PM >= 4) f(std::integral_constant<int, 4>()); break;
+    case 5: if constexpr (PM >= 5) f(std::integral_constant<int, 5>()); break;
+    case 6: if constexpr (PM >= 6) f(std::integral_constant<int, 6>()); break;
+    case 7: if constexpr (PM >= 7) f(std::integral_constant<int, 7>()); break;
+    case 8: if constexpr (PM >= 8) f(std::integral_constant<int, 8>()); break;
+    case 9: if constexpr (PM >= 9) f(std::integral_constant<int, 9>()); break;
+    default: f(std::integral_constant<int, PM>()); break;
   }
 }
 
-template <int BR, typename TV>
+// The passes are compiled for at most PM = 5 and PM = 10 stored pairs (m <= 5 is
+// the default): a kernel's registers are those of its largest case.
+template <int BR, int PM, typename TV>
 __global__ __launch_bounds__(kBlock) void bdir_kernel(BBufs B) {
   const int p = find_pos(B.ablk, B.na, blockIdx.x);
   const BDyn& q = B.dyn[B.map ? B.map[p] : p];
@@ -460,8 +462,8 @@ __global__ __launch_bounds__(kBlock) void bdir_kernel(BBufs B) {
   double acc[kKD];
 #pragma unroll
   for (int k = 0; k < kKD; k++) acc[k] = 0;
-  bdir_any<BR, TV>(B, q, I, lb, acc);
-  block_partials<kKD>(acc, (1ull << (2 + q.np)) - 1, B.part);
+  with_pairs<PM>(q.np, [&](auto p) { bdir_body<BR, decltype(p)::value, TV>(B, q, I, lb, acc); });
+  block_partials<kKD>(acc, ((1ull << (2 + q.np)) - 1) & ((1ull << (2 + PM)) - 1), B.part);
 }
 
 // The step, gradient and Gram passes of an iteration in one: x' = x + tau d
@@ -557,7 +559,7 @@ __device__ __forceinline__ void bstep_body(const BBufs& B, const BDyn& q, const 
 }
 
 // The partials a step pass with P stored pairs sums (bit k: partial k).
-__device__ __forceinline__ unsigned long long bstep_mask(int P) {
+__device__ __forceinline__ constexpr unsigned long long bstep_mask(int P) {
   const unsigned long long dm = (1ull << (P + 1)) - 1, ym = (1ull << P) - 1;
   const unsigned long long gon = dm | (ym << kBS) | (3ull << (2 * kBS)) | (dm << (2 * kBS + 2)) |
                                  (ym << (3 * kBS + 2)) | (1ull << (4 * kBS + 2));
@@ -571,26 +573,13 @@ __device__ __forceinline__ void bstep_prec(const BBufs& B, const BDyn& q, const 
   else bstep_body<BR, P, double, TV>(B, q, I, lb, acc);
 }
 
-// The step pass with the number of stored pairs as a compile-time value.
-template <int BR, typename TV>
+template <int BR, int PM, typename TV>
 __device__ __forceinline__ void bstep_any(const BBufs& B, const BDyn& q, const BInst& I, int lb,
                                           double (&acc)[kKS]) {
-  switch (q.np) {
-    case 0: bstep_prec<BR, 0, TV>(B, q, I, lb, acc); break;
-    case 1: bstep_prec<BR, 1, TV>(B, q, I, lb, acc); break;
-    case 2: bstep_prec<BR, 2, TV>(B, q, I, lb, acc); break;
-    case 3: bstep_prec<BR, 3, TV>(B, q, I, lb, acc); break;
-    case 4: bstep_prec<BR, 4, TV>(B, q, I, lb, acc); break;
-    case 5: bstep_prec<BR, 5, TV>(B, q, I, lb, acc); break;
-    case 6: bstep_prec<BR, 6, TV>(B, q, I, lb, acc); break;
-    case 7: bstep_prec<BR, 7, TV>(B, q, I, lb, acc); break;
-    case 8: bstep_prec<BR, 8, TV>(B, q, I, lb, acc); break;
-    case 9: bstep_prec<BR, 9, TV>(B, q, I, lb, acc); break;
-    default: bstep_prec<BR, 10, TV>(B, q, I, lb, acc); break;
-  }
+  with_pairs<PM>(q.np, [&](auto p) { bstep_prec<BR, decltype(p)::value, TV>(B, q, I, lb, acc); });
 }
 
-template <int BR, typename TV>
+template <int BR, int PM, typename TV>
 __global__ __launch_bounds__(kBlock) void bstep_kernel(BBufs B) {
   const int p = find_pos(B.ablk, B.na, blockIdx.x);
   const BDyn& q = B.dyn[B.map ? B.map[p] : p];
@@ -600,14 +589,14 @@ __global__ __launch_bounds__(kBlock) void bstep_kernel(BBufs B) {
   double acc[kKS];
 #pragma unroll
   for (int k = 0; k < kKS; k++) acc[k] = 0;
-  bstep_any<BR, TV>(B, q, I, lb, acc);
-  block_partials<kKS>(acc, bstep_mask(q.np), B.part);
+  bstep_any<BR, PM, TV>(B, q, I, lb, acc);
+  block_partials<kKS>(acc, bstep_mask(q.np) & bstep_mask(PM), B.part);
 }
 
 // Device control: one launch for the line-search pass of the instances still
 // searching and the step pass of those whose search has ended (the phase is
 // uniform over an instance's blocks).  Both write rows of kKS partials.
-template <int BR, typename TV>
+template <int BR, int PM, typename TV>
 __global__ __launch_bounds__(kBlock) void bts_kernel(BBufs B) {
   const int p = find_pos(B.ablk, B.na, blockIdx.x);
   const BDyn& q = B.dyn[B.map[p]];
@@ -618,8 +607,8 @@ __global__ __launch_bounds__(kBlock) void bts_kernel(BBufs B) {
     double acc[kKS];
 #pragma unroll
     for (int k = 0; k < kKS; k++) acc[k] = 0;
-    bstep_any<BR, TV>(B, q, I, lb, acc);
-    block_partials<kKS>(acc, bstep_mask(q.np), B.part);
+    bstep_any<BR, PM, TV>(B, q, I, lb, acc);
+    block_partials<kKS>(acc, bstep_mask(q.np) & bstep_mask(PM), B.part);
   } else {
     double acc[kNT];
 #pragma unroll
@@ -1203,26 +1192,41 @@ struct Inst {
 using KFn = void (*)(BBufs);
 struct Kernels {
   KFn pf_eg, pf_trial, dir, step, fresh, round, ts;
-  void (*resident5)(BBufs, BCtlArgs);   // FP64 only, m <= 5
-  void (*resident10)(BBufs, BCtlArgs);  // FP64 only, m <= 10
+  void (*resident)(BBufs, BCtlArgs);  // FP64 only
 };
-template <int BR, typename TV>
+template <int BR, int PM, typename TV>
 Kernels kernels_br() {
-  Kernels k{bpf_kernel<BR, 3, TV>,  btrial_kernel<BR, TV>, bdir_kernel<BR, TV>, bstep_kernel<BR, TV>,
-            bpf_kernel<BR, 11, TV>, bround_kernel<BR>,     bts_kernel<BR, TV>,  nullptr,
-            nullptr};
-  if constexpr (sizeof(TV) == 8) {
-    k.resident5 = bres_kernel<BR, 5, TV>;
-    k.resident10 = bres_kernel<BR, 10, TV>;
-  }
+  Kernels k{bpf_kernel<BR, 3, TV>,  btrial_kernel<BR, TV>, bdir_kernel<BR, PM, TV>, bstep_kernel<BR, PM, TV>,
+            bpf_kernel<BR, 11, TV>, bround_kernel<BR>,     bts_kernel<BR, PM, TV>,  nullptr};
+  if constexpr (sizeof(TV) == 8) k.resident = bres_kernel<BR, PM, TV>;
   return k;
 }
-template <typename TV>
-Kernels kernels_for(int br) {
+template <int PM, typename TV>
+Kernels kernels_pm(int br) {
   switch (br) {
-    case 4: return kernels_br<4, TV>();
-    case 16: return kernels_br<16, TV>();
-    default: return kernels_br<8, TV>();
+    case 4: return kernels_br<4, PM, TV>();
+    case 16: return kernels_br<16, PM, TV>();
+    default: return kernels_br<8, PM, TV>();
+  }
+}
+template <typename TV>
+Kernels kernels_for(int br, int m) {
+  return m <= 5 ? kernels_pm<5, TV>(br) : kernels_pm<10, TV>(br);
+}
+
+// A State's coordinates and their place in the batch.
+struct BCopy {
+  double* state;
+  double* batch;
+  int n;
+};
+__global__ __launch_bounds__(kBlock) void bcopy_kernel(const BCopy* __restrict__ list, int ni, int toBatch) {
+  for (int j = blockIdx.y; j < ni; j += gridDim.y) {
+    const BCopy c = list[j];
+    const double* __restrict__ src = toBatch ? c.state : c.batch;
+    double* __restrict__ dst = toBatch ? c.batch : c.state;
+    for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < (size_t)c.n; i += (size_t)gridDim.x * kBlock)
+      dst[i] = src[i];
   }
 }
 
@@ -1237,6 +1241,47 @@ struct Launch {
 }  // namespace minim_amd
 
 namespace minim {
+
+// Device and pinned memory, stream and events of minimiseBatch: kept by the
+// Lbfgs for its next call (each buffer grows to the largest batch seen, and all
+// go with the object), because allocating and freeing some twenty of them took
+// a fifth of a short batch.  One call at a time, as for the rest of an Lbfgs.
+struct Lbfgs::BatchMem {
+  int device = -1;
+  static constexpr int kDev = 18, kPin = 5;
+  minim_amd::DeviceBuffer buf[kDev];
+  void* pin_[kPin] = {};
+  size_t pinBytes[kPin] = {};
+  hipStream_t stream = nullptr;
+  hipEvent_t event[2] = {nullptr, nullptr};
+  explicit BatchMem(int dev) : device(dev) {
+    MINIM_HIP_CHECK(hipStreamCreate(&stream));
+    for (auto& e : event) MINIM_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  ~BatchMem() {
+    for (void* p : pin_)
+      if (p) (void)hipHostFree(p);
+    for (auto& e : event)
+      if (e) (void)hipEventDestroy(e);
+    if (stream) (void)hipStreamDestroy(stream);
+  }
+  BatchMem(const BatchMem&) = delete;
+  BatchMem& operator=(const BatchMem&) = delete;
+  minim_amd::DeviceBuffer& dev(int i, size_t bytes) {
+    if (buf[i].bytes() < bytes) buf[i].reset(bytes);
+    return buf[i];
+  }
+  void* pin(int i, size_t bytes) {
+    if (pinBytes[i] < bytes) {
+      if (pin_[i]) MINIM_HIP_CHECK(hipHostFree(pin_[i]));
+      pin_[i] = nullptr;
+      pinBytes[i] = 0;
+      MINIM_HIP_CHECK(hipHostMalloc(&pin_[i], bytes));
+      pinBytes[i] = bytes;
+    }
+    return pin_[i];
+  }
+};
 
 std::vector<MinimiseStats> Lbfgs::minimiseBatch(const std::vector<State*>& states) {
   return batchRun(states, 0, 0, true);
@@ -1306,7 +1351,7 @@ std::vector<MinimiseStats> Lbfgs::batchRun(const std::vector<State*>& states, in
     if (block != 4 && block != 8 && block != 16) block = nTot < kSmallBatch ? kBlockSmall : kBlockDefault;
   }
   const int kBE = block * kBlock;  // elements per block
-  const Kernels K = mixed ? kernels_for<float>(block) : kernels_for<double>(block);
+  const Kernels K = mixed ? kernels_for<float>(block, _m) : kernels_for<double>(block, _m);
 
   std::vector<Inst> in(ni);
   size_t N = 0;
@@ -1353,31 +1398,44 @@ std::vector<MinimiseStats> Lbfgs::batchRun(const std::vector<State*>& states, in
   auto since = [&] { return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count(); };
 
   const int S = _m + 1;
-  DeviceBuffer Xa(N * 8), Xb(N * 8), G0(N * vb), G1(N * vb), Dm(N * vb * S), Ym(N * vb * S);
+  int device = 0;
+  MINIM_HIP_CHECK(hipGetDevice(&device));
+  if (!_batchMem || _batchMem->device != device) _batchMem = std::make_shared<BatchMem>(device);
+  BatchMem& W = *_batchMem;
+  DeviceBuffer &Xa = W.dev(0, N * 8), &Xb = W.dev(1, N * 8), &G0 = W.dev(2, N * vb), &G1 = W.dev(3, N * vb),
+               &Dm = W.dev(4, N * vb * S), &Ym = W.dev(5, N * vb * S);
   // per-phase staging, one copy per phase: block prefix sums, then the BDyn of
   // each instance in the launch
   const size_t ablkBytes = (sizeof(int) * (ni + 1) + 15) / 16 * 16;
   const size_t stageBytes = ablkBytes + sizeof(BDyn) * ni;
-  DeviceBuffer instD(sizeof(BInst) * ni), stageD(stageBytes);
+  DeviceBuffer &instD = W.dev(6, sizeof(BInst) * ni), &stageD = W.dev(7, stageBytes);
   // results of one fetch: fresh (pf + dots), direction + trials, or step
   constexpr int kRes = std::max(std::max(kKF, kKD + kNT), kKS);
-  DeviceBuffer part(sizeof(double) * (size_t)totalBlocks * kKS), res(sizeof(double) * (size_t)ni * kRes);
-  struct Pinned {
-    void* p = nullptr;
-    explicit Pinned(size_t b) { MINIM_HIP_CHECK(hipHostMalloc(&p, b)); }
-    ~Pinned() { (void)hipHostFree(p); }
+  DeviceBuffer &part = W.dev(8, sizeof(double) * (size_t)totalBlocks * kKS),
+               &res = W.dev(9, sizeof(double) * (size_t)ni * kRes), &copyD = W.dev(10, sizeof(BCopy) * ni);
+  BCopy* copyh = static_cast<BCopy*>(W.pin(0, sizeof(BCopy) * ni));
+  void* stageH = W.pin(1, stageBytes);
+  int* ablkh = static_cast<int*>(stageH);
+  BDyn* dynh = reinterpret_cast<BDyn*>(static_cast<char*>(stageH) + ablkBytes);
+  double* resh = static_cast<double*>(W.pin(2, sizeof(double) * (size_t)ni * kRes));
+  // the coordinates of every State, in one launch
+  auto copyCoords = [&](bool in_) {
+    MINIM_HIP_CHECK(hipMemcpyAsync(copyD.get(), copyh, sizeof(BCopy) * ni, hipMemcpyHostToDevice, st));
+    int most = 0;
+    for (const Inst& I : in) most = std::max(most, I.bi.n);
+    const dim3 grid((unsigned)grid_blocks(most, 8, 128), (unsigned)std::min(ni, 65535));
+    bcopy_kernel<<<grid, kBlock, 0, st>>>(static_cast<const BCopy*>(copyD.get()), ni, in_ ? 1 : 0);
+    MINIM_HIP_CHECK(hipGetLastError());
   };
-  Pinned stageH(stageBytes), resH(sizeof(double) * (size_t)ni * kRes);
-  int* ablkh = static_cast<int*>(stageH.p);
-  BDyn* dynh = reinterpret_cast<BDyn*>(static_cast<char*>(stageH.p) + ablkBytes);
-  double* resh = static_cast<double*>(resH.p);
 
   {
     std::vector<BInst> bi(ni);
     for (int j = 0; j < ni; j++) bi[j] = in[j].bi;
     MINIM_HIP_CHECK(hipMemcpyAsync(instD.get(), bi.data(), sizeof(BInst) * ni, hipMemcpyHostToDevice, st));
     for (int j = 0; j < ni; j++)
-      device_copy(static_cast<double*>(Xa.get()) + in[j].bi.off, in[j].s->deviceCoords(), in[j].bi.n * 8, st);
+      copyh[j] = {static_cast<double*>(in[j].s->deviceCoords()), static_cast<double*>(Xa.get()) + in[j].bi.off,
+                  in[j].bi.n};
+    copyCoords(true);
     MINIM_HIP_CHECK(hipStreamSynchronize(st));  // bi leaves scope
   }
 
@@ -1403,7 +1461,7 @@ std::vector<MinimiseStats> Lbfgs::batchRun(const std::vector<State*>& states, in
     for (int p = 0; p < L.na; p++) ablkh[p + 1] = ablkh[p] + in[L.pos[p]].nblk;
     L.nb = ablkh[L.na];
     MINIM_HIP_CHECK(
-        hipMemcpyAsync(stageD.get(), stageH.p, ablkBytes + sizeof(BDyn) * L.na, hipMemcpyHostToDevice, st));
+        hipMemcpyAsync(stageD.get(), stageH, ablkBytes + sizeof(BDyn) * L.na, hipMemcpyHostToDevice, st));
     B.na = L.na;
   };
   auto finalize = [&](const Launch& L, int K, size_t resOff) {
@@ -1472,21 +1530,18 @@ std::vector<MinimiseStats> Lbfgs::batchRun(const std::vector<State*>& states, in
     const size_t rPF = 0, rF = rPF + (size_t)ni * kKP, rEnd = rF + (size_t)ni * kKF;
     // the start clock at byte 8, the live flags from byte 64
     const size_t cntBytes = 64 + sizeof(int) * (size_t)ni;
-    DeviceBuffer ablkA(sizeof(int) * (ni + 1)), mapA(sizeof(int) * ni), dynA(sizeof(BDyn) * ni),
-        ctlA(sizeof(BCtl) * ni), resA(8 * rEnd), cntA(cntBytes), part2(sizeof(double) * (size_t)totalBlocks * kNT);
-    Pinned cntH(cntBytes), cntH2(cntBytes);  // the flags of two chunks in turn
-    std::memset(cntH.p, 0, cntBytes);
+    DeviceBuffer &ablkA = W.dev(11, sizeof(int) * (ni + 1)), &mapA = W.dev(12, sizeof(int) * ni),
+                 &dynA = W.dev(13, sizeof(BDyn) * ni), &ctlA = W.dev(14, sizeof(BCtl) * ni),
+                 &resA = W.dev(15, 8 * rEnd), &cntA = W.dev(16, cntBytes),
+                 &part2 = W.dev(17, sizeof(double) * (size_t)totalBlocks * kNT);
+    void* flagsH[2] = {W.pin(3, cntBytes), W.pin(4, cntBytes)};  // the flags of two chunks in turn
+    std::memset(flagsH[0], 0, cntBytes);
     MINIM_HIP_CHECK(hipMemcpyAsync(dynA.get(), dy0.data(), sizeof(BDyn) * ni, hipMemcpyHostToDevice, st));
     MINIM_HIP_CHECK(hipMemcpyAsync(ctlA.get(), c0.data(), sizeof(BCtl) * ni, hipMemcpyHostToDevice, st));
-    MINIM_HIP_CHECK(hipMemcpyAsync(cntA.get(), cntH.p, cntBytes, hipMemcpyHostToDevice, st));
+    MINIM_HIP_CHECK(hipMemcpyAsync(cntA.get(), flagsH[0], cntBytes, hipMemcpyHostToDevice, st));
     MINIM_HIP_CHECK(hipStreamSynchronize(st));
     // a stream of its own: graph capture needs one other than the null stream
-    hipStream_t cs = nullptr;
-    MINIM_HIP_CHECK(hipStreamCreate(&cs));
-    struct StreamGuard {
-      hipStream_t s;
-      ~StreamGuard() { (void)hipStreamDestroy(s); }
-    } csGuard{cs};
+    hipStream_t cs = W.stream;
     BBufs G = B;
     G.ablk = static_cast<const int*>(ablkA.get());
     G.map = static_cast<const int*>(mapA.get());
@@ -1603,7 +1658,7 @@ std::vector<MinimiseStats> Lbfgs::batchRun(const std::vector<State*>& states, in
       MINIM_HIP_CHECK(hipGetLastError());
       // autotuneBatch's bounded runs: at most replayLimit iterations each
       if (replayLimit > 0) A.maxIter = (int)std::min<long>(maxIter, replayLimit - 1);
-      auto* kres = _m <= 5 ? K.resident5 : K.resident10;
+      auto* kres = K.resident;
       if (!kres) throw std::logic_error("Lbfgs::minimiseBatch: no resident kernel for this storage type.");
       BBufs R = G;
       R.map = nullptr;
@@ -1667,16 +1722,6 @@ std::vector<MinimiseStats> Lbfgs::batchRun(const std::vector<State*>& states, in
     // fresh phase) take effect a chunk later; an instance's result does not
     // depend on when.  After an admission or a new layout (which drain the
     // stream) the flags still in flight are dropped: they predate it.
-    struct Events {
-      hipEvent_t e[2] = {nullptr, nullptr};
-      Events() {
-        for (auto& x : e) MINIM_HIP_CHECK(hipEventCreateWithFlags(&x, hipEventDisableTiming));
-      }
-      ~Events() {
-        for (auto& x : e) (void)hipEventDestroy(x);
-      }
-    } ev;
-    void* flagsH[2] = {cntH.p, cntH2.p};
     long chunk = 0, unread = -1;  // the chunk whose flags are in flight, or -1
     for (;;) {
       for (int k = 0; k < kChunk; k++) {
@@ -1693,12 +1738,12 @@ std::vector<MinimiseStats> Lbfgs::batchRun(const std::vector<State*>& states, in
       }
       const int cb = (int)(chunk & 1);
       MINIM_HIP_CHECK(hipMemcpyAsync(flagsH[cb], cntA.get(), cntBytes, hipMemcpyDeviceToHost, cs));
-      MINIM_HIP_CHECK(hipEventRecord(ev.e[cb], cs));
+      MINIM_HIP_CHECK(hipEventRecord(W.event[cb], cs));
       const long readable = unread;
       unread = chunk++;
       if (readable < 0) continue;  // nothing to read yet: queue another chunk first
       const int rb = (int)(readable & 1);
-      MINIM_HIP_CHECK(hipEventSynchronize(ev.e[rb]));
+      MINIM_HIP_CHECK(hipEventSynchronize(W.event[rb]));
       hostSyncs++;
       const int* liveH = reinterpret_cast<const int*>(static_cast<const char*>(flagsH[rb]) + 64);
       long liveBlocks = 0;
@@ -2060,12 +2105,14 @@ std::vector<MinimiseStats> Lbfgs::batchRun(const std::vector<State*>& states, in
   }
   for (int j = 0; j < ni; j++) {
     Inst& I = in[j];
-    device_copy(I.s->deviceCoords(), static_cast<double*>(I.xcur ? Xb.get() : Xa.get()) + I.bi.off, I.bi.n * 8, st);
+    copyh[j] = {static_cast<double*>(I.s->deviceCoords()),
+                static_cast<double*>(I.xcur ? Xb.get() : Xa.get()) + I.bi.off, I.bi.n};
     I.s->invalidateHost();
     I.st.energy = I.e;
     I.st.gradRms = std::sqrt(I.gg / I.bi.n);
     out[j] = I.st;
   }
+  copyCoords(false);
   MINIM_HIP_CHECK(hipStreamSynchronize(st));
   stats = MinimiseStats{};
   iter = maxIters;

@@ -504,3 +504,21 @@ def test_batch_resident_autotune(gpu):
     assert lb.batchReport()["block"] == min(t, key=t.get)
     assert all(r["converged"] for r in res)
     m.autotune_clear()
+
+
+@pytest.mark.parametrize("pairs", [5, 6, 10])
+def test_batch_memory_is_reused(gpu, pairs):
+    """One Lbfgs over batches that grow, shrink and change the schedule, at the
+    pair counts on either side of the two compiled limits: each result is bit
+    for bit that of an Lbfgs that has run nothing before."""
+    m = gpu
+    kept = m.Lbfgs().setM(pairs).setMaxIter(25)
+    for sides, mode in (((8, 50), "fp64"), ((64, 100, 13), "mixed"), ((9,), "fp64"), ((33, 64, 8, 100), "fp64")):
+        cs = cases(len(sides), sides=sides, extra=())
+        out = []
+        for lb in (kept, m.Lbfgs().setM(pairs).setMaxIter(25)):
+            states = [make_state(m, c) for c in cs]
+            res = lb.setPrecision(mode).minimiseBatch(states)
+            out.append(([s.coords() for s in states], [r["energy"] for r in res]))
+        assert all(np.array_equal(a, b) for a, b in zip(out[0][0], out[1][0]))
+        assert out[0][1] == out[1][1]
