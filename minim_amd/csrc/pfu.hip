@@ -508,8 +508,9 @@ __global__ __launch_bounds__(kBlock) void pfu_site_kernel(PFUArgs u, PFArgs con,
 #pragma nounroll
   for (int i = x0; i < x1; i++) {
     const int b = (i - x0) & 1;
+    const bool more = i + 1 < x1;  // the chunk's last plane needs no further one
     Plane q;
-    load(i + 2, q);
+    if (more) load(i + 2, q);
     T* gp = g + (size_t)i * YZ * NF;
 #pragma unroll
     for (int r = 0; r < R; r++) {
@@ -537,6 +538,7 @@ __global__ __launch_bounds__(kBlock) void pfu_site_kernel(PFUArgs u, PFArgs con,
         }
       }
     }
+    if (!more) break;
     lds_barrier();  // every wave is done reading buffer b
     fill(b, q);
 #pragma unroll
