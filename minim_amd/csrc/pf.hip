@@ -163,33 +163,36 @@ __device__ __forceinline__ void site_tile(const PFArgs& a, const T (&c)[NF], con
   }
 }
 
-// Plane data of the R own rows and the halo site, as loaded (x, and d for a
+// Plane data of the R own rows and the H halo sites, as loaded (x, and d for a
 // trial point).
-template <typename T, typename TV, int NF, int R, bool DIR>
+template <typename T, typename TV, int NF, int R, bool DIR, int H = 1>
 struct PlaneIn {
   T x[R][NF];
-  T hx[NF];
+  T hx[H][NF];
   TV d[DIR ? R : 1][NF];
-  TV hd[NF];
+  TV hd[H][NF];
 };
 
-template <typename T, typename TV, int NF, int R, bool DIR>
+template <typename T, typename TV, int NF, int R, bool DIR, int H>
 __device__ __forceinline__ void load_plane(const T* __restrict__ xp, const TV* __restrict__ dp,
-                                           const unsigned (&ox)[R], const unsigned (&od)[R], unsigned hox,
-                                           unsigned hod, PlaneIn<T, TV, NF, R, DIR>& p) {
+                                           const unsigned (&ox)[R], const unsigned (&od)[R],
+                                           const unsigned (&hox)[H], const unsigned (&hod)[H],
+                                           PlaneIn<T, TV, NF, R, DIR, H>& p) {
 #pragma unroll
   for (int r = 0; r < R; r++) ld_site<T, NF>(xp, ox[r], p.x[r]);
-  ld_site<T, NF>(xp, hox, p.hx);
+#pragma unroll
+  for (int h = 0; h < H; h++) ld_site<T, NF>(xp, hox[h], p.hx[h]);
   if constexpr (DIR) {
 #pragma unroll
     for (int r = 0; r < R; r++) ld_site<TV, NF>(dp, od[r], p.d[r]);
-    ld_site<TV, NF>(dp, hod, p.hd);
+#pragma unroll
+    for (int h = 0; h < H; h++) ld_site<TV, NF>(dp, hod[h], p.hd[h]);
   }
 }
 
 // Coordinates of a loaded plane: x, or the trial point x + (t*d).
-template <typename T, typename TV, int NF, int R, bool DIR>
-__device__ __forceinline__ void resolve_plane(PlaneIn<T, TV, NF, R, DIR>& p, T t) {
+template <typename T, typename TV, int NF, int R, bool DIR, int H>
+__device__ __forceinline__ void resolve_plane(PlaneIn<T, TV, NF, R, DIR, H>& p, T t) {
   if constexpr (DIR) {
 #pragma unroll
     for (int r = 0; r < R; r++)
@@ -199,10 +202,12 @@ __device__ __forceinline__ void resolve_plane(PlaneIn<T, TV, NF, R, DIR>& p, T t
         p.x[r][k] = p.x[r][k] + s;
       }
 #pragma unroll
-    for (int k = 0; k < NF; k++) {
-      const T s = t * (T)p.hd[k];
-      p.hx[k] = p.hx[k] + s;
-    }
+    for (int h = 0; h < H; h++)
+#pragma unroll
+      for (int k = 0; k < NF; k++) {
+        const T s = t * (T)p.hd[h][k];
+        p.hx[h][k] = p.hx[h][k] + s;
+      }
   }
 }
 
@@ -227,8 +232,8 @@ __global__ __launch_bounds__(kBlock) void pf_tile_kernel(PFArgs a, TileGeom G, c
     ox[r] = th.site[r] * (unsigned)(NF * sizeof(T));
     od[r] = th.site[r] * (unsigned)(NF * sizeof(TV));
   }
-  const unsigned hox = th.hsite * (unsigned)(NF * sizeof(T));
-  const unsigned hod = th.hsite * (unsigned)(NF * sizeof(TV));
+  const unsigned hox[1] = {th.hsite * (unsigned)(NF * sizeof(T))};
+  const unsigned hod[1] = {th.hsite * (unsigned)(NF * sizeof(TV))};
   const bool halo = th.hrow >= 0;
   const int x0 = th.x0, x1 = th.x1;
 
@@ -237,12 +242,12 @@ __global__ __launch_bounds__(kBlock) void pf_tile_kernel(PFArgs a, TileGeom G, c
     PlaneIn<T, TV, NF, R, DIR> pm, p0, p1;
     const size_t sm = (size_t)tile_plane(x0 - 1, X) * plane, s0 = (size_t)tile_plane(x0, X) * plane,
                  s1 = (size_t)tile_plane(x0 + 1, X) * plane;
-    load_plane<T, TV, NF, R, DIR>(x + sm, d + sm, ox, od, hox, hod, pm);
-    load_plane<T, TV, NF, R, DIR>(x + s0, d + s0, ox, od, hox, hod, p0);
-    load_plane<T, TV, NF, R, DIR>(x + s1, d + s1, ox, od, hox, hod, p1);
-    resolve_plane<T, TV, NF, R, DIR>(pm, t);
-    resolve_plane<T, TV, NF, R, DIR>(p0, t);
-    resolve_plane<T, TV, NF, R, DIR>(p1, t);
+    load_plane(x + sm, d + sm, ox, od, hox, hod, pm);
+    load_plane(x + s0, d + s0, ox, od, hox, hod, p0);
+    load_plane(x + s1, d + s1, ox, od, hox, hod, p1);
+    resolve_plane(pm, t);
+    resolve_plane(p0, t);
+    resolve_plane(p1, t);
 #pragma unroll
     for (int r = 0; r < R; r++)
 #pragma unroll
@@ -256,8 +261,8 @@ __global__ __launch_bounds__(kBlock) void pf_tile_kernel(PFArgs a, TileGeom G, c
     if (halo)
 #pragma unroll
       for (int k = 0; k < NF; k++) {
-        lds[0][th.hrow][th.hcol][k] = p0.hx[k];
-        lds[1][th.hrow][th.hcol][k] = p1.hx[k];
+        lds[0][th.hrow][th.hcol][k] = p0.hx[0][k];
+        lds[1][th.hrow][th.hcol][k] = p1.hx[0][k];
       }
   }
   __syncthreads();
@@ -269,7 +274,7 @@ __global__ __launch_bounds__(kBlock) void pf_tile_kernel(PFArgs a, TileGeom G, c
     // plane i+2 in flight while plane i is computed (wrapped: always a valid plane)
     PlaneIn<T, TV, NF, R, DIR> q;
     const size_t sq = (size_t)tile_plane(i + 2, X) * plane;
-    load_plane<T, TV, NF, R, DIR>(x + sq, d + sq, ox, od, hox, hod, q);
+    load_plane(x + sq, d + sq, ox, od, hox, hod, q);
 
     TV* gp = g + (size_t)i * plane;
     T* xop = xo + (size_t)i * plane;
@@ -303,7 +308,7 @@ __global__ __launch_bounds__(kBlock) void pf_tile_kernel(PFArgs a, TileGeom G, c
     if (WG) acc[1] += (double)gacc;
 
     lds_barrier();  // every wave is done reading buffer b
-    resolve_plane<T, TV, NF, R, DIR>(q, t);
+    resolve_plane(q, t);
 #pragma unroll
     for (int r = 0; r < R; r++)
 #pragma unroll
@@ -315,9 +320,122 @@ __global__ __launch_bounds__(kBlock) void pf_tile_kernel(PFArgs a, TileGeom G, c
       }
     if (halo)
 #pragma unroll
-      for (int k = 0; k < NF; k++) lds[b][th.hrow][th.hcol][k] = q.hx[k];
+      for (int k = 0; k < NF; k++) lds[b][th.hrow][th.hcol][k] = q.hx[0][k];
   }
   grid_sum_store<2, SELF>(acc, rs);
+}
+
+// The same march over flat chunks (pf_tile.hpp), for gradients at x: every
+// in-plane neighbour comes from LDS.  H: halo sites per thread.  Bound by VALU
+// issue and the march's latency like the tiles, but with all lanes inside the
+// grid (tiles: 69 % of them at Y = 131, Z = 97).  Energy and gradient, three
+// fluids: 150x131x97 24.4 -> 22.5 us in FP64 and 15.7 -> 13.8 in FP32,
+// 160x150x141 38.5 -> 35.7 and 22.8 -> 20.3, 100^3 15.5 -> 13.6 and 11.1 -> 10.3.
+template <typename T, typename TV, int NF, int DM, int MODE, int R, int H>
+__global__ __launch_bounds__(kBlock) void pf_flat_kernel(PFArgs a, TileGeom G, const T* __restrict__ x,
+                                                         const TV* __restrict__ d, T t, TV* __restrict__ g,
+                                                         RedScratch rs, T* __restrict__) {
+  constexpr bool WE = MODE & 1, WG = MODE & 2, DIR = false;
+  static_assert((MODE & 6) == 2, "a gradient at x");
+  __shared__ T lds[2][flat_slots(R, H)][NF];
+  FlatThread th;
+  flat_thread(G, xcd_logical_block(blockIdx.x, gridDim.x), threadIdx.x, th);
+  const size_t plane = (size_t)G.Y * G.Z * NF;  // elements per x plane
+  const int X = G.X, Z = G.Z;
+  unsigned ox[R], od[R], hox[H], hod[H];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    ox[r] = th.site[r] * (unsigned)(NF * sizeof(T));
+    od[r] = th.site[r] * (unsigned)(NF * sizeof(TV));
+  }
+#pragma unroll
+  for (int h = 0; h < H; h++) {
+    hox[h] = th.hsite[h] * (unsigned)(NF * sizeof(T));
+    hod[h] = th.hsite[h] * (unsigned)(NF * sizeof(TV));
+  }
+  const int x0 = th.x0, x1 = th.x1;
+  using Plane = PlaneIn<T, TV, NF, R, DIR, H>;
+  auto fill = [&](int b, const Plane& p) {
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+      for (int k = 0; k < NF; k++) lds[b][th.slot[r]][k] = p.x[r][k];
+#pragma unroll
+    for (int h = 0; h < H; h++)
+      if (th.hslot[h] >= 0)
+#pragma unroll
+        for (int k = 0; k < NF; k++) lds[b][th.hslot[h]][k] = p.hx[h][k];
+  };
+
+  T A[R][NF], B[R][NF], Cn[R][NF];  // planes i-1, i, i+1 of the own rows
+  {
+    Plane pm, p0, p1;
+    const size_t sm = (size_t)tile_plane(x0 - 1, X) * plane, s0 = (size_t)tile_plane(x0, X) * plane,
+                 s1 = (size_t)tile_plane(x0 + 1, X) * plane;
+    load_plane(x + sm, d + sm, ox, od, hox, hod, pm);
+    load_plane(x + s0, d + s0, ox, od, hox, hod, p0);
+    load_plane(x + s1, d + s1, ox, od, hox, hod, p1);
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+      for (int k = 0; k < NF; k++) {
+        A[r][k] = pm.x[r][k];
+        B[r][k] = p0.x[r][k];
+        Cn[r][k] = p1.x[r][k];
+      }
+    fill(0, p0);
+    fill(1, p1);
+  }
+  __syncthreads();
+
+  double acc[2] = {0.0, 0.0};  // energy, g.g
+#pragma nounroll
+  for (int i = x0; i < x1; i++) {
+    const int b = (i - x0) & 1;
+    Plane q;
+    const size_t sq = (size_t)tile_plane(i + 2, X) * plane;
+    load_plane(x + sq, d + sq, ox, od, hox, hod, q);
+    TV* gp = g + (size_t)i * plane;
+    T eacc = (T)0, gacc = (T)0;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      T ym[NF], yp[NF], zm[NF], zp[NF], gv[NF], es;
+#pragma unroll
+      for (int k = 0; k < NF; k++) {
+        ym[k] = lds[b][th.slot[r] - Z][k];
+        yp[k] = lds[b][th.slot[r] + Z][k];
+        zm[k] = lds[b][th.zm[r]][k];
+        zp[k] = lds[b][th.zp[r]][k];
+      }
+      site_tile<T, NF, DM, WE, WG>(a, B[r], A[r], Cn[r], ym, yp, zm, zp, es, gv);
+      if (th.own & (1u << r)) {
+        if (WE) eacc = eacc + es;
+        if (WG) {
+          TV gs[NF];
+#pragma unroll
+          for (int k = 0; k < NF; k++) {
+            gs[k] = (TV)gv[k];
+            gacc = fmad((T)gs[k], (T)gs[k], gacc);
+          }
+          st_site<TV, NF>(gp, od[r], gs);
+        }
+      }
+    }
+    if (WE) acc[0] += (double)eacc;
+    if (WG) acc[1] += (double)gacc;
+
+    lds_barrier();  // every wave is done reading buffer b
+    fill(b, q);
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+      for (int k = 0; k < NF; k++) {
+        A[r][k] = B[r][k];
+        B[r][k] = Cn[r][k];
+        Cn[r][k] = q.x[r][k];
+      }
+  }
+  grid_sum_store<2>(acc, rs);
 }
 
 // Rows per thread: the three plane copies of the own rows plus the plane in
@@ -473,7 +591,7 @@ int density_mode(const PFArgs& a) {
 }
 
 template <typename T, typename TV, int NF>
-TileGeom tile_geom_for(const PFArgs& a) {
+TileGeom tile_geom_for(const PFArgs& a, int mode) {
   TileGeom G;
   const int pi = sizeof(T) == 8 ? 0 : 1;
   const bool user = a.target_blocks > 0 || a.xchunk_override > 0;
@@ -481,8 +599,16 @@ TileGeom tile_geom_for(const PFArgs& a) {
                      : (!user && a.tuned_target[pi] > 0) ? a.tuned_target[pi]
                                                          : kTileTargetBlocks;
   const int xo = user ? a.xchunk_override : a.tuned_xchunk[pi];
-  if (!tile_geom(a.X, a.Y, a.Z, tile_rows<T, NF>(), xo, target, kMaxRedBlocks, G))
+  constexpr int R = tile_rows<T, NF>();
+  if (!tile_geom(a.X, a.Y, a.Z, R, xo, target, kMaxRedBlocks, G))
     throw std::invalid_argument("PhaseField: grid too large for one launch");
+  // flat chunks for gradients at x (with or without the energy) that more than
+  // kSelfBlocks blocks share.  Energies alone read two neighbours of a site and
+  // gain nothing, and the fused step sums its energy as the trials do.
+  TileGeom F;
+  if ((mode & 6) == 2 && G.nblocks > kSelfBlocks &&
+      tile_geom(a.X, a.Y, a.Z, R, xo, target, kMaxRedBlocks, F, flat_halo(a.Y, a.Z, R)) && F.nblocks > kSelfBlocks)
+    G = F;
   if ((double)a.Y * a.Z * NF * sizeof(T) >= 4294967296.0)
     throw std::invalid_argument("PhaseField: one x plane of the grid exceeds 4 GiB");
   return G;
@@ -500,12 +626,17 @@ void launch_tile(const PFArgs& a, const TileGeom& G, const void* x, const void* 
   const TV* dd = static_cast<const TV*>((MODE & 4) ? d : x);
   TV* gg = static_cast<TV*>((MODE & 2) ? g : const_cast<void*>(x));
   T* xx = static_cast<T*>((MODE & 8) ? xo : const_cast<void*>(x));
-  if (pf_self(rs, G.nblocks))
-    pf_tile_kernel<T, TV, NF, DM, MODE, R, true>
-        <<<G.nblocks, kBlock, 0, s>>>(a, G, static_cast<const T*>(x), dd, (T)t, gg, rs, xx);
-  else
-    pf_tile_kernel<T, TV, NF, DM, MODE, R, false>
-        <<<G.nblocks, kBlock, 0, s>>>(a, G, static_cast<const T*>(x), dd, (T)t, gg, rs, xx);
+  auto run = [&](auto kernel) {
+    kernel<<<G.nblocks, kBlock, 0, s>>>(a, G, static_cast<const T*>(x), dd, (T)t, gg, rs, xx);
+  };
+  if (G.flat == 0) {
+    if (pf_self(rs, G.nblocks)) run(pf_tile_kernel<T, TV, NF, DM, MODE, R, true>);
+    else run(pf_tile_kernel<T, TV, NF, DM, MODE, R, false>);
+  }
+  if constexpr ((MODE & 6) == 2) {
+    if (G.flat == 1) run(pf_flat_kernel<T, TV, NF, DM, MODE, R, 1>);
+    else if (G.flat == 2) run(pf_flat_kernel<T, TV, NF, DM, MODE, R, 2>);
+  }
 }
 
 template <typename T, typename TV, int NF, int MODE>
@@ -529,7 +660,7 @@ void launch_tile_dm(const PFArgs& a, const TileGeom& G, const void* x, const voi
 template <typename T, typename TV, int NF>
 int launch_tile_nf(const PFArgs& a, int mode, const void* x, const void* d, double t, void* g, RedScratch rs,
                    hipStream_t s, void* xo) {
-  const TileGeom G = tile_geom_for<T, TV, NF>(a);
+  const TileGeom G = tile_geom_for<T, TV, NF>(a, mode);
   switch (mode) {
     case 1: launch_tile_dm<T, T, NF, 1>(a, G, x, d, t, g, rs, s, xo); break;  // no vector is touched
     case 2: launch_tile_dm<T, TV, NF, 2>(a, G, x, d, t, g, rs, s, xo); break;

@@ -15,6 +15,12 @@
 // still loads valid sites: its overhanging lanes/rows hold exactly the
 // wrapped neighbours the last in-grid sites need, and only "owned" rows are
 // stored or summed.
+//
+// Where such tiles leave many lanes outside the grid (Z just above a multiple of
+// 64), a block takes 256 R consecutive sites of the plane's linear order instead
+// (flat chunks): thread t owns sites t, t + 256, ...  Its LDS slot j holds site
+// base - Z + j of the plane (wrapped), so the y neighbours lie Z slots away and
+// the z neighbours one slot away, or Z - 1 at the ends of a grid row.
 #pragma once
 
 #ifndef MINIM_HD
@@ -37,6 +43,22 @@ struct TileGeom {
   int ntz, nty, ntile;  // tiles per plane
   int xchunk, nxc;      // x planes per block, chunks along x
   int nblocks;          // ntile * nxc, x-chunk major
+  int flat;             // 0: tiles; else flat chunks, with so many halo sites per thread
+};
+
+// Flat chunks: LDS slots for R rows and H halo sites per thread.  With H = 2 the
+// slots, not the threads, set the largest Z.
+constexpr int kFlatMaxZ = 192;
+MINIM_HD constexpr int flat_slots(int R, int H) { return kTileWaves * kTileZ * R + (H == 1 ? 256 : 2 * kFlatMaxZ); }
+
+struct FlatThread {
+  int x0, x1;                // planes [x0, x1) marched by this block
+  unsigned site[kMaxTileR];  // in-plane index of own rows, wrapped into the grid
+  int slot[kMaxTileR];       // their LDS slots
+  unsigned own;              // bit r: own row r lies inside the grid
+  int zm[kMaxTileR], zp[kMaxTileR];  // LDS slots of their z neighbours
+  unsigned hsite[2];         // halo sites this thread stages (own row 0 when none)
+  int hslot[2];              // and their slots (negative: none)
 };
 
 struct TileThread {
@@ -108,14 +130,54 @@ MINIM_HD inline void tile_thread(const TileGeom& G, int L, int t, TileThread& o)
   }
 }
 
-// Tile geometry for R rows per thread.  xchunk > 0 forces the x-march length,
+MINIM_HD inline void flat_thread(const TileGeom& G, int Lb, int t, FlatThread& o) {
+  const int T = kTileWaves * kTileZ, L = T * G.R, YZ = G.Y * G.Z;
+  const int xc = Lb / G.ntile, base = (Lb - xc * G.ntile) * L;
+  o.x0 = xc * G.xchunk;
+  o.x1 = (o.x0 + G.xchunk < G.X) ? o.x0 + G.xchunk : G.X;
+  o.own = 0;
+  for (int r = 0; r < kMaxTileR; r++) {
+    const int j = r * T + t, f = base + j, s = f % YZ, z = s % G.Z;
+    o.site[r] = (unsigned)s;
+    o.slot[r] = G.Z + j;
+    o.zm[r] = o.slot[r] + (z == 0 ? G.Z - 1 : -1);
+    o.zp[r] = o.slot[r] + (z == G.Z - 1 ? 1 - G.Z : 1);
+    if (r < G.R && f < YZ) o.own |= 1u << r;
+  }
+  for (int h = 0; h < 2; h++) {
+    const int j = h * T + t;
+    if (h < G.flat && j < 2 * G.Z) {
+      o.hslot[h] = j < G.Z ? j : L + j;
+      o.hsite[h] = (unsigned)wrap_mod(base - G.Z + o.hslot[h], YZ);
+    } else {
+      o.hslot[h] = -1;
+      o.hsite[h] = o.site[0];
+    }
+  }
+}
+
+// Flat chunks where they leave less to do: sites computed (lanes outside the
+// grid included) and sites staged count alike, and the tiles, whose y neighbours
+// come from registers, keep the grids where flat chunks save under a tenth.
+MINIM_HD inline int flat_halo(int Y, int Z, int R) {
+  if (Z > kFlatMaxZ) return 0;
+  const long L = kTileWaves * kTileZ * R, TY = kTileWaves * R;
+  const long tiles = (long)((Z + kTileZ - 1) / kTileZ) * ((Y + TY - 1) / TY);
+  const long chunks = ((long)Y * Z + L - 1) / L;
+  const long tile_cost = tiles * (kTileZ * TY + (kTileZ + 2) * (TY + 2)), flat_cost = chunks * (2 * L + 2 * Z);
+  if (10 * flat_cost >= 9 * tile_cost) return 0;
+  return Z <= 128 ? 1 : 2;
+}
+
+// Tile geometry for R rows per thread (flat: from flat_halo).  xchunk > 0 forces
+// the x-march length,
 // else the march is as short as at most target_blocks blocks allow (two per CU
 // by default: the blocks run together, and a few more than fit run after them;
 // 160x150x141x3, energy and gradient in FP64: 540 blocks 48.6 us, 480 38.8;
 // 190x180x187x3: 540 76.8, 504 62.8).  Returns false when the grid cannot be
 // launched (more than max_blocks blocks).
 MINIM_HD inline bool tile_geom(int X, int Y, int Z, int R, int xchunk, int target_blocks, int max_blocks,
-                               TileGeom& G) {
+                               TileGeom& G, int flat = 0) {
   G.X = X;
   G.Y = Y;
   G.Z = Z;
@@ -124,6 +186,11 @@ MINIM_HD inline bool tile_geom(int X, int Y, int Z, int R, int xchunk, int targe
   G.ntz = (Z + kTileZ - 1) / kTileZ;
   G.nty = (Y + G.TY - 1) / G.TY;
   G.ntile = G.ntz * G.nty;
+  G.flat = flat;
+  if (flat) {
+    const long L = kTileWaves * kTileZ * R;
+    G.ntile = (int)(((long)Y * Z + L - 1) / L);
+  }
   if (xchunk <= 0) {
     long nxc = target_blocks / G.ntile;  // at most the target: a few blocks more take a second round
     if (nxc < 1) nxc = 1;

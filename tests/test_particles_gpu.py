@@ -446,8 +446,7 @@ def test_bah_fused_step_matches_separate_passes(gpu, prec):
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 def test_bah_lbfgs_fused_step_keeps_the_trajectory(gpu, prec):
     """L-BFGS on the bar-and-hinge sheet takes its accepted first trials
-    through the fused step, which keeps the hinge store for the gradient that
-    follows.  A maxStep too large to bind runs the same algorithm through the
+    through the fused step, whose gradient follows in a pass of its own.  A maxStep too large to bind runs the same algorithm through the
     separate trial energy, axpy and gradient passes: after 300 iterations the
     coordinates, energy and evaluation counts agree bit for bit."""
     from bench import sheet_triangles

@@ -391,3 +391,33 @@ def test_autotune_general_kernel_and_vector_passes(gpu):
     e0 = m.State(plain, x).energy()
     assert abs(s2.energy() - e_ref) <= 1e-8 * max(abs(e_ref), abs(e0))
     m.autotune_clear()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("grid", [(40, 33, 97), (23, 30, 128), (30, 20, 141), (26, 41, 192), (70, 20, 15)])
+@pytest.mark.parametrize("nf,dens", [(1, "hard"), (2, "hard"), (3, "soft"), (4, "hard")])
+def test_flat_chunks(gpu, grid, nf, dens, prec):
+    """Grids whose gradient runs over flat chunks of a plane (Z up to 128 with
+    one halo site per thread, up to 192 with two, and the short rows of a plane
+    that is less than a chunk): energy and gradient against the oracle, and the
+    same gradient without the energy; the fused step, which stays on the tiles,
+    still gives the separate trial's energy and that gradient bit for bit."""
+    import torch
+
+    m = gpu
+    rng = np.random.default_rng(sum(grid) + nf)
+    n = int(np.prod(grid)) * nf
+    st, iw = ([1.0, 0.8, 1.2], [2.0]) if nf == 3 else ([1.0] * (nf if nf > 3 else 1), [1.5])
+    x = rng.uniform(-1.1, 1.1, n) if nf == 1 else rng.uniform(-0.1, 1.1, n)
+    check(m, grid, nf, st, iw, dens, x, prec)
+    dt = torch.float64 if prec == "fp64" else torch.float32
+    h = make_pf(m, grid, nf, st, iw, dens).handle(x)
+    xd = torch.tensor(x, dtype=dt, device="cuda")
+    d = torch.tensor(rng.normal(0, 0.1, n), dtype=dt, device="cuda")
+    xo, g, gr, ge = (torch.empty_like(xd) for _ in range(4))
+    e = m.potential_eval_step(h, prec, prec, xd.data_ptr(), n, d.data_ptr(), 0.75, xo.data_ptr(), g.data_ptr())
+    assert e == m.potential_eval(h, prec, xd.data_ptr(), n, d_ptr=d.data_ptr(), t=0.75)
+    m.potential_eval(h, prec, xo.data_ptr(), n, g_ptr=gr.data_ptr(), want_energy=False)
+    m.potential_eval(h, prec, xo.data_ptr(), n, g_ptr=ge.data_ptr())
+    torch.cuda.synchronize()
+    assert torch.equal(g, gr) and torch.equal(g, ge)
