@@ -72,7 +72,9 @@ Workspace::Workspace() {
   char* base = static_cast<char*>(mem_.get());
   few_ = reinterpret_cast<double*>(base + partial_bytes + result_bytes);
   tickets_ = reinterpret_cast<unsigned*>(base + partial_bytes + result_bytes + few_bytes);
-  MINIM_HIP_CHECK(hipMemset(tickets_, 0, sizeof(unsigned) * kTickets));
+  // a synchronous copy: zero before any stream's first launch counts on them
+  const unsigned zero[kTickets] = {};
+  MINIM_HIP_CHECK(hipMemcpy(tickets_, zero, sizeof(zero), hipMemcpyHostToDevice));
   rs_.partials = reinterpret_cast<double*>(base);
   rs_.result = reinterpret_cast<double*>(base + partial_bytes);
   MINIM_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_), result_bytes, hipHostMallocCoherent));
