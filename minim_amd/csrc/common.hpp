@@ -164,8 +164,12 @@ __device__ inline void finish_in_kernel(double (&v)[K], const RedScratch& rs) {
 }
 
 // All threads of the (1-D) grid must call this; v is each thread's contribution.
-template <int K, bool SELF = false>
-__device__ inline void grid_sum_store(double (&v)[K], RedScratch rs) {
+// RS: RedScratch, or Partials for kernels that need no more of it.
+struct Partials {
+  double* partials;
+};
+template <int K, bool SELF = false, typename RS>
+__device__ inline void grid_sum_store(double (&v)[K], const RS& rs) {
   __shared__ double lds[(kBlock / kWave) * (K > 0 ? K : 1)];
   block_sum<K>(v, lds);
   if constexpr (SELF) {

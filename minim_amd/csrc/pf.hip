@@ -217,7 +217,8 @@ __device__ __forceinline__ void resolve_plane(PlaneIn<T, TV, NF, R, DIR, H>& p, 
 template <typename T, typename TV, int NF, int DM, int MODE, int R, bool SELF>
 __global__ __launch_bounds__(kBlock) void pf_tile_kernel(PFArgs a, TileGeom G, const T* __restrict__ x,
                                                          const TV* __restrict__ d, T t, TV* __restrict__ g,
-                                                         RedScratch rs, T* __restrict__ xo) {
+                                                         std::conditional_t<SELF, RedScratch, Partials> rs,
+                                                         T* __restrict__ xo) {
   constexpr bool WE = MODE & 1, WG = MODE & 2, DIR = MODE & 4, XW = (MODE & 8) && DIR;
   constexpr int LH = kTileWaves * R + 2, LW = kTileZ + 2;
   __shared__ T lds[2][LH][LW][NF];
@@ -626,16 +627,16 @@ void launch_tile(const PFArgs& a, const TileGeom& G, const void* x, const void* 
   const TV* dd = static_cast<const TV*>((MODE & 4) ? d : x);
   TV* gg = static_cast<TV*>((MODE & 2) ? g : const_cast<void*>(x));
   T* xx = static_cast<T*>((MODE & 8) ? xo : const_cast<void*>(x));
-  auto run = [&](auto kernel) {
-    kernel<<<G.nblocks, kBlock, 0, s>>>(a, G, static_cast<const T*>(x), dd, (T)t, gg, rs, xx);
+  auto run = [&](auto kernel, const auto& r) {
+    kernel<<<G.nblocks, kBlock, 0, s>>>(a, G, static_cast<const T*>(x), dd, (T)t, gg, r, xx);
   };
   if (G.flat == 0) {
-    if (pf_self(rs, G.nblocks)) run(pf_tile_kernel<T, TV, NF, DM, MODE, R, true>);
-    else run(pf_tile_kernel<T, TV, NF, DM, MODE, R, false>);
+    if (pf_self(rs, G.nblocks)) run(pf_tile_kernel<T, TV, NF, DM, MODE, R, true>, rs);
+    else run(pf_tile_kernel<T, TV, NF, DM, MODE, R, false>, Partials{rs.partials});
   }
   if constexpr ((MODE & 6) == 2) {
-    if (G.flat == 1) run(pf_flat_kernel<T, TV, NF, DM, MODE, R, 1>);
-    else if (G.flat == 2) run(pf_flat_kernel<T, TV, NF, DM, MODE, R, 2>);
+    if (G.flat == 1) run(pf_flat_kernel<T, TV, NF, DM, MODE, R, 1>, rs);
+    else if (G.flat == 2) run(pf_flat_kernel<T, TV, NF, DM, MODE, R, 2>, rs);
   }
 }
 
