@@ -464,9 +464,9 @@ void PhaseFieldUnstructured::init(const vector<double>& coords) {
   // no soft constraint but the three-fluid one, every element's contribution
   // to a site follows from the concentrations around it, and the device
   // gathers the elements per site (pfu_site_kernel): 128x112x120x3 FP64 energy
-  // and gradient 156 us through the list, 21.7 us per site (FP32: 130 and 16.4
-  // us); 700x900x1x2 FP64 43 and 10.8 us.  Fluid counts and planes as the tiled
-  // kernel takes them.
+  // and gradient 156 us through the list, 21.1 us per site (FP32: 130 and 16.4
+  // us); 700x900x1x2 FP64 43 and 10.8 us.  Grids whose planes the kernel cannot
+  // cover in one launch (pfu_site_fits) keep the list.
   bool anySolid = false, surfaces = false, forces = false, confined = false;
   for (size_t i = 0; i < ng; i++) {
     anySolid |= solid[i] != 0;
@@ -476,10 +476,11 @@ void PhaseFieldUnstructured::init(const vector<double>& coords) {
     forces |= fMag[f] > 0;
     confined |= confinementStrength[f] != 0;
   }
+  int canon[3], cmap[3];
+  pf_canonical(gridSize.data(), canon, cmap);
   const bool gather = nF <= 4 && densityConstraint != minim_amd::kDensityFixed &&
                       (densityConstraint != minim_amd::kDensitySoft || nF == 1 || nF == 3) && !forces && !confined &&
-                      !(surfaces && nF == 1) &&
-                      8.0 * nF * ((double)gridSize[1] * gridSize[2]) < 4294967296.0;
+                      !(surfaces && nF == 1) && minim_amd::pfu_site_fits(canon, nF, anySolid);
   RefElements el;
   auto push = [&el](int t, std::initializer_list<int32_t> ids, std::initializer_list<double> par) {
     el.push(t, ids, par);
@@ -544,8 +545,6 @@ void PhaseFieldUnstructured::init(const vector<double>& coords) {
   if (ng * (size_t)nF >= ((size_t)1 << 31)) throw std::invalid_argument("PhaseFieldUnstructured: more than 2^31 DOFs");
   if (nElements >= ((size_t)1 << 32)) throw std::invalid_argument("PhaseFieldUnstructured: more than 2^32 elements");
   if (gather) {
-    int canon[3], cmap[3];
-    pf_canonical(gridSize.data(), canon, cmap);
     minim_amd::PFUArgs& u = h->u;
     u.gather = 1;
     u.X = canon[0];

@@ -439,7 +439,7 @@ __device__ __forceinline__ void site_elements(const PFUArgs& u, const PFArgs& co
 // a 64 x 4R (z, y) tile through a two-plane LDS ring, the loads of plane i+2
 // in flight while plane i is computed; own columns and x neighbours stay in
 // registers.  Bound by memory: 128x112x120x3, energy and gradient with the
-// reduction, FP64 21.7 us = 3.8 TB/s of concentrations in and gradient out,
+// reduction, FP64 21.1 us = 3.9 TB/s of concentrations in and gradient out,
 // FP32 16.4 us; the list form, which reads 16 bytes and issues some 200
 // instructions per element, took 156 and 130 us there.  Gradient error against
 // 64 bits 1.53e-16 (list 1.59e-16) and 2.8e-8 in FP32 (list 5.5e-8).
@@ -722,7 +722,29 @@ void eval_t(const PFUArgs& u, const PFArgs& con, int mode, const void* x, const 
   if ((mode & 2) && (!u.gather || u.volfix)) pf_launch_constrain(con, sizeof(T) == 8 ? F64 : F32, gg, u.ngrid, rs, s);
 }
 
+// The fewest rows per thread (so the most tiles) of the two precisions.
+template <int NF>
+constexpr int least_rows(bool solid) {
+  constexpr int a = std::min(site_rows<double, NF, true>(), site_rows<float, NF, true>());
+  constexpr int b = std::min(site_rows<double, NF, false>(), site_rows<float, NF, false>());
+  return solid ? a : b;
+}
+
 }  // namespace
+
+bool pfu_site_fits(const int canon[3], int nf, bool solid) {
+  if ((double)canon[1] * canon[2] * nf * sizeof(double) >= 4294967296.0) return false;
+  int R;
+  switch (nf) {
+    case 1: R = least_rows<1>(solid); break;
+    case 2: R = least_rows<2>(solid); break;
+    case 3: R = least_rows<3>(solid); break;
+    case 4: R = least_rows<4>(solid); break;
+    default: return false;
+  }
+  TileGeom G;
+  return tile_geom(canon[0], canon[1], canon[2], R, 0, kSiteTargetBlocks, kMaxRedBlocks, G);
+}
 
 void pfu_launch_eval(const PFUArgs& u, const PFArgs& con, int prec, int mode, const void* x, const void* d, double t,
                      void* g, RedScratch rs, hipStream_t s, double* eOut) {

@@ -69,6 +69,11 @@ struct PFUArgs {
 // x + t*d.  prec is the storage precision of x, d and g.
 void pfu_launch_eval(const PFUArgs& u, const PFArgs& con, int prec, int mode, const void* x, const void* d, double t,
                      void* g, RedScratch rs, hipStream_t s, double* eOut = nullptr);
+// The per-site kernel can launch the canonical grid, in either precision: its
+// blocks cover whole x chunks of a tile, so all tiles of a plane have to fit in
+// one launch (kMaxRedBlocks) and a plane in 32-bit byte offsets.  The list has
+// neither limit.
+bool pfu_site_fits(const int canon[3], int nf, bool solid);
 // Average duration (ms) of reps launches of the element kernel (with the
 // gather pass of the shared sites when mode has the gradient).
 double pfu_time_elements(const PFUArgs& u, const PFArgs& con, int prec, int mode, const void* x, void* g, int reps, RedScratch rs,

@@ -380,3 +380,32 @@ def test_elements_gathered_per_site_vs_oracle(gpu, grid, nf, density, layout, pr
     assert rel_err(g.cpu().numpy(), o.gradient(x)) <= TOL[prec]
     for got, at in ((e, x), (et, x + 0.5 * d)):
         assert abs(got - o.energy(at)) <= TOL[prec] * max(energy_scale(c, at), abs(o.energy(at)))
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("grid,nf,wall", [((524289, 1, 1), 1, False), ((65537, 2, 1), 2, True)])
+def test_planes_beyond_one_per_site_launch_vs_oracle(gpu, grid, nf, wall, prec):
+    """One tile more than the per-site kernel can launch: the list takes the
+    call, as it takes every size."""
+    import torch
+
+    m = gpu
+    print("case pfu large plane", grid, nf, prec, flush=True)
+    rng = np.random.default_rng(nf)
+    n = int(np.prod(grid)) * nf
+    x = rng.uniform(0, 1, n).astype(np.float32).astype(np.float64)
+    opts = {}
+    if wall:
+        opts["solid"] = (np.arange(n // nf) < 2).astype(np.uint8)
+    c = dict(grid=grid, nfluid=nf, resolution=1.0, surface_tension=[1.0], interface_size=[1.5], density="hard",
+             opts=opts, x0=x)
+    o = oracle_of(c)
+    h = device_pf(m, c, "PhaseFieldUnstructured").handle(x)
+    dt = torch.float64 if prec == "fp64" else torch.float32
+    xd = torch.tensor(x, dtype=dt, device="cuda")
+    g = torch.empty_like(xd)
+    e = m.potential_eval(h, prec, xd.data_ptr(), n, g_ptr=g.data_ptr())
+    torch.cuda.synchronize()
+    eo = o.energy(x)
+    assert abs(e - eo) <= TOL[prec] * max(1.0, abs(eo))  # every term is positive
+    assert rel_err(g.cpu().numpy(), o.gradient(x)) <= TOL[prec]

@@ -49,3 +49,21 @@ def test_element_form_rejects_what_it_cannot_hold():
         base().setContactAngle([90.0] * 24).nElements(x)
     with pytest.raises(NotImplementedError):
         base().energyComponents(x)
+
+
+# The per-site kernel covers a plane of the canonical grid (64 sites by 16 or 8
+# rows a tile) in one launch of at most 8,192 blocks, in either precision.
+@pytest.mark.parametrize("grid,nf,solid,per_site", [
+    ((524288, 1, 1), 1, False, True), ((524289, 1, 1), 1, False, False),
+    ((1, 131072, 2), 3, False, True), ((131073, 2, 1), 3, False, False),
+    ((65536, 1, 2), 4, False, True), ((65537, 1, 2), 4, False, False),
+    ((65536, 2, 1), 2, True, True), ((65537, 2, 1), 2, True, False),
+])
+def test_list_kept_where_the_per_site_kernel_cannot_launch(grid, nf, solid, per_site):
+    n = int(np.prod(grid))
+    pf = m.PhaseFieldUnstructured().setNFluid(nf).setGridSize(list(grid))
+    if solid:
+        pf.setSolid((np.arange(n) < 2).astype(np.uint8))
+    elements, size = pf.elementList(np.full(n * nf, 0.5))
+    assert elements == (n - 2 * solid) * nf
+    assert (size < 16 * elements) == per_site  # a list record has 16 bytes
