@@ -17,6 +17,8 @@
 #include <stdexcept>
 #include <string>
 
+#include "arrival.hpp"
+
 namespace minim_amd {
 
 constexpr int kBlock = 256;          // threads per block (4 wavefronts of 64)
@@ -24,6 +26,7 @@ constexpr int kWave = 64;
 constexpr int kMaxRedBlocks = 8192;  // upper bound on blocks of any reducing launch
 constexpr int kMaxDots = 96;         // upper bound on values reduced by one launch
 constexpr int kSelfBlocks = kWave;    // largest launch that finishes its own reduction
+static_assert(kSelfBlocks <= (int)kArrivals, "one lane and one arrival per block");
 // Result slot of a deferred validity flag (Potential::gradientDeferred): the
 // last one, written by that launch and read by the caller's next fetch.
 constexpr int kDeferSlot = kMaxDots - 1;
@@ -97,7 +100,7 @@ struct RedScratch {
   double* partials;  // [kMaxDots][kMaxRedBlocks], value k of block b at k * gridDim + b
   double* result;    // [kMaxDots]
   double* mirror = nullptr;   // the same values in pinned host memory, for Workspace::fetch
-  unsigned* ticket = nullptr; // arrivals of this launch (zero before and after), or null: two stages only
+  unsigned* ticket = nullptr; // this launch's arrival counter (arrival.hpp), or null: two stages only
   double* few = nullptr;      // its partials, [kMaxDots][kSelfBlocks]
   double* copy = nullptr;     // value copyK goes there too (a caller's device slot)
   int copyK = -1;
@@ -134,7 +137,8 @@ __device__ inline void finish_in_kernel(double (&v)[K], const RedScratch& rs) {
     for (int k = 0; k < K; k++)
       __hip_atomic_store(&rs.few[(size_t)k * nb + blockIdx.x], v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    last = __hip_atomic_fetch_add(rs.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)nb - 1;
+    const unsigned w = arrival_weight(nb, blockIdx.x);
+    last = arrival_last(__hip_atomic_fetch_add(rs.ticket, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), w);
   }
   __syncthreads();
   if (!last) return;
@@ -160,7 +164,6 @@ __device__ inline void finish_in_kernel(double (&v)[K], const RedScratch& rs) {
       if (k == rs.copyK) *rs.copy = s[j];
     }
   }
-  if (threadIdx.x == 0) __hip_atomic_store(rs.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // All threads of the (1-D) grid must call this; v is each thread's contribution.

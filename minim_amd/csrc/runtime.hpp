@@ -57,9 +57,12 @@ class Workspace {
   ~Workspace();
   Workspace(const Workspace&) = delete;
   Workspace& operator=(const Workspace&) = delete;
-  // The scratch for one launch (or several in stream order): each call hands out
-  // the next of kTickets arrival counters with its partials, so that launches on
-  // several streams do not count together.
+  // The scratch for one launch (or several in stream order).  Partials, results
+  // and mirror are those of the host thread, which may have one stream at work at
+  // a time.  Each call hands out the next of kTickets arrival counters with its
+  // partials: should a thread's launches overlap all the same (a captured graph
+  // replayed beside eager calls), those on one counter spoil each other's sums,
+  // and the counter is good again after them (arrival.hpp).
   RedScratch rs();
   // Wait for stream s and copy result[0..k) into out.  Whatever writes a result
   // slot on the device also writes its mirror in pinned host memory, so no copy

@@ -37,3 +37,15 @@ def test_flat_mapping(tmp_path):
     r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     print(r.stdout[-2000:])
     assert r.returncode == 0, r.stdout[-2000:]
+
+
+def test_arrival_counts(tmp_path):
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    exe = str(tmp_path / "arrival_check")
+    subprocess.run([cxx, "-O2", "-std=c++17", "-I", os.path.join(ROOT, "minim_amd", "csrc"),
+                    os.path.join(HERE, "arrival_check.cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    print(r.stdout[-2000:])
+    assert r.returncode == 0, r.stdout[-2000:]
