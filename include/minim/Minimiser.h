@@ -183,7 +183,7 @@ class Lbfgs : public NewMinimiser<Lbfgs> {
   struct Impl;
   std::unique_ptr<Impl> impl_;
   struct BatchMem;
-  std::shared_ptr<BatchMem> _batchMem;  // minimiseBatch's memory; a copy has its own
+  std::shared_ptr<BatchMem> _batchMem;  // minimiseBatch's memory (2 GiB at most); a copy has its own
 };
 
 class Fire : public NewMinimiser<Fire> {

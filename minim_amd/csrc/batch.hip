@@ -1245,8 +1245,12 @@ namespace minim {
 // Device and pinned memory, stream and events of minimiseBatch: kept by the
 // Lbfgs for its next call (each buffer grows to the largest batch seen, and all
 // go with the object), because allocating and freeing some twenty of them took
-// a fifth of a short batch.  One call at a time, as for the rest of an Lbfgs.
+// a fifth of a short batch.  A call takes them for itself and puts them back when
+// its work is done: a call meanwhile, or after one that ended by an exception,
+// allocates its own.  Above kKeep they are freed with the call, as a batch of that
+// size (16 M sites at m = 5) runs for much longer than that takes.
 struct Lbfgs::BatchMem {
+  static constexpr size_t kKeep = size_t(2) << 30;
   int device = -1;
   static constexpr int kDev = 18, kPin = 5;
   minim_amd::DeviceBuffer buf[kDev];
@@ -1267,6 +1271,11 @@ struct Lbfgs::BatchMem {
   }
   BatchMem(const BatchMem&) = delete;
   BatchMem& operator=(const BatchMem&) = delete;
+  size_t deviceBytes() const {
+    size_t n = 0;
+    for (const auto& b : buf) n += b.bytes();
+    return n;
+  }
   minim_amd::DeviceBuffer& dev(int i, size_t bytes) {
     if (buf[i].bytes() < bytes) buf[i].reset(bytes);
     return buf[i];
@@ -1400,8 +1409,23 @@ std::vector<MinimiseStats> Lbfgs::batchRun(const std::vector<State*>& states, in
   const int S = _m + 1;
   int device = 0;
   MINIM_HIP_CHECK(hipGetDevice(&device));
-  if (!_batchMem || _batchMem->device != device) _batchMem = std::make_shared<BatchMem>(device);
-  BatchMem& W = *_batchMem;
+  auto mem = std::atomic_exchange(&_batchMem, std::shared_ptr<BatchMem>());
+  if (!mem || mem->device != device) mem = std::make_shared<BatchMem>(device);
+  struct Lease {
+    std::shared_ptr<BatchMem>& mem;
+    std::shared_ptr<BatchMem>& keeper;
+    hipStream_t st;
+    bool done = false;  // nothing is queued any more
+    ~Lease() {
+      if (!done) {  // an exception: what is queued still uses the memory and this call's tables
+        (void)hipStreamSynchronize(mem->stream);
+        (void)hipStreamSynchronize(st);
+      } else if (mem->deviceBytes() <= BatchMem::kKeep) {
+        std::atomic_store(&keeper, mem);
+      }
+    }
+  } lease{mem, _batchMem, st};
+  BatchMem& W = *mem;
   DeviceBuffer &Xa = W.dev(0, N * 8), &Xb = W.dev(1, N * 8), &G0 = W.dev(2, N * vb), &G1 = W.dev(3, N * vb),
                &Dm = W.dev(4, N * vb * S), &Ym = W.dev(5, N * vb * S);
   // per-phase staging, one copy per phase: block prefix sums, then the BDyn of
@@ -2101,6 +2125,7 @@ std::vector<MinimiseStats> Lbfgs::batchRun(const std::vector<State*>& states, in
   batchReport.block = block;
   if (!writeBack) {
     MINIM_HIP_CHECK(hipStreamSynchronize(st));
+    lease.done = true;
     return {};
   }
   for (int j = 0; j < ni; j++) {
@@ -2114,6 +2139,7 @@ std::vector<MinimiseStats> Lbfgs::batchRun(const std::vector<State*>& states, in
   }
   copyCoords(false);
   MINIM_HIP_CHECK(hipStreamSynchronize(st));
+  lease.done = true;
   stats = MinimiseStats{};
   iter = maxIters;
   return out;
