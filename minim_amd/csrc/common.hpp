@@ -42,9 +42,11 @@ struct HipError : std::runtime_error {
 #define MINIM_HIP_CHECK(expr)                                                                  \
   do {                                                                                         \
     hipError_t _e = (expr);                                                                    \
-    if (_e != hipSuccess)                                                                      \
+    if (_e != hipSuccess) {                                                                    \
+      (void)hipGetLastError(); /* reported here, not by the next launch's check */             \
       throw ::minim_amd::HipError(std::string("HIP error ") + hipGetErrorString(_e) + " at " + \
                                   __FILE__ + ":" + std::to_string(__LINE__) + " (" #expr ")"); \
+    }                                                                                          \
   } while (0)
 
 // ---------------------------------------------------------------- reductions

@@ -781,10 +781,15 @@ void rebuild_list(LjNd::Impl& I, int prec, const void* x, const void* d, double 
   I.builds++;
 }
 
-// Rows for lists of up to longest entries; the list is built again after.
+// Rows for lists of up to longest entries; the list is built again after.  Where
+// the memory does not suffice (an exception), there are no rows and no list: the
+// next evaluation builds one that outgrows them, and comes here again.
 void grow_list(LjNd::Impl& I, int N, int longest) {
-  I.maxn = (longest + 2 * minim_amd::kListPad - 1) / minim_amd::kListPad * minim_amd::kListPad;
-  I.nbr.reset(sizeof(int) * minim_amd::nbr_elems(N, I.maxn));
+  const int maxn = (longest + 2 * minim_amd::kListPad - 1) / minim_amd::kListPad * minim_amd::kListPad;
+  I.built = false;
+  I.maxn = 0;
+  I.nbr.reset(sizeof(int) * minim_amd::nbr_elems(N, maxn));
+  I.maxn = maxn;
   I.builds--;
 }
 

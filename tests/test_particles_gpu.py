@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from conftest import golden
+from minim_amd._capi import MinimError
 from oracle_bind import OracleBaH, OracleLJ, OracleLJPBC, oracle_fire, oracle_lbfgs
 
 pytestmark = pytest.mark.gpu
@@ -599,3 +600,23 @@ def test_lj_list_longer_than_its_rows(gpu, prec):
         tol = 1e-12 if prec == "fp64" else 1e-4
         assert abs(e - o.energy(x)) <= tol * abs(o.energy(x)) + tol
         assert rel_err(g, o.gradient(x)) <= tol
+
+
+def test_lj_list_that_does_not_fit_in_memory(gpu):
+    """Lists that would take 410 GB (320,000 particles, all within the list
+    radius of each other): every evaluation fails with the allocation's error,
+    and the next one of another system is as good as ever."""
+    m = gpu
+    rng = np.random.default_rng(8)
+    n, L = 320000, 10.0
+    s = m.State(m.Lj3d().setCutoff(5.0, [L] * 3, 4.0), rng.uniform(0, L, 3 * n), "fp32")
+    for k in range(3):
+        print("evaluation", k, flush=True)
+        with pytest.raises(MinimError, match="memory"):
+            s.energyGradient()
+    del s
+    x = lattice(4, 1.1, 0.05, rng)
+    o = OracleLJPBC(64, 5.0, 2.5)
+    e, g = m.State(m.Lj3d().setCutoff(2.5, [5.0] * 3, 0.3), x).energyGradient()
+    assert abs(e - o.energy(x)) <= 1e-12 * abs(o.energy(x))
+    assert rel_err(g, o.gradient(x)) <= 1e-12
