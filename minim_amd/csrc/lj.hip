@@ -13,6 +13,7 @@
 // list; the list is rebuilt when any particle has moved more than skin/2 from
 // where the list was built.  Lists are built deterministically (cell contents
 // sorted by particle id), so energies and gradients are reproducible.
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <stdexcept>
@@ -52,11 +53,16 @@ __device__ inline void load_pos(const T* __restrict__ x, const T* __restrict__ d
 // FP64, so the gradient's error against 64 bits fell too (1,000 particles,
 // 3-D: 1.2e-15 -> 6e-16 in FP64, 1.1e-6 -> 7.6e-7 in FP32).  MODE bit 1
 // energy, bit 2 gradient.
+//
+// s2: 4^-k with 2^k <= sigma < 2^(k+1), and sig6 the sixth power of sigma / 2^k,
+// so that 1 / r^6 stays in range wherever (sigma / r)^6 does (a power of two
+// rounds nothing); where r^4 does not, the pair's force is zero.
 template <typename T, int D, int R, int MODE>
 __global__ __launch_bounds__(kBlock) void lj_allpairs_kernel(const T* __restrict__ x, const T* __restrict__ d, T t,
-                                                             int N, T sig6, T eps, T* __restrict__ g,
+                                                             int N, T sig6, T eps, T s2, T* __restrict__ g,
                                                              RedScratch rs) {
   constexpr bool WE = MODE & 1, WG = MODE & 2;
+  constexpr T most = sizeof(T) == 8 ? (T)1.79769313486231571e308 : (T)3.40282347e38f;
   constexpr int U = 4;  // positions requested before any is used
   __shared__ double lds[(kBlock / kWave) * (WG ? R * D : 1)];
   const int ngroup = (N + R - 1) / R;
@@ -87,13 +93,13 @@ __global__ __launch_bounds__(kBlock) void lj_allpairs_kernel(const T* __restrict
             r2 = fma(dx[k], dx[k], r2);
           }
           if (j == i || i >= N) continue;
-          const T r4 = r2 * r2;
-          const T ir6 = (T)1 / (r4 * r2);  // one division per pair
+          const T q2 = s2 * r2, q4 = q2 * q2;
+          const T ir6 = (T)1 / (q4 * q2);  // one division per pair
           const T lj6 = sig6 * ir6;
           const T lj12 = lj6 * lj6;
           if (WE) ei += 0.5 * (double)((T)4 * eps * (lj12 - lj6));
           if (WG) {
-            const T f = (T)-24 * eps * ((T)2 * lj12 - lj6) * (ir6 * r4);
+            const T f = (T)-24 * eps * s2 * ((T)2 * lj12 - lj6) * (ir6 * fmin(q4, most));
 #pragma unroll
             for (int k = 0; k < D; k++) gi[r][k] = fma(dx[k], f, gi[r][k]);
           }
@@ -523,15 +529,15 @@ __global__ __launch_bounds__(kBlock) void lj_cut_kernel(const T* __restrict__ x,
 }
 
 template <typename T, int D>
-int launch_allpairs_d(const T* x, const T* d, T t, int N, T sig6, T eps, int mode, T* g, RedScratch rs,
+int launch_allpairs_d(const T* x, const T* d, T t, int N, T sig6, T eps, T s2, int mode, T* g, RedScratch rs,
                       hipStream_t s) {
   auto go = [&](auto rtag) {
     constexpr int R = decltype(rtag)::value;
     const int nb = grid_blocks((size_t)((N + R - 1) / R) * kBlock);
     switch (mode) {
-      case 1: lj_allpairs_kernel<T, D, R, 1><<<nb, kBlock, 0, s>>>(x, d, t, N, sig6, eps, g, rs); break;
-      case 2: lj_allpairs_kernel<T, D, R, 2><<<nb, kBlock, 0, s>>>(x, d, t, N, sig6, eps, g, rs); break;
-      default: lj_allpairs_kernel<T, D, R, 3><<<nb, kBlock, 0, s>>>(x, d, t, N, sig6, eps, g, rs); break;
+      case 1: lj_allpairs_kernel<T, D, R, 1><<<nb, kBlock, 0, s>>>(x, d, t, N, sig6, eps, s2, g, rs); break;
+      case 2: lj_allpairs_kernel<T, D, R, 2><<<nb, kBlock, 0, s>>>(x, d, t, N, sig6, eps, s2, g, rs); break;
+      default: lj_allpairs_kernel<T, D, R, 3><<<nb, kBlock, 0, s>>>(x, d, t, N, sig6, eps, s2, g, rs); break;
     }
     return nb;
   };
@@ -549,14 +555,15 @@ void launch_allpairs(int D, const void* x, const void* d, double t, int N, doubl
   const T* xx = (const T*)x;
   const T* dd = (const T*)d;
   T* gg = (T*)g;
-  const T sig6 = (T)std::pow(sigma, 6), tt = (T)t, ee = (T)eps;
+  const int k = sigma != 0 && std::isfinite(sigma) ? std::max(-60, std::min(60, std::ilogb(sigma))) : 0;
+  const T sig6 = (T)std::pow(std::ldexp(sigma, -k), 6), s2 = (T)std::ldexp(1.0, -2 * k), tt = (T)t, ee = (T)eps;
   rs = rs.only(0, (mode & 1) ? eDev : nullptr);
   int nb = 0;
   switch (D) {
-    case 1: nb = launch_allpairs_d<T, 1>(xx, dd, tt, N, sig6, ee, mode, gg, rs, s); break;
-    case 2: nb = launch_allpairs_d<T, 2>(xx, dd, tt, N, sig6, ee, mode, gg, rs, s); break;
-    case 3: nb = launch_allpairs_d<T, 3>(xx, dd, tt, N, sig6, ee, mode, gg, rs, s); break;
-    case 4: nb = launch_allpairs_d<T, 4>(xx, dd, tt, N, sig6, ee, mode, gg, rs, s); break;
+    case 1: nb = launch_allpairs_d<T, 1>(xx, dd, tt, N, sig6, ee, s2, mode, gg, rs, s); break;
+    case 2: nb = launch_allpairs_d<T, 2>(xx, dd, tt, N, sig6, ee, s2, mode, gg, rs, s); break;
+    case 3: nb = launch_allpairs_d<T, 3>(xx, dd, tt, N, sig6, ee, s2, mode, gg, rs, s); break;
+    case 4: nb = launch_allpairs_d<T, 4>(xx, dd, tt, N, sig6, ee, s2, mode, gg, rs, s); break;
     default: throw std::invalid_argument("LjNd: nDim must be 1..4 on the device path");
   }
   MINIM_HIP_CHECK(hipGetLastError());

@@ -620,3 +620,24 @@ def test_lj_list_that_does_not_fit_in_memory(gpu):
     e, g = m.State(m.Lj3d().setCutoff(2.5, [5.0] * 3, 0.3), x).energyGradient()
     assert abs(e - o.energy(x)) <= 1e-12 * abs(o.energy(x))
     assert rel_err(g, o.gradient(x)) <= 1e-12
+
+
+@pytest.mark.parametrize("prec,sigma,eps,x", [
+    ("fp32", 1.0, 1.0, [0.0, 1.1, 1e10]),        # r^4 out of range
+    ("fp64", 1.0, 1.0, [0.0, 1.1, 1e80]),
+    ("fp32", 5e-7, 2.0, [0.0, 3.7e-7, 1.1e-6]),  # 1 / r^6 out of range, (sigma / r)^6 not
+    ("fp32", 3e9, 0.5, [0.0, 2.7e9, 9e9]),
+    ("fp32", 3.4e-10, 1.65e-21, [0.0, 3.7e-10, 8e-10]),
+])
+def test_lj_all_pairs_range(gpu, prec, sigma, eps, x):
+    """Separations and units whose powers leave the range of the type, while
+    (sigma / r)^6 and the forces stay within it."""
+    m = gpu
+    x = np.array(x) if prec == "fp64" else r32(x)
+    s = m.State(m.LjNd(1).setSigma(sigma).setEpsilon(eps), x, prec)
+    e, g = s.energyGradient()
+    dx = x[:, None] - x[None, :]
+    np.fill_diagonal(dx, np.inf)
+    q = (sigma / dx) ** 6
+    assert e == pytest.approx(2 * eps * (q * q - q).sum(), rel=TOL[prec])
+    assert rel_err(g, (-24 * eps * (2 * q * q - q) / dx).sum(axis=1)) <= TOL[prec]
