@@ -477,7 +477,7 @@ __global__ __launch_bounds__(kBlock) void lj_cut_kernel(const T* __restrict__ x,
           pairs += in;
         }
         if (WG) {
-          const T f = fma((T)2 * lj6, lj6, -lj6) * ir2;
+          const T f = fma((T)2 * lj6, lj6, -lj6) * s2;  // in units of epsilon and sigma: in range as lj6^2 is
           gi[0] = fma(r0, f, gi[0]);
           gi[1] = fma(r1, f, gi[1]);
           gi[2] = fma(r2v, f, gi[2]);
@@ -500,7 +500,7 @@ __global__ __launch_bounds__(kBlock) void lj_cut_kernel(const T* __restrict__ x,
       }
       if (dr2 > b.half_skin2) moved = 1.0;
       if (WG) {
-        const T f = (T)(-24 * eps);
+        const T f = (T)(-24 * eps / (double)sig2);
 #pragma unroll
         for (int k = 0; k < 3; k++) {
           const T gk = f * gi[k];

@@ -641,3 +641,21 @@ def test_lj_all_pairs_range(gpu, prec, sigma, eps, x):
     q = (sigma / dx) ** 6
     assert e == pytest.approx(2 * eps * (q * q - q).sum(), rel=TOL[prec])
     assert rel_err(g, (-24 * eps * (2 * q * q - q) / dx).sum(axis=1)) <= TOL[prec]
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_lj_cutoff_range(gpu, prec):
+    """Argon in SI units with a pair at 0.02 sigma: (sigma / r)^12 / r^2 leaves
+    FP32's range, the force (3e12 N) does not."""
+    m = gpu
+    sigma, eps, rc, L = 3.4e-10, 1.65e-21, 8.5e-10, 5e-9
+    x = r32([0, 0, 0, 6.8e-12, 0, 0, 2e-9, 0, 0, 2.4e-9, 0, 0])
+    s = m.State(m.Lj3d().setSigma(sigma).setEpsilon(eps).setCutoff(rc, [L] * 3, 1e-10), x, prec)
+    e, g = s.energyGradient()
+    r = np.array([x[3], x[9] - x[6]])
+    q, qc = (sigma / r) ** 6, (sigma / rc) ** 6
+    f = 24 * eps * (2 * q * q - q) / r
+    assert e == pytest.approx(4 * eps * (q * q - q - (qc * qc - qc)).sum(), rel=TOL[prec])
+    gx = g.reshape(-1, 3)[:, 0]
+    np.testing.assert_allclose(gx, [f[0], -f[0], f[1], -f[1]], rtol=10 * TOL[prec])
+    assert not g.reshape(-1, 3)[:, 1:].any()
