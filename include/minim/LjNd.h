@@ -64,6 +64,7 @@ class LjNd : public NewPotential<LjNd> {
 
  private:
   std::shared_ptr<Impl> impl_;  // device neighbour-list state (rebuilt lazily)
+  bool plain() const;
   void launch(int prec, const void* x, const void* d, double t, bool wantE, double* eDev, void* g,
               void* stream) const;
 };

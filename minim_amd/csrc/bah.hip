@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <cmath>
 #include <stdexcept>
+#include <typeinfo>
 
 #include "bah_mesh.hpp"
 #include "common.hpp"
@@ -778,13 +779,16 @@ void launch_bah(const BarAndHinge::Dev& dv, int prec, int pv, const void* x, con
 }
 }  // namespace
 
-// The node flags hold every constraint (none was added since the upload, and
-// none reads the coordinates): the kernel zeroes the fixed components itself.
-bool BarAndHinge::maskHolds() const { return constraints.size() == dev_->nFixed && !hasNormalConstraints(); }
+// The node flags hold every constraint (none was added since the upload, none
+// reads the coordinates, and no derived class has its own): the kernel zeroes the
+// fixed components itself.
+bool BarAndHinge::maskHolds() const {
+  return constraints.size() == dev_->nFixed && !hasNormalConstraints() && typeid(*this) == typeid(BarAndHinge);
+}
 
 void BarAndHinge::evaluate(int prec, const void* x, const void* d, double t, double* e, void* g,
                            void* stream) const {
-  evaluateAsync(prec, x, d, t, e != nullptr, nullptr, g, stream);
+  BarAndHinge::evaluateAsync(prec, x, d, t, e != nullptr, nullptr, g, stream);
   if (e) {
     double r[1];
     minim_amd::Workspace::current().fetch(static_cast<hipStream_t>(stream), 1, r);

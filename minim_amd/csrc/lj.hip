@@ -18,6 +18,7 @@
 #include <cmath>
 #include <stdexcept>
 #include <type_traits>
+#include <typeinfo>
 #include <vector>
 
 #include "common.hpp"
@@ -859,8 +860,15 @@ void LjNd::evaluate(int prec, const void* x, const void* d, double t, double* e,
   }
 }
 
+// A class derived from these may have its own evaluate or constraints, which the
+// general paths call.
+bool LjNd::plain() const {
+  return typeid(*this) == typeid(LjNd) || typeid(*this) == typeid(Lj2d) || typeid(*this) == typeid(Lj3d);
+}
+
 void LjNd::evaluateAsync(int prec, const void* x, const void* d, double t, bool wantE, double* e_dev, void* g,
                          void* stream) const {
+  if (!plain()) return Potential::evaluateAsync(prec, x, d, t, wantE, e_dev, g, stream);
   if (!impl_) throw std::runtime_error("LjNd: not initialised (construct a State first).");
   if (wantE || g) launch(prec, x, d, t, wantE, e_dev, g, stream);
 }
@@ -903,7 +911,7 @@ void LjNd::redoGradient(int prec, const void* x, void* g, void* stream) const {
 // Cutoff mode without constraints: the force pass has each particle's force in
 // registers, so that FIRE's dots and largest force need no pass of their own.
 bool LjNd::fusesFire(int dim) const {
-  return cutoff > 0 && constraints.empty() && (dim == 0 || dim == 3) &&
+  return plain() && cutoff > 0 && constraints.empty() && (dim == 0 || dim == 3) &&
          cut_blocks(nParticle) <= minim_amd::kMaxRedBlocks;
 }
 

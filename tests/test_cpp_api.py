@@ -12,14 +12,14 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(ROOT, "minim_amd")
 
 
-def build(tmp_path):
+def build(tmp_path, source="cpp_api_example"):
     cxx = shutil.which("g++")
     if cxx is None:
         pytest.skip("g++ not available")
     if not os.path.exists(os.path.join(LIB, "libminim_amd.so")):
         pytest.fail("libminim_amd.so is not built")
-    exe = str(tmp_path / "cpp_api_example")
-    cmd = [cxx, "-std=c++17", "-O1", os.path.join(ROOT, "tests", "cpp_api_example.cpp"), "-I",
+    exe = str(tmp_path / source)
+    cmd = [cxx, "-std=c++17", "-O1", os.path.join(ROOT, "tests", source + ".cpp"), "-I",
            os.path.join(ROOT, "include"), "-L", LIB, "-lminim_amd", "-Wl,-rpath," + LIB, "-o", exe]
     subprocess.run(cmd, check=True, capture_output=True, text=True, timeout=300)
     return exe
@@ -36,4 +36,10 @@ def test_cpp_api_compiles_links_and_sets_up(tmp_path):
 def test_cpp_api_minimises_on_the_gpu(gpu, tmp_path):
     exe = build(tmp_path)
     r = subprocess.run([exe, "gpu"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_derived_potentials_keep_their_own_evaluations(tmp_path):
+    exe = build(tmp_path, "subclass_check")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
