@@ -844,7 +844,10 @@ void BarAndHinge::evaluateStepAsync(int px, int pv, const void* x, const void* d
     const auto a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
     return p && q && a < b + n3 * bq && b < a + n3 * bp;
   };
-  if (overlap(xout, bx, x, bx) || overlap(xout, bx, d, bv) || overlap(g, bv, x, bx) || overlap(g, bv, d, bv)) {
+  const bool scales = xout == x && d == x && px == pv;  // x = x + t*x
+  if ((overlap(xout, bx, d, bv) && !scales) || overlap(xout, bx, g, bv) || (xout != x && overlap(xout, bx, x, bx)))
+    throw std::invalid_argument("BarAndHinge: x + t*d must go to x or to memory of its own.");
+  if (xout == x || overlap(g, bv, x, bx) || overlap(g, bv, d, bv)) {
     // a cluster reads x and d at its neighbours' nodes too: with an output over
     // an input, the point is formed first
     if (xout != x) minim_amd::device_copy(xout, x, n3 * bx, s);

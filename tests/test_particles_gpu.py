@@ -659,3 +659,45 @@ def test_lj_cutoff_range(gpu, prec):
     gx = g.reshape(-1, 3)[:, 0]
     np.testing.assert_allclose(gx, [f[0], -f[0], f[1], -f[1]], rtol=10 * TOL[prec])
     assert not g.reshape(-1, 3)[:, 1:].any()
+
+
+def test_bah_step_overlaps(gpu):
+    """Where the fused step's outputs may lie over its inputs it gives what it
+    gives in memory of its own, and it refuses the rest, touching nothing."""
+    import torch
+    from bench import sheet_triangles
+
+    m = gpu
+    nside, t = 12, 0.5
+    rng = np.random.default_rng(3)
+    i, j = np.meshgrid(np.arange(nside), np.arange(nside), indexing="ij")
+    x0 = np.stack([0.95 * (i - 0.5 * j), (np.sqrt(3) / 2) * j, rng.normal(0, 0.1, i.shape)], -1).reshape(-1)
+    n = x0.size
+    h = (m.BarAndHinge().setTriangulation(sheet_triangles(nside, nside)).setRigidity(1.0, 0.01).setLength0(1.0)
+         .setTheta0(np.pi).handle(x0))
+    v = [x0, rng.normal(0, 0.01, n)]
+
+    def run(x, d, xo, g):  # offsets in one buffer of 6 n
+        b = torch.full((6 * n,), 7.0, dtype=torch.float64, device="cuda")
+        b[x:x + n] = torch.tensor(v[0])
+        if d != x:
+            b[d:d + n] = torch.tensor(v[1])
+        before = b.clone()
+        p = b.data_ptr()
+        try:
+            e = m.potential_eval_step(h, "fp64", "fp64", p + 8 * x, n, p + 8 * d, t, p + 8 * xo, p + 8 * g)
+        except ValueError:
+            assert torch.equal(b, before)
+            return None
+        return e, b[xo:xo + n].clone(), b[g:g + n].clone()
+
+    def same(a, b):
+        return a[0] == b[0] and torch.equal(a[1], b[1]) and torch.equal(a[2], b[2])
+
+    want = run(0, n, 2 * n, 3 * n)
+    for args in ((0, n, 0, 3 * n), (0, n, 2 * n, 0), (0, n, 2 * n, n), (0, n, 0, n), (n, 3 * n, 5 * n, n + 3)):
+        assert same(run(*args), want), args
+    assert same(run(0, 0, 0, 3 * n), run(0, 0, 2 * n, 3 * n))  # x = x + t x
+    for args in ((0, n, n, 3 * n), (0, n, n - 3, 3 * n), (0, n, 2 * n, 2 * n), (0, n, 2 * n, 3 * n - 3),
+                 (0, 4 * n, 3, 2 * n), (3, 4 * n, 0, 2 * n)):
+        assert run(*args) is None, args
