@@ -108,7 +108,7 @@ class PhaseField : public NewPotential<PhaseField> {
   // take precedence.  The shape changes the tiling only: gradients are the
   // same bit for bit.
   std::vector<std::array<double, 3>> autotune(const vector<double>& coords, int prec,
-                                              vector<int> targets = {256, 512, 1024, 2048},
+                                              vector<int> targets = {256, 512, 768, 1024, 2048},
                                               vector<int> marches = {0, 4, 8, 16, 32}, int reps = 10);
   // The tuned (target blocks, x-march) for a precision; (0, 0) = the heuristic.
   std::pair<int, int> tunedShape(int prec) const;
@@ -139,9 +139,10 @@ class PhaseField : public NewPotential<PhaseField> {
   vector<double> fMag;
   vector2d<double> fNorm;
 
-  // Launch tuning: x-march length of the stencil and target block count
-  // (0 = automatic for both); stencilKernel 1 forces the general kernel
-  // (solid-aware, every term) where the tiled one would run.
+  // Launch tuning: x-march length of the stencil and target block count (blocks
+  // at most, where a whole march per tile is not more; 0 = automatic for both);
+  // stencilKernel 1 forces the general kernel (solid-aware, every term) where
+  // the tiled one would run.
   int stencilXChunk = 0;
   int stencilTargetBlocks = 0;
   int stencilKernel = 0;

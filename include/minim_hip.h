@@ -52,7 +52,7 @@ typedef struct minim_pf_params {
   double density_const;
   const unsigned char* fix_fluid; /* NULL or n_fluid flags (setFixFluid) */
   int stencil_xchunk;             /* 0 = automatic x-march length */
-  int stencil_target_blocks;      /* 0 = automatic */
+  int stencil_target_blocks;      /* blocks at most, where a whole x march per tile is not more; 0 = automatic */
   /* The remaining terms (PhaseField.h:36-68, PhaseField.cpp:818-895); NULL / 0
    * leaves a setter uncalled.  n_surface_tension may also be
    * ngrid * n_fluid: per-site tensions. */

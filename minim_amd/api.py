@@ -261,7 +261,7 @@ class PhaseField(Potential):
 
     COMPONENTS = ("fluid", "surface", "pressure", "density constraint", "force", "confinement", "volume constraint")
 
-    def autotune(self, coords, precision="fp32", blocks=(256, 512, 1024, 2048), marches=(0, 4, 8, 16, 32), reps=10):
+    def autotune(self, coords, precision="fp32", blocks=(256, 512, 768, 1024, 2048), marches=(0, 4, 8, 16, 32), reps=10):
         """Launch-shape autotuner of the evaluation kernel this field uses
         (PhaseField::autotune, minim_pf_autotune): one energy+gradient launch
         (HIP events, kernel only) is timed for every pair of target block count

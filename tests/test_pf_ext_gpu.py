@@ -375,3 +375,32 @@ def test_general_kernel_full_size_256cubed_pillars(gpu):
         es = max(1.0, sum(abs(v[0]) for v in o.components(x).values()))
         assert abs(e - eo) <= tol * es, (prec, e, eo)
         assert rel_err(g.double().cpu().numpy(), go) <= tol, prec
+
+
+def test_launch_shapes_asked_for_are_launched(gpu):
+    """The general kernel at a grid where the automatic shape is three blocks
+    per CU: a target or a tuned shape of 512 blocks is launched as such.  (The
+    energy's partial sums tell the shapes apart: bit for bit those of the same
+    march given as a length, and not those of the automatic shape.)"""
+    m = gpu
+    m.autotune_clear()
+    grid = (160, 150, 141)
+    rng = np.random.default_rng(6)
+    u = rng.uniform(0, 1, (int(np.prod(grid)), 3))
+    x = (u / u.sum(axis=1, keepdims=True)).reshape(-1)
+
+    def energy(target=0, march=0):
+        pf = m.PhaseField().setNFluid(3).setGridSize(list(grid)).setInterfaceSize(2.0)
+        pf.stencilKernel, pf.stencilTargetBlocks, pf.stencilXChunk = 1, target, march
+        s = m.State(pf, x)
+        return [s.energy(f * x) for f in np.linspace(0.5, 1.0, 8)]
+
+    automatic, by_march = energy(), energy(march=20)  # 57 tiles of 8 marches
+    assert energy(target=512) == by_march
+    assert automatic != by_march
+    assert energy(target=768) == automatic
+    pf = m.PhaseField().setNFluid(3).setGridSize(list(grid)).setInterfaceSize(2.0)
+    pf.stencilKernel = 1
+    pf.autotune(x, "fp64", blocks=(512,), marches=(0,), reps=1)
+    assert energy() == by_march
+    m.autotune_clear()
