@@ -69,6 +69,7 @@ class BarAndHinge : public NewPotential<BarAndHinge> {
   vector<double> kBond_, kHinge_, length0_, theta0_, force_;
   std::shared_ptr<Dev> dev_;
   std::shared_ptr<const vector<int>> order_;  // the nodes in cluster order
+  bool tablesStale_ = false;                  // a setter was called since the tables were made
   void upload();
   bool maskHolds() const;
 };

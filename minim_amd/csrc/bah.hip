@@ -415,50 +415,62 @@ using minim_amd::kBlock;
 
 struct BarAndHinge::Dev {
   minim_amd::BaHArgs args{};
-  DeviceBuffer mem;
-  size_t nFixed = 0;  // single-DOF constraints that the node flags hold
+  std::shared_ptr<DeviceBuffer> mem, ht0;  // the tables; rest angles that were set one by one
+  std::vector<int> hinge;                  // the hinge of each record
+  std::vector<int> fixed;                  // the single-DOF constraints that the tables are for
+  size_t nFixed = 0;                       // constraints that the node flags hold
 };
 
 BarAndHinge& BarAndHinge::setTriangulation(const vector2d<int>& triList) {
   tri_ = triList;
+  tablesStale_ = true;
   return *this;
 }
 BarAndHinge& BarAndHinge::setBondList(const vector2d<int>& b) {
   bonds_ = b;
+  tablesStale_ = true;
   return *this;
 }
 BarAndHinge& BarAndHinge::setHingeList(const vector2d<int>& h) {
   hinges_ = h;
+  tablesStale_ = true;
   return *this;
 }
 BarAndHinge& BarAndHinge::setRigidity(double kb, double kh) {
   kBond_ = {kb};
   kHinge_ = {kh};
+  tablesStale_ = true;
   return *this;
 }
 BarAndHinge& BarAndHinge::setRigidity(const vector<double>& kb, const vector<double>& kh) {
   if (!kb.empty()) kBond_ = kb;
   if (!kh.empty()) kHinge_ = kh;
+  tablesStale_ = true;
   return *this;
 }
 BarAndHinge& BarAndHinge::setLength0(double l) {
   length0_ = {l};
+  tablesStale_ = true;
   return *this;
 }
 BarAndHinge& BarAndHinge::setLength0(const vector<double>& l) {
   length0_ = l;
+  tablesStale_ = true;
   return *this;
 }
 BarAndHinge& BarAndHinge::setTheta0(double t) {
   theta0_ = {t};
+  tablesStale_ = true;
   return *this;
 }
 BarAndHinge& BarAndHinge::setTheta0(const vector<double>& t) {
   theta0_ = t;
+  tablesStale_ = true;
   return *this;
 }
 BarAndHinge& BarAndHinge::setForce(const vector<double>& f) {
   force_ = f;
+  tablesStale_ = true;
   return *this;
 }
 
@@ -637,9 +649,33 @@ void BarAndHinge::init(const vector<double>& coords) {
   upload();
 }
 
+// With tables on the device that are for these lists and constraints, only the
+// angle's records change, in a copy of the angles (a copy of this potential may
+// share them): at 150^2 nodes 0.1 ms, all tables anew 11.
 void BarAndHinge::setHingeTheta0(int iHinge, double t0) {
   theta0_.at(iHinge) = t0;
-  if (dev_) upload();
+  if (!dev_) return;
+  if (tablesStale_ || dev_->fixed != fixedDofs() || dev_->nFixed != constraints.size()) {
+    upload();
+    return;
+  }
+  const size_t n = dev_->hinge.size();
+  if (n == 0) return;
+  auto dev = std::make_shared<Dev>(*dev_);
+  dev->ht0 = std::make_shared<DeviceBuffer>(sizeof(double) * n);
+  double* to = static_cast<double*>(dev->ht0->get());
+  if (dev_->args.ht0) {
+    MINIM_HIP_CHECK(hipMemcpy(to, dev_->args.ht0, sizeof(double) * n, hipMemcpyDeviceToDevice));
+  } else {
+    const std::vector<double> all(n, dev_->args.ht0U);
+    MINIM_HIP_CHECK(hipMemcpy(to, all.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+  }
+  for (size_t r = 0; r < n; r++)
+    if (dev->hinge[r] == iHinge)
+      MINIM_HIP_CHECK(hipMemcpy(to + r, &t0, sizeof(double), hipMemcpyHostToDevice));
+  MINIM_HIP_CHECK(hipStreamSynchronize(nullptr));  // other streams read the angles next
+  dev->args.ht0 = to;
+  dev_ = dev;
 }
 
 void BarAndHinge::upload() {
@@ -654,7 +690,7 @@ void BarAndHinge::upload() {
     return true;
   };
   auto dev = std::make_shared<Dev>();
-  std::vector<int> bar, hin;
+  std::vector<int> bar, hin, hinId;
   std::vector<double> bk, bl, hk, ht;
   bar.reserve(2 * bonds_.size());
   hin.reserve(4 * hinges_.size());
@@ -669,6 +705,7 @@ void BarAndHinge::upload() {
     int nd[4] = {hinges_[i][0], hinges_[i][1], hinges_[i][2], hinges_[i][3]};
     if (allFixed(nd, 4)) continue;
     hin.insert(hin.end(), nd, nd + 4);
+    hinId.push_back((int)i);
     hk.push_back(kHinge_[i]);
     ht.push_back(theta0_[i]);
   }
@@ -688,6 +725,9 @@ void BarAndHinge::upload() {
     if (!allFixed(&n, 1)) flags[o] |= minim_amd::kForced;
   }
   dev->nFixed = constraints.size();
+  dev->fixed = fixedDofs();
+  dev->hinge.reserve(mesh.hingeId.size());
+  for (int h : mesh.hingeId) dev->hinge.push_back(hinId[h]);
   // parameters shared by every element go as scalars, others per bar code and hinge record
   auto uniform = [](const std::vector<double>& v) {
     for (double x : v)
@@ -717,8 +757,8 @@ void BarAndHinge::upload() {
                i_hinge = reserve(mesh.hinge), i_bcode = reserve(mesh.bcode),
                i_hcode = reserve(mesh.hcode), i_bk = reserve(bkR), i_bl = reserve(blR), i_hk = reserve(hkR),
                i_ht = reserve(htR), i_fz = reserve(fz), i_flags = reserve(flags);
-  dev->mem.reset(off + 256);
-  char* base = static_cast<char*>(dev->mem.get());
+  dev->mem = std::make_shared<DeviceBuffer>(off + 256);
+  char* base = static_cast<char*>(dev->mem->get());
   for (size_t i = 0; i < src.size(); i++)
     if (src[i].second) MINIM_HIP_CHECK(hipMemcpy(base + at[i], src[i].first, src[i].second, hipMemcpyHostToDevice));
   auto dptr = [&](size_t i) { return (const double*)(src[i].second ? base + at[i] : nullptr); };
@@ -743,6 +783,7 @@ void BarAndHinge::upload() {
   a.fz = dptr(i_fz);
   a.flags = (const unsigned char*)(base + at[i_flags]);
   dev_ = dev;
+  tablesStale_ = false;
 }
 
 namespace {

@@ -28,6 +28,7 @@
 #include <cstdint>
 #include <future>
 #include <stdexcept>
+#include <system_error>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -80,16 +81,32 @@ struct BaHMesh {
 
 namespace bah_mesh {
 
-// f(range) on contiguous ranges of [0, n), in parallel when there is enough work.
+// f() on a thread of its own, or where there is none to be had when it is waited for.
+template <typename F>
+inline std::future<void> start(F f) {
+  try {
+    return std::async(std::launch::async, f);
+  } catch (const std::system_error&) {
+    return std::async(std::launch::deferred, f);
+  }
+}
+
+// f(range) on contiguous ranges of [0, n), in parallel.
 template <typename F>
 inline void ranges(int n, int parts, F f) {
   std::vector<std::future<void>> job;
-  for (int p = 1; p < parts; p++)
-    job.push_back(std::async(std::launch::async, f, p, (int)((long long)n * p / parts),
-                             (int)((long long)n * (p + 1) / parts)));
+  for (int p = 1; p < parts; p++) {
+    const int a = (int)((long long)n * p / parts), b = (int)((long long)n * (p + 1) / parts);
+    job.push_back(start([=] { f(p, a, b); }));
+  }
   f(0, 0, (int)((long long)n / parts));
   for (auto& j : job) j.get();
 }
+
+// Threads for the tables of n nodes: one takes about 0.4 us a node, and starting
+// one some 30 us.
+constexpr int kPerThread = 512;
+inline int threads_for(int n) { return std::max(1, std::min(8, n / kPerThread)); }
 
 struct Point {
   float c[3];
@@ -118,8 +135,8 @@ inline void bisect(Point* p, long long n, int m, int m0, int m1, int threads) {
     std::nth_element(a, c, b, [ax](const Point& u, const Point& v) {
       return u.c[ax] != v.c[ax] ? u.c[ax] < v.c[ax] : u.id < v.id;
     });
-  if (threads > 1 && b - a > 8192) {
-    auto left = std::async(std::launch::async, bisect, p, n, m, m0, mid, threads / 2);
+  if (threads > 1 && b - a > 2 * kPerThread) {
+    auto left = start([=] { bisect(p, n, m, m0, mid, threads / 2); });
     bisect(p, n, m, mid, m1, threads - threads / 2);
     left.get();
   } else {
@@ -127,8 +144,6 @@ inline void bisect(Point* p, long long n, int m, int m0, int m1, int threads) {
     bisect(p, n, m, mid, m1, 1);
   }
 }
-
-inline int threads_for(size_t work) { return work > (size_t(1) << 16) ? 8 : 1; }
 
 // Nodes in cluster order; part k of m holds [n k / m, n (k + 1) / m).
 inline std::vector<int> order(const std::vector<double>& coords, int m) {

@@ -43,3 +43,10 @@ def test_derived_potentials_keep_their_own_evaluations(tmp_path):
     exe = build(tmp_path, "subclass_check")
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.gpu
+def test_hinge_angles_set_one_by_one(gpu, tmp_path):
+    exe = build(tmp_path, "hinge_angle_check")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
