@@ -701,3 +701,94 @@ def test_bah_step_overlaps(gpu):
     for args in ((0, n, n, 3 * n), (0, n, n - 3, 3 * n), (0, n, 2 * n, 2 * n), (0, n, 2 * n, 3 * n - 3),
                  (0, 4 * n, 3, 2 * n), (3, 4 * n, 0, 2 * n)):
         assert run(*args) is None, args
+
+
+def fire_replay(m, h, prec, x, steps, dt0, dt_max):
+    """FIRE without line search (Fire.cpp:41-84) in torch around potential_eval's
+    gradients: coordinates and gradient after the steps."""
+    import torch
+
+    g = torch.empty_like(x)
+
+    def gradient():
+        m.potential_eval(h, prec, x.data_ptr(), x.numel(), g_ptr=g.data_ptr(), want_energy=False)
+        torch.cuda.synchronize()
+
+    def dot(a, b):
+        return float((a.double() * b.double()).sum())
+
+    v, a, dt, n = torch.zeros_like(x), 0.1, dt0, 0
+    gradient()
+    for _ in range(steps):
+        p = -dot(v, g)
+        if p > 0:
+            v = (1 - a) * v - (a * math.sqrt(dot(v, v)) / math.sqrt(dot(g, g)) + dt) * g
+            n += 1
+            if n > 5:
+                a, dt = a * 0.99, min(dt * 1.1, dt_max)
+        else:
+            v = -dt * g
+            n, a, dt = 0, 0.1, dt * 0.5
+        x += dt * v
+        gradient()
+    return x, g
+
+
+# sides: 16 lanes per particle in the force pass and the list build, 4 and 8, 1 and 8
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("side,dim", [(9, 3), (9, 0), (26, 3), (41, 0)])
+def test_fused_fire_vs_replay(gpu, side, dim, prec):
+    """Forty fused steps with a skin that forces cell-list rebuilds against the
+    replay: the gradients are the same kernels' and the sums differ in order
+    only, so the steps' factors agree to a few units in the last place of their
+    type; forty steps of the crystal amplify that by less than 1e3."""
+    import torch
+
+    m = gpu
+    print("case fused fire", side, dim, prec, flush=True)
+    a, steps = 0.85 ** (-1 / 3), 40
+    x0 = r32(lattice(side, a, 0.12, np.random.default_rng(side)))
+    dt = torch.float64 if prec == "fp64" else torch.float32
+    pot = m.Lj3d().setCutoff(2.5, [side * a] * 3, 0.1)
+    s = m.State(pot, x0, prec)
+    s.convergence = 1e-30
+    f = m.Fire(0.02).setDt0(0.004).setMaxIter(steps - 1)
+    if dim:
+        f.setMaxForceConvergence(dim)
+    x = f.minimise(s)
+    assert pot.listBuilds(s) >= 3
+    xr, gr = fire_replay(m, pot.handle(x0), prec, torch.tensor(x0, dtype=dt, device="cuda"), steps, 0.004, 0.02)
+    xr, gr = xr.double().cpu().numpy(), gr.double().cpu().numpy()
+    tol = 1e3 * (2.0 ** -52 if prec == "fp64" else 2.0 ** -23)
+    assert np.linalg.norm(x - xr) <= tol * np.linalg.norm(xr - x0)
+    assert f.stats["grad_rms"] == pytest.approx(math.sqrt((gr * gr).mean()), rel=tol)
+    if dim:
+        assert f.stats["grad_max"] == pytest.approx(np.linalg.norm(gr.reshape(-1, 3), axis=1).max(), rel=tol)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("L", [11.0, 12.0])
+def test_fused_fire_list_outgrows_its_rows(gpu, L, prec):
+    """A stretched crystal of 343 particles that contracts: lists of at most 122
+    entries at first (rows hold 128), over 128 when one is built again under
+    way, in brute-force (L = 11, fewer than three cells a side) and cell mode."""
+    import torch
+
+    m = gpu
+    print("case fused fire rows", L, prec, flush=True)
+    a, rc, skin, steps = 1.25, 3.675, 0.2, 80
+    x0 = r32(lattice(7, a, 0.005, np.random.default_rng(5)))
+    p = x0.reshape(-1, 3)
+    d = p[:, None] - p[None]
+    d -= L * np.rint(d / L)
+    assert ((d * d).sum(-1) < (rc + skin) ** 2).sum(1).max() - 1 <= 128
+    dt = torch.float64 if prec == "fp64" else torch.float32
+    pot = m.Lj3d().setCutoff(rc, [L] * 3, skin)
+    s = m.State(pot, x0, prec)
+    s.convergence = 1e-30
+    x = m.Fire(0.02).setDt0(0.01).setMaxIter(steps - 1).minimise(s)
+    assert pot.maxNeighbours(s) > 128
+    xr, _ = fire_replay(m, pot.handle(x0), prec, torch.tensor(x0, dtype=dt, device="cuda"), steps, 0.01, 0.02)
+    xr = xr.double().cpu().numpy()
+    tol = 1e3 * (2.0 ** -52 if prec == "fp64" else 2.0 ** -23)
+    assert np.linalg.norm(x - xr) <= tol * np.linalg.norm(xr - x0)
