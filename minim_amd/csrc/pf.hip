@@ -601,14 +601,16 @@ TileGeom tile_geom_for(const PFArgs& a, int mode) {
                                                          : kTileTargetBlocks;
   const int xo = user ? a.xchunk_override : a.tuned_xchunk[pi];
   constexpr int R = tile_rows<T, NF>();
-  if (!tile_geom(a.X, a.Y, a.Z, R, xo, target, kMaxRedBlocks, G))
+  const int busy = user || a.tuned_target[pi] > 0 ? 0 : march_busy(NF * sizeof(T));
+  if (!tile_geom(a.X, a.Y, a.Z, R, xo, target, kMaxRedBlocks, G, 0, busy))
     throw std::invalid_argument("PhaseField: grid too large for one launch");
   // flat chunks for gradients at x (with or without the energy) that more than
   // kSelfBlocks blocks share.  Energies alone read two neighbours of a site and
   // gain nothing, and the fused step sums its energy as the trials do.
   TileGeom F;
   if ((mode & 6) == 2 && G.nblocks > kSelfBlocks &&
-      tile_geom(a.X, a.Y, a.Z, R, xo, target, kMaxRedBlocks, F, flat_halo(a.Y, a.Z, R)) && F.nblocks > kSelfBlocks)
+      tile_geom(a.X, a.Y, a.Z, R, xo, target, kMaxRedBlocks, F, flat_halo(a.Y, a.Z, R), busy) &&
+      F.nblocks > kSelfBlocks)
     G = F;
   if ((double)a.Y * a.Z * NF * sizeof(T) >= 4294967296.0)
     throw std::invalid_argument("PhaseField: one x plane of the grid exceeds 4 GiB");

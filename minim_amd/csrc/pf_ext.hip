@@ -876,9 +876,10 @@ int ext_tile_full(const PFArgs& a, int mode, const void* x, const void* d, doubl
                      : (!user && a.tuned_target[pi] > 0) ? a.tuned_target[pi]
                                                          : kExtTileTarget;
   const int xo = user ? a.xchunk_override : a.tuned_xchunk[pi];
-  if (!tile_geom(a.X, a.Y, a.Z, R, xo, target, kMaxRedBlocks, G))
+  const bool automatic = !user && a.tuned_target[pi] <= 0 && xo <= 0;
+  if (!tile_geom(a.X, a.Y, a.Z, R, xo, target, kMaxRedBlocks, G, 0, automatic ? march_busy(NF * sizeof(T)) : 0))
     throw std::invalid_argument("PhaseField: grid too large for one launch");
-  if (R == 2 && sizeof(T) * NF <= 24 && !user && a.tuned_target[pi] <= 0 && xo <= 0) {
+  if (R == 2 && sizeof(T) * NF <= 24 && automatic) {
     // no shape asked for, and three blocks of two rows per thread fit on a CU: as
     // many, where they fill
     // their places better than two do (160x150x141x3 in FP64: 456 of 512 places

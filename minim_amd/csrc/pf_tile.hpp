@@ -169,15 +169,24 @@ MINIM_HD inline int flat_halo(int Y, int Z, int R) {
   return Z <= 128 ? 1 : 2;
 }
 
+// Blocks per CU, in quarters, below which the march does not keep the chip busy, by
+// the bytes of a site: a lane of a one-fluid field has little to do per plane.
+MINIM_HD constexpr int march_busy(int siteBytes) { return siteBytes <= 4 ? 11 : siteBytes <= 8 ? 10 : 8; }
+
 // Tile geometry for R rows per thread (flat: from flat_halo).  xchunk > 0 forces
-// the x-march length,
-// else the march is as short as at most target_blocks blocks allow (two per CU
-// by default: the blocks run together, and a few more than fit run after them;
-// 160x150x141x3, energy and gradient in FP64: 540 blocks 48.6 us, 480 38.8;
-// 190x180x187x3: 540 76.8, 504 62.8).  Returns false when the grid cannot be
-// launched (more than max_blocks blocks).
+// the x-march length, else the march is as short as at most target_blocks blocks
+// allow (two per CU by default), or, with busy (from march_busy), one chunk
+// more where that takes the fullest CU less time: its blocks, but busy / 4 of
+// them at least, times their planes and six more for the start of the march.
+// Energy and gradient, one chunk fewer and one more: 160x150x141x3 in FP64 480
+// blocks 38.8 us, 540 48.6; 190x180x187x3 504 62.8, 540 76.8; 64x320x896x3 280
+// blocks 251, 560 216; 40x512x576x1 in FP32 288 blocks 40.9, 576 25.9.  Over 2,455
+// launches of one to four fluids, 0.25 to 22 M sites, the choice is 0.1 % off the
+// better one in the mean (2.2 % for at most, 9.6 % for at least the target) and
+// 14 % at worst (65, 40).  Returns false when the grid cannot be launched (more
+// than max_blocks blocks).
 MINIM_HD inline bool tile_geom(int X, int Y, int Z, int R, int xchunk, int target_blocks, int max_blocks,
-                               TileGeom& G, int flat = 0) {
+                               TileGeom& G, int flat = 0, int busy = 0) {
   G.X = X;
   G.Y = Y;
   G.Z = Z;
@@ -192,10 +201,20 @@ MINIM_HD inline bool tile_geom(int X, int Y, int Z, int R, int xchunk, int targe
     G.ntile = (int)(((long)Y * Z + L - 1) / L);
   }
   if (xchunk <= 0) {
-    long nxc = target_blocks / G.ntile;  // at most the target: a few blocks more take a second round
+    long nxc = target_blocks / G.ntile;
     if (nxc < 1) nxc = 1;
     if (nxc > X) nxc = X;
     xchunk = (int)((X + nxc - 1) / nxc);
+    if (busy > 0 && nxc < X && G.ntile < target_blocks && target_blocks % G.ntile != 0) {
+      const long CUs = 256;
+      long cost[2];
+      int chunk[2] = {xchunk, (int)((X + nxc) / (nxc + 1))};
+      for (int k = 0; k < 2; k++) {
+        const long blocks = (long)G.ntile * ((X + chunk[k] - 1) / chunk[k]), quarters = 4 * ((blocks + CUs - 1) / CUs);
+        cost[k] = (quarters > busy ? quarters : busy) * (chunk[k] + 6);
+      }
+      if (cost[1] < cost[0]) xchunk = chunk[1];
+    }
   }
   if (xchunk > X) xchunk = X;
   if (xchunk < 1) xchunk = 1;

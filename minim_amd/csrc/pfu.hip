@@ -573,7 +573,7 @@ int launch_site_solid(const PFUArgs& u, const PFArgs& con, const T* x, const T* 
                       hipStream_t s) {
   constexpr int R = site_rows<T, NF, SOLID>();
   TileGeom G;
-  if (!tile_geom(u.X, u.Y, u.Z, R, 0, kSiteTargetBlocks, kMaxRedBlocks, G))
+  if (!tile_geom(u.X, u.Y, u.Z, R, 0, kSiteTargetBlocks, kMaxRedBlocks, G, 0, march_busy(NF * sizeof(T))))
     throw std::invalid_argument("PhaseFieldUnstructured: grid too large for one launch");
   pfu_site_kernel<T, NF, MODE, R, SOLID><<<G.nblocks, kBlock, 0, s>>>(u, con, G, x, d, t, g, rs);
   return G.nblocks;

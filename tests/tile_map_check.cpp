@@ -17,9 +17,9 @@
 
 using namespace minim_amd;
 
-static int check_shape(int X, int Y, int Z, int R, int xchunk, int target) {
+static int check_shape(int X, int Y, int Z, int R, int xchunk, int target, int busy = 0) {
   TileGeom G;
-  if (!tile_geom(X, Y, Z, R, xchunk, target, 8192, G)) {
+  if (!tile_geom(X, Y, Z, R, xchunk, target, 8192, G, 0, busy)) {
     std::printf("shape %dx%dx%d R=%d: rejected\n", X, Y, Z, R);
     return 1;
   }
@@ -114,7 +114,25 @@ int main() {
         for (int target : {1, 512}) {
           fails += check_shape(s[0], s[1], s[2], R, xc, target);
           n++;
+          for (int busy : {march_busy(4), march_busy(24)}) {
+            fails += check_shape(s[0], s[1], s[2], R, xc, target, busy);
+            n++;
+          }
         }
+  // the choice between one chunk fewer and one more, as measured
+  const struct {
+    int X, Y, Z, R, bytes, blocks;
+  } choice[] = {{256, 256, 256, 4, 12, 512}, {160, 150, 141, 4, 24, 480}, {190, 180, 187, 4, 24, 504},
+                {64, 320, 896, 4, 24, 560},  {24, 640, 640, 4, 12, 400},  {40, 512, 576, 4, 4, 576}};
+  for (const auto& c : choice) {
+    TileGeom G;
+    tile_geom(c.X, c.Y, c.Z, c.R, 0, 512, 8192, G, 0, march_busy(c.bytes));
+    if (G.nblocks != c.blocks) {
+      std::printf("%dx%dx%d: %d blocks, not %d\n", c.X, c.Y, c.Z, G.nblocks, c.blocks);
+      fails++;
+    }
+    n++;
+  }
   std::printf("%d cases, %d failed\n", n, fails);
   return fails ? 1 : 0;
 }
