@@ -154,17 +154,22 @@ __global__ __launch_bounds__(kBlock) void lj_cell_index_kernel(const T* __restri
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= N) return;
   int c[3];
+  bool lost = false;
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     const double v = (double)x[(size_t)i * 3 + k];
     xbuild[(size_t)i * 3 + k] = v;
     double w = v - b.L[k] * floor(v / b.L[k]);  // wrapped into [0, L)
+    lost = lost || !isfinite(w);
     int ci = (int)(w * b.inv_cell[k]);
     if (ci >= b.nc[k]) ci = b.nc[k] - 1;
     if (ci < 0) ci = 0;
     c[k] = ci;
   }
-  const int id = (c[0] * b.nc[1] + c[1]) * b.nc[2] + c[2];
+  int id = (c[0] * b.nc[1] + c[1]) * b.nc[2] + c[2];
+  // no pair of such a particle is within the list radius: any cell will do, and
+  // all of a diverged system in one would be sorted and paired there
+  if (lost) id = i % (b.nc[0] * b.nc[1] * b.nc[2]);
   cell[i] = id;
   atomicAdd(&count[id], 1);
 }
@@ -217,17 +222,17 @@ __global__ __launch_bounds__(kBlock) void lj_fill_kernel(const int* __restrict__
 __device__ __forceinline__ double wrap_box(double v, double L) { return v - L * floor(v / L); }
 
 // Sort each cell's members by particle id so the neighbour order is
-// reproducible: one wavefront per cell; with up to 64 members each lane
-// holds one and computes its rank by comparing with the others (ids are
-// distinct, so the ranks are a permutation); larger cells are sorted by one
-// lane with an insertion sort.  The members' positions go out in that order,
-// wrapped into the box, each with its particle id: xc[p] = (x, y, z, j) (FP64,
-// the list is built in FP64 in either precision), so that the list build reads
-// one contiguous 32-byte entry per candidate instead of an index and then three
-// scattered coordinates.
+// reproducible: one wavefront per cell; a lane computes the rank of a member by
+// comparing it with all others (ids are distinct, so the ranks are a
+// permutation), with up to 64 members from registers.  The members' positions go
+// out in that order, wrapped into the box, each with its particle id: xc[p] =
+// (x, y, z, j) (FP64, the list is built in FP64 in either precision), so that the
+// list build reads one contiguous 32-byte entry per candidate instead of an
+// index and then three scattered coordinates.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void lj_sort_cells_kernel(const T* __restrict__ x, BoxArgs b,
-                                                               const int* __restrict__ start, int* order, int ncell,
+                                                               const int* __restrict__ start,
+                                                               const int* __restrict__ order, int ncell,
                                                                double4* __restrict__ xc) {
   const int lane = threadIdx.x % kWave;
   const int c = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
@@ -242,17 +247,13 @@ __global__ __launch_bounds__(kBlock) void lj_sort_cells_kernel(const T* __restri
     int rank = 0;
     for (int q = 0; q < k; q++) rank += __shfl(v, q, kWave) < v ? 1 : 0;
     if (lane < k) put(lo + rank, v);
-  } else if (lane == 0) {
-    for (int a = lo + 1; a < hi; a++) {
-      int v = order[a];
-      int q = a - 1;
-      while (q >= lo && order[q] > v) {
-        order[q + 1] = order[q];
-        q--;
-      }
-      order[q + 1] = v;
+  } else {
+    for (int a = lane; a < k; a += kWave) {
+      const int v = order[lo + a];
+      int rank = 0;
+      for (int q = 0; q < k; q++) rank += order[lo + q] < v ? 1 : 0;
+      put(lo + rank, v);
     }
-    for (int p = lo; p < hi; p++) put(p, order[p]);
   }
 }
 
@@ -768,7 +769,7 @@ void rebuild_list(LjNd::Impl& I, int prec, const void* x, const void* d, double 
       minim_amd::lj_fill_kernel<<<nb, kBlock, 0, s>>>((const int*)I.cell.get(), N, (const int*)I.start.get(),
                                                       (int*)I.cursor.get(), (int*)I.order.get());
       minim_amd::lj_sort_cells_kernel<T><<<nbc, kBlock, 0, s>>>(xx, I.box, (const int*)I.start.get(),
-                                                                (int*)I.order.get(), I.ncell, xc);
+                                                                (const int*)I.order.get(), I.ncell, xc);
       auto build = [&](auto kernel, int lanes) {
         kernel<<<(int)(((size_t)N * lanes + kBlock - 1) / kBlock), kBlock, 0, s>>>(
             N, I.box, (const int*)I.cell.get(), (const int*)I.start.get(), xc, I.maxn, (int*)I.nn.get(),

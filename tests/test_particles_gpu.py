@@ -792,3 +792,43 @@ def test_fused_fire_list_outgrows_its_rows(gpu, L, prec):
     xr = xr.double().cpu().numpy()
     tol = 1e3 * (2.0 ** -52 if prec == "fp64" else 2.0 ** -23)
     assert np.linalg.norm(x - xr) <= tol * np.linalg.norm(xr - x0)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_lj_crowded_cell_vs_oracle(gpu, prec):
+    """A thousand particles in one cell of the list build (a wavefront sorts
+    it), two thirds of a sigma and less apart."""
+    m = gpu
+    print("case lj crowded cell", prec, flush=True)
+    k = np.arange(10) * 0.28 + 0.1
+    x = np.stack(np.meshgrid(k, k, k, indexing="ij"), -1).reshape(-1, 3)
+    rng = np.random.default_rng(12)
+    x = r32((x + rng.uniform(-0.01, 0.01, x.shape))[rng.permutation(1000)].reshape(-1))
+    o = OracleLJPBC(1000, 12.0, 2.5)
+    e, g = m.State(m.Lj3d().setCutoff(2.5, [12.0] * 3, 0.3), x, prec).energyGradient()
+    tol = 1e-12 if prec == "fp64" else 1e-4  # 14 ulp of 3 over 0.26 in a pair's force
+    assert abs(e - o.energy(x)) <= tol * abs(o.energy(x))
+    assert rel_err(g, o.gradient(x)) <= tol
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_lj_diverged_particles_are_no_neighbours(gpu, prec):
+    """Particles at NaN and infinity when the list is built: nobody's
+    neighbours, wherever they are filed, and the rest as if they were not there."""
+    m = gpu
+    print("case lj diverged", prec, flush=True)
+    side, a = 20, 0.85 ** (-1 / 3)
+    rng = np.random.default_rng(9)
+    x = r32(lattice(side, a, 0.1, rng)).reshape(-1, 3)
+    lost = rng.permutation(side ** 3)[:5000]
+    y = x.copy()
+    y[lost[:3000], rng.integers(0, 3, 3000)] = np.nan
+    y[lost[3000:], rng.integers(0, 3, 2000)] = np.inf
+    kept = np.setdiff1d(np.arange(side ** 3), lost)
+    pot = m.Lj3d().setCutoff(2.5, [side * a] * 3, 0.3)
+    e, g = m.State(pot, y.reshape(-1), prec).energyGradient()
+    e0, g0 = m.State(pot, x[kept].reshape(-1), prec).energyGradient()
+    tol = 1e-12 if prec == "fp64" else 1e-5  # lists in another order
+    assert abs(e - e0) <= tol * abs(e0)
+    assert rel_err(g.reshape(-1, 3)[kept], g0.reshape(-1, 3)) <= tol
+    assert not g.reshape(-1, 3)[lost].any()
