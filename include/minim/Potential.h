@@ -170,8 +170,9 @@ class Potential {
   virtual void evaluateMixedAsync(const void* x, const void* d, double t, bool wantE, double* e_dev, void* g,
                                   void* stream) const;
   // Benchmark support: average duration (ms, HIP events on the stream) of
-  // reps back-to-back launches of the evaluation kernel alone, without the
-  // cross-block reduction that follows it.  The default throws
+  // reps back-to-back launches of the evaluation kernel alone, without a
+  // cross-block reduction that follows it (what each potential launches:
+  // minim_hip.h).  The default throws
   // std::invalid_argument.
   virtual double timeKernel(int prec, const void* x, bool wantE, void* g, int reps, void* stream) const;
   // Benchmark support: `steps` whole energy+gradient evaluations at x on the
@@ -203,10 +204,9 @@ class Potential {
   // std::invalid_argument.
   virtual bool supportsStep() const { return false; }
   // True when evaluateStepAsync also takes g = nullptr: the energy at
-  // x + t*d and x + t*d in xout, keeping what the gradient there needs, so
-  // that the next gradient evaluation at xout (with no other evaluation in
-  // between) costs less.  The line search then pays for that gradient only
-  // when it accepts the trial.
+  // x + t*d and x + t*d in xout, for potentials whose gradient is worth
+  // leaving to an evaluation of its own: the line search then pays for it
+  // only when it accepts the trial.
   virtual bool stepDefersGradient() const { return false; }
   virtual void evaluateStepAsync(int px, int pv, const void* x, const void* d, double t, void* xout, void* g,
                                  void* stream) const;

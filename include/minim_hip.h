@@ -241,11 +241,12 @@ int minim_potential_eval_step(const minim_potential* pot, int precision_x, int p
 /* Benchmark support (no reference counterpart): average duration in ms,
  * measured with HIP events on stream, of reps back-to-back launches of the
  * evaluation kernels (energy when want_energy, gradient into g when g !=
- * NULL).  PhaseField: the stencil kernel without the cross-block reduction;
- * PhaseFieldUnstructured: the element kernel (and the gather of shared sites
- * with g); LjNd: the padding and force passes (cutoff mode) or the all-pairs
- * kernel with its reduction; BarAndHinge: the energy pass with its reduction
- * and the gradient pass.  MINIM_EINVAL for other potentials. */
+ * NULL).  PhaseField: the stencil kernel without the cross-block reduction
+ * (which launches of up to 64 blocks contain); PhaseFieldUnstructured: the
+ * per-site kernel, or the list's element kernel (and the gather of shared
+ * sites with g); LjNd: the force pass (cutoff mode) or the all-pairs kernel
+ * with its reduction; BarAndHinge: the cluster kernel, with the energy's
+ * reduction when want_energy.  MINIM_EINVAL for other potentials. */
 int minim_potential_time_kernel(const minim_potential* pot, int precision, const void* x, size_t ndof,
                                 int want_energy, void* g, int reps, void* stream, double* ms_per_launch);
 /* Benchmark support (no reference counterpart): steps whole energy+gradient

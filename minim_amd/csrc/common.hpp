@@ -5,7 +5,8 @@
 //    PhaseField layout is AoS, index = site * nFluid + fluid, site = (x*Ny+y)*Nz+z;
 //  * every reduction accumulates in FP64, per thread, then per wavefront
 //    (64 lanes, shuffles), then per block (LDS), then across blocks in a fixed
-//    order by the last block to finish -- results are bitwise reproducible;
+//    order by a second, small kernel (or, for small launches of the tiled
+//    PhaseField kernel, by the last block) -- results are bitwise reproducible;
 //  * kernels are compiled with -ffp-contract=off: every product is rounded
 //    before it is added, as in the reference's element-wise vector operators.
 #pragma once

@@ -46,11 +46,11 @@ __device__ inline void load_pos(const T* __restrict__ x, const T* __restrict__ d
 // other particles j over its threads, so that a cluster of N particles has
 // N/R blocks of N/256 steps each; the block sums the R gradients in FP64 and
 // one thread stores them.  Bound by FP64 issue (the division) when N is large
-// and by the latency of one pass over the positions when it is small.  Whole
-// evaluations (energy and gradient, host synchronisation included, 3-D FP64):
-// 35 us at 64 particles, 38 us at 1,000 and 57 us at 4,096; one thread per
-// particle with a serial loop over j (4 blocks for 1,000 particles) took 44,
-// 220 and 804 us.  Lanes add N/256 terms each and the block adds the lanes in
+// and by the latency of one pass over the positions when it is small.  Energy and
+// gradient, both on the device, in 3-D FP64: 9.6 us at 64 particles and 10 us at
+// 1,000 (the host's two launches; the pairs take 6 us), 29 us at 4,096; one thread
+// per particle with a serial loop over j (4 blocks for 1,000 particles), waited
+// for by the host, took 45, 221 and 807 us.  Lanes add N/256 terms each and the block adds the lanes in
 // FP64, so the gradient's error against 64 bits fell too (1,000 particles,
 // 3-D: 1.2e-15 -> 6e-16 in FP64, 1.1e-6 -> 7.6e-7 in FP32).  MODE bit 1
 // energy, bit 2 gradient.

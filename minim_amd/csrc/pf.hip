@@ -605,8 +605,10 @@ TileGeom tile_geom_for(const PFArgs& a, int mode) {
   if (!tile_geom(a.X, a.Y, a.Z, R, xo, target, kMaxRedBlocks, G, 0, busy))
     throw std::invalid_argument("PhaseField: grid too large for one launch");
   // flat chunks for gradients at x (with or without the energy) that more than
-  // kSelfBlocks blocks share.  Energies alone read two neighbours of a site and
-  // gain nothing, and the fused step sums its energy as the trials do.
+  // kSelfBlocks blocks share.  An energy alone would gain too (150x131x97x3 at x:
+  // FP64 15.7 -> 14.5 us, FP32 11.2 -> 10.7), but stays on the tiles with the trial
+  // energies and the fused step, whose flat form is not written, so that a
+  // search's energies are summed alike.
   TileGeom F;
   if ((mode & 6) == 2 && G.nblocks > kSelfBlocks &&
       tile_geom(a.X, a.Y, a.Z, R, xo, target, kMaxRedBlocks, F, flat_halo(a.Y, a.Z, R), busy) &&
