@@ -77,11 +77,7 @@ __device__ inline T dot3(const T (&a)[3], const T (&b)[3]) {
 // 1 to 4; the angle's cosine already takes one to the power 8.  A reciprocal by
 // Newton's iteration, then one correction by the exact remainder (Markstein,
 // IA-64 and Elementary Functions, 2000, ch. 8 and 9).
-__device__ inline double reciprocal(double b) {
-  double r = __builtin_amdgcn_rcp(b);
-  r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
-  return __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
-}
+__device__ inline double reciprocal(double b) { return newton_rcp(b); }
 __device__ inline float reciprocal(float b) { return b; }
 // a / b, with r = reciprocal(b)
 __device__ inline double quotient(double a, double b, double r) {
@@ -176,9 +172,6 @@ __device__ inline void hinge_gradient(const HingeGeo<T>& G, T k, T (&f)[4][3]) {
     f[3][c] = B;
   }
 }
-
-// Barrier that orders LDS traffic only (no wait on outstanding global accesses).
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // What a thread reads for a chunk: one node of the table, two hinge records,
 // and the first codes of the node that it adds up.

@@ -50,6 +50,21 @@ struct HipError : std::runtime_error {
     }                                                                                          \
   } while (0)
 
+// Barrier that orders LDS traffic only: waits for this wave's LDS operations,
+// not for its outstanding global loads and stores.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// 1 / v by the hardware's estimate and Newton's iteration: within an ulp.
+__device__ __forceinline__ float newton_rcp(float v) {
+  const float r = __builtin_amdgcn_rcpf(v);
+  return __builtin_fmaf(__builtin_fmaf(-v, r, 1.0f), r, r);
+}
+__device__ __forceinline__ double newton_rcp(double v) {
+  double r = __builtin_amdgcn_rcp(v);
+  r = __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
+}
+
 // ---------------------------------------------------------------- reductions
 // Sum K doubles over the 64 lanes of a wavefront.
 template <int K>

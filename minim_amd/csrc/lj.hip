@@ -397,17 +397,6 @@ __global__ __launch_bounds__(kBlock) void lj_point_kernel(const T* __restrict__ 
   xt[i] = x[i] + s;
 }
 
-// 1 / v by the hardware's estimate and Newton's iteration: within an ulp.
-__device__ __forceinline__ float newton_rcp(float v) {
-  const float r = __builtin_amdgcn_rcpf(v);
-  return __builtin_fmaf(__builtin_fmaf(-v, r, 1.0f), r, r);
-}
-__device__ __forceinline__ double newton_rcp(double v) {
-  double r = __builtin_amdgcn_rcp(v);
-  r = __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
-  return __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
-}
-
 template <typename T>
 struct Pos3 {
   T c[3];

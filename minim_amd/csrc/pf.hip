@@ -38,10 +38,6 @@ namespace minim_amd {
 
 namespace {
 
-// Barrier that orders LDS traffic only: waits for this wave's LDS operations,
-// not for its outstanding global loads and stores.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 template <typename T>
 __device__ __forceinline__ T fmad(T a, T b, T c) {
   return fma(a, b, c);

@@ -347,9 +347,6 @@ __global__ __launch_bounds__(kBlock) void pf_ext_kernel(PFArgs a, PFCall cl, con
 }
 
 // ---------------------------------------------------------------- tiled kernel
-// Barrier that orders LDS traffic only (no wait on outstanding global accesses).
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // Node volume of a site kind relative to a bulk site: 0 (solid), 1 (bulk) or
 // type/8 (surface types 1..7), all exact.
 template <typename T>

@@ -282,9 +282,6 @@ __global__ __launch_bounds__(kBlock) void pfu_gather_kernel(PFUArgs u, T* __rest
 }
 
 // ---------------------------------------------------------------- per-site form
-// Barrier that orders LDS traffic only (no wait on outstanding global accesses).
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 template <typename T, int N>
 struct SiteVec {
   T v[N];
