@@ -878,9 +878,9 @@ int ext_tile_full(const PFArgs& a, int mode, const void* x, const void* d, doubl
     throw std::invalid_argument("PhaseField: grid too large for one launch");
   if (R == 2 && sizeof(T) * NF <= 24 && automatic) {
     // no shape asked for, and three blocks of two rows per thread fit on a CU: as
-    // many, where they fill
-    // their places better than two do (160x150x141x3 in FP64: 456 of 512 places
-    // 54 us, 741 of 768 47 us; 128^3x3: 512 of 512 26.6 us, 704 of 768 27.8 us)
+    // many, where they fill their places better than two do (160x150x141x3 in FP64:
+    // 456 of 512 places 54 us, 741 of 768 47 us; 128^3x3: 512 of 512 26.6 us, 704 of
+    // 768 27.8 us)
     TileGeom G3;
     if (tile_geom(a.X, a.Y, a.Z, R, 0, kExtTileTarget / 2 * 3, kMaxRedBlocks, G3) && 2 * G3.nblocks > 3 * G.nblocks)
       G = G3;
